@@ -317,36 +317,77 @@ __global__ __launch_bounds__(DF_BLOCK) void direct_f64_kernel(const float4* __re
 }
 
 // ---- FP64 brute force (glam::DVec3 / f64: particular/src/gravity/impls/glam.rs:234) ------------
-// The reference's scalar kernel in FP64 (impls/mod.rs:151-166): IEEE sqrt and division, pairs
-// folded in affecting order per tile; tiles of BF_TILE bodies staged in LDS, one affected body per
-// lane. checked: zero unsoftened distance contributes nothing.
+// The reference's scalar kernel in FP64 (impls/mod.rs:151-166). A workgroup of BF64_WAVES
+// wavefronts holds 64 affected bodies; the affecting range is split over grid.y and, inside a
+// workgroup, over its wavefronts (scalar loads), whose sums are added in wavefront order, and the
+// grid.y partial sums in order by bf64_reduce_kernel. checked: zero distance contributes nothing.
 
-__global__ __launch_bounds__(BF_BLOCK) void bf64_kernel(const double4* __restrict__ aff, uint32_t n,
-                                                        const double4* __restrict__ afg, uint32_t m,
-                                                        double eps2, int checked,
-                                                        double4* __restrict__ out) {
-    __shared__ double4 tile[BF_TILE];
-    const uint32_t i = blockIdx.x * BF_BLOCK + threadIdx.x;
+constexpr int BF64_WAVES = 8;
+
+// |r2|^-1/2 to the last bit or two: v_rsq_f64 (about 1e-8 relative) and one third-order step
+// y (1 + e/2 + 3 e^2 / 8), e = 1 - r2 y^2. An infinite r2 (y = 0) stays 0.
+__device__ __forceinline__ double rsqrt64(double r2) {
+    const double y = __builtin_amdgcn_rsq(r2);
+    const double e = fma(-(fmin(r2, 1.7976931348623157e308) * y), y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+template <bool MASK>
+__global__ __launch_bounds__(64 * BF64_WAVES) void bf64_kernel(const double4* __restrict__ aff,
+                                                               uint32_t n,
+                                                               const double4* __restrict__ afg,
+                                                               uint32_t m, uint32_t j_chunk,
+                                                               double eps2,
+                                                               double4* __restrict__ out) {
+    __shared__ double part[BF64_WAVES][3][64];
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    const uint32_t i = blockIdx.x * 64 + lane;
     const double4 p = aff[i < n ? i : n - 1];
+    const uint32_t b0 = blockIdx.y * j_chunk, b1 = min(m, b0 + j_chunk);
+    const uint32_t per = (b1 - b0 + BF64_WAVES - 1) / BF64_WAVES;
+    const uint32_t jb = min(b1, b0 + wave * per), je = min(b1, jb + per);
     double ax = 0.0, ay = 0.0, az = 0.0;
-    for (uint32_t j0 = 0; j0 < m; j0 += BF_TILE) {
-        const uint32_t cnt = min(uint32_t(BF_TILE), m - j0);
-        __syncthreads();
-        if (threadIdx.x < cnt) tile[threadIdx.x] = afg[j0 + threadIdx.x];
-        __syncthreads();
-        for (uint32_t j = 0; j < cnt; ++j) {
-            const double4 q = tile[j];
-            const double dx = q.x - p.x, dy = q.y - p.y, dz = q.z - p.z;
-            const double r2 = __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz));
-            if (checked && r2 == 0.0) continue;
-            const double rs = r2 + eps2;
-            const double s = q.w / (rs * sqrt(rs));
-            ax += dx * s;
-            ay += dy * s;
-            az += dz * s;
-        }
+#pragma unroll 4
+    for (uint32_t j = jb; j < je; ++j) {
+        const double4 q = afg[j];  // wave-uniform: a scalar load
+        const double dx = q.x - p.x, dy = q.y - p.y, dz = q.z - p.z;
+        // MASK tests the unsoftened distance
+        const double d2 = fma(dx, dx, fma(dy, dy, MASK ? dz * dz : fma(dz, dz, eps2)));
+        double inv = rsqrt64(MASK ? d2 + eps2 : d2);
+        if (MASK) inv = d2 == 0.0 ? 0.0 : inv;
+        const double s = (q.w * inv) * (inv * inv);
+        ax = fma(dx, s, ax);
+        ay = fma(dy, s, ay);
+        az = fma(dz, s, az);
     }
-    if (i < n) out[i] = make_double4(ax, ay, az, 0.0);
+    part[wave][0][lane] = ax;
+    part[wave][1][lane] = ay;
+    part[wave][2][lane] = az;
+    __syncthreads();
+    if (wave != 0) return;
+    for (int w = 1; w < BF64_WAVES; ++w) {
+        ax += part[w][0][lane];
+        ay += part[w][1][lane];
+        az += part[w][2][lane];
+    }
+    if (i < n) out[size_t(blockIdx.y) * n + i] = make_double4(ax, ay, az, 0.0);
+}
+
+__global__ __launch_bounds__(64) void bf64_reduce_kernel(const double4* __restrict__ partial,
+                                                         uint32_t n, uint32_t splits,
+                                                         double4* __restrict__ out) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double ax = 0.0, ay = 0.0, az = 0.0;
+#pragma unroll 8
+    for (uint32_t s = 0; s < splits; ++s) {
+        const double4 p = partial[size_t(s) * n + i];
+        ax += p.x;
+        ay += p.y;
+        az += p.z;
+    }
+    out[i] = make_double4(ax, ay, az, 0.0);
 }
 
 static int copy_in(pnb_ctx* c, DevBuf& b, const float* src, size_t count) {
@@ -502,11 +543,38 @@ int pnb_bf_accel_f64_dev(pnb_ctx* c, const double* affected, size_t n, const dou
     if (n == 0) return PNB_OK;
     if (n > 0x7fffffffu || m > 0x7fffffffu) return fail(c, PNB_E_ARG, "too many particles");
     if (int rc = activate(c)) return rc;
-    bf64_kernel<<<div_up(n, BF_BLOCK), BF_BLOCK, 0, c->stream>>>(
+    // Workgroups over the affecting range until the launch holds about four rounds of wavefronts
+    // (32 per CU), with at least 32 affecting bodies for each of a workgroup's wavefronts.
+    const size_t cus = c->cu_count > 0 ? size_t(c->cu_count) : 256;
+    const size_t blocks = div_up(n, 64);
+    size_t splits = 1;
+    while (splits < 64 && blocks * splits * BF64_WAVES < 128 * cus && m / (splits * 2) >= 32 * BF64_WAVES)
+        splits <<= 1;
+    uint32_t chunk = std::max(1u, div_up(m, splits));
+    splits = std::max<size_t>(1, div_up(m, chunk));
+    double4* o = reinterpret_cast<double4*>(out);
+    double4* dst = o;
+    // inside a caller's capture nothing can be allocated: one range when the scratch is too small
+    if (splits > 1 && c->bf_partial.cap < splits * n * sizeof(double4) && stream_capturing(c)) {
+        splits = 1;
+        chunk = uint32_t(m);
+    }
+    if (splits > 1) {
+        PNB_HIP(c, c->bf_partial.ensure(splits * n * sizeof(double4)));
+        dst = c->bf_partial.as<double4>();
+    }
+    // The self term and coincident pairs add d * s = 0 with s finite when the softening is not
+    // tiny (mu < 1e263 here), so only a vanishing softening needs the mask.
+    const double eps2 = softening * softening;
+    auto k = checked && eps2 < 1e-30 ? bf64_kernel<true> : bf64_kernel<false>;
+    k<<<dim3(unsigned(blocks), unsigned(splits)), 64 * BF64_WAVES, 0, c->stream>>>(
         reinterpret_cast<const double4*>(affected), uint32_t(n),
-        reinterpret_cast<const double4*>(affecting), uint32_t(m), softening * softening, checked,
-        reinterpret_cast<double4*>(out));
+        reinterpret_cast<const double4*>(affecting), uint32_t(m), chunk, eps2, dst);
     PNB_CHECK_LAUNCH(c);
+    if (splits > 1) {
+        bf64_reduce_kernel<<<div_up(n, 64), 64, 0, c->stream>>>(dst, uint32_t(n), uint32_t(splits), o);
+        PNB_CHECK_LAUNCH(c);
+    }
     return PNB_OK;
 }
 

@@ -1804,16 +1804,6 @@ static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = fa
     });
 }
 
-// Whether work is being captured on the context's stream into a graph.
-static bool stream_capturing(pnb_ctx* c) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(c->stream, &st) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    return st != hipStreamCaptureStatusNone;
-}
-
 // Capacities of a capturable build from an ordinary build of the same size (its node count and
 // depth known on the host): a quarter more nodes and 8 more levels, so that later trees of
 // similar inputs fit.

@@ -63,6 +63,15 @@ int activate(pnb_ctx* c) {
     return PNB_OK;
 }
 
+bool stream_capturing(pnb_ctx* c) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
 // ---- exclusive scan (reduce, scan block sums recursively, add) --------------------------------
 
 constexpr int SCAN_BLOCK = 256;

@@ -74,6 +74,8 @@ namespace pnb {
 int fail(pnb_ctx* c, int code, const char* fmt, ...);
 int hip_fail(pnb_ctx* c, hipError_t e, const char* expr, const char* file, int line);
 int activate(pnb_ctx* c);  // hipSetDevice(c->device)
+// Whether work is being captured on the context's stream into a graph.
+bool stream_capturing(pnb_ctx* c);
 
 // Device-wide exclusive scan of n uint32 values (in place allowed). out[n] receives the total
 // when out has room for n + 1 entries and with_total is set.
