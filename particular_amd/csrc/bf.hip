@@ -16,6 +16,7 @@
 // Pair semantics follow particular/src/gravity/impls/mod.rs:151-166: with `checked` a pair at
 // zero unsoftened distance contributes nothing; with softening > 0 that pair contributes
 // d * finite = 0 anyway, so only checked && softening == 0 needs the explicit mask.
+#include "bf_common.hpp"
 #include "pnb_internal.hpp"
 
 #include <algorithm>
@@ -37,36 +38,12 @@ struct BfTune {
 
 void bf_tune_free(BfTune* t) { delete t; }
 
-template <int R, bool MASK>
-__device__ __forceinline__ void bf_body(const float4 q, const float (&xi)[R], const float (&yi)[R],
-                                        const float (&zi)[R], float eps2, float (&px)[R],
-                                        float (&py)[R], float (&pz)[R]) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const float dx = q.x - xi[r];
-        const float dy = q.y - yi[r];
-        const float dz = q.z - zi[r];
-        const float r2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
-        float inv = __builtin_amdgcn_rsqf(r2);
-        if (MASK) inv = (r2 > 0.0f) ? inv : 0.0f;
-        const float s = (q.w * inv) * (inv * inv);
-        px[r] = fmaf(dx, s, px[r]);
-        py[r] = fmaf(dy, s, py[r]);
-        pz[r] = fmaf(dz, s, pz[r]);
-    }
-}
-
-__device__ __forceinline__ void kahan_add(float& sum, float& comp, float v) {
-    const float y = v - comp;
-    const float t = sum + y;
-    comp = (t - sum) - y;
-    sum = t;
-}
-
 // grid.x: affected tiles of BF_BLOCK * R particles; grid.y: affecting ranges of j_chunk bodies.
 // With gridDim.y == 1 the result goes to `out`, else to partial[blockIdx.y * n + i].
-// VAR 0: LDS tile; 1: wave-uniform global reads (scalar loads).
-template <int R, bool MASK, int VAR>
+// VAR 0: LDS tile; 1: wave-uniform global reads (scalar loads). SELF: aff and afg are one array and
+// a body's pair with itself adds nothing; only the tiles that meet the workgroup's own bodies test
+// for it.
+template <int R, bool MASK, int VAR, bool SELF = false>
 __global__ __launch_bounds__(BF_BLOCK) void bf_kernel(const float4* __restrict__ aff, uint32_t n,
                                                       const float4* __restrict__ afg, uint32_t m,
                                                       uint32_t j_chunk, float eps2,
@@ -97,7 +74,11 @@ __global__ __launch_bounds__(BF_BLOCK) void bf_kernel(const float4* __restrict__
         float px[R], py[R], pz[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) px[r] = py[r] = pz[r] = 0.0f;
-        if (cnt == BF_TILE) {
+        const uint32_t own = blockIdx.x * uint32_t(BF_BLOCK * R);
+        if (SELF && j0 < own + BF_BLOCK * R && own < j0 + cnt) {
+            for (uint32_t j = 0; j < cnt; ++j)
+                bf_body<R, MASK, true>(LDS ? tile[j] : afg[j0 + j], xi, yi, zi, eps2, px, py, pz, j0 + j, i0, BF_BLOCK);
+        } else if (cnt == BF_TILE) {
 #pragma unroll 8
             for (int j = 0; j < BF_TILE; ++j)
                 bf_body<R, MASK>(LDS ? tile[j] : afg[j0 + j], xi, yi, zi, eps2, px, py, pz);
@@ -121,12 +102,39 @@ __global__ __launch_bounds__(BF_BLOCK) void bf_kernel(const float4* __restrict__
     }
 }
 
+// Small and middle affected counts: one workgroup of COOP_WAVES wavefronts per 64 affected bodies
+// (and per affecting range, grid.y), the wavefronts sharing the affecting bodies tile by tile
+// (coop_sum). Up to 512 affected tiles there are too few wavefronts for one of them per tile to
+// fill the chip, and each is bound by its own issue rate.
+constexpr int COOP_WAVES = 16;
+
+template <bool MASK, bool SELF, int T>
+__global__ __launch_bounds__(64 * COOP_WAVES) void bf_coop_kernel(const float4* __restrict__ aff,
+                                                                  uint32_t n,
+                                                                  const float4* __restrict__ afg,
+                                                                  uint32_t m, uint32_t j_chunk,
+                                                                  float eps2,
+                                                                  float4* __restrict__ out) {
+    __shared__ CoopLds<1, COOP_WAVES> lds;
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+    const uint32_t i = blockIdx.x * 64 + (threadIdx.x & 63);
+    const uint32_t jb = blockIdx.y * j_chunk, je = min(m, jb + j_chunk);
+    const float4 p = aff[i < n ? i : n - 1];
+    const float xi[1] = {p.x}, yi[1] = {p.y}, zi[1] = {p.z};
+    float ax[1], ay[1], az[1];
+    coop_sum<1, MASK, SELF, T, COOP_WAVES>(lds, afg, jb, je, COOP_WAVES, wave, true, eps2, i, xi, yi,
+                                           zi, ax, ay, az);
+    if (wave == 0 && i < n)
+        out[size_t(blockIdx.y) * n + i] = make_float4(ax[0], ay[0], az[0], 0.0f);
+}
+
 // Fixed-order compensated reduction of j_split partial sums.
 __global__ void bf_reduce_kernel(const float4* __restrict__ partial, uint32_t n, uint32_t splits,
                                  float4* __restrict__ out) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     float ax = 0, ay = 0, az = 0, cx = 0, cy = 0, cz = 0;
+#pragma unroll 8
     for (uint32_t s = 0; s < splits; ++s) {
         const float4 p = partial[size_t(s) * n + i];
         kahan_add(ax, cx, p.x);
@@ -158,13 +166,60 @@ static BfKernel pick_mask(int r, bool mask) {
     return mask ? pick_r<true, VAR>(r) : pick_r<false, VAR>(r);
 }
 
-static BfKernel pick_kernel(int variant, int r, bool mask) {
-    return variant == 0 ? pick_mask<0>(r, mask) : pick_mask<1>(r, mask);
+// One set on itself: the default shapes only (tuning entries are for two sets).
+template <bool MASK>
+static BfKernel pick_self(int r) {
+    return r == 4 ? bf_kernel<4, MASK, 1, true> : r == 2 ? bf_kernel<2, MASK, 0, true> : bf_kernel<1, MASK, 0, true>;
 }
+
+template <bool SELF>
+static BfKernel pick_coop(bool mask, int tile) {
+    switch (tile) {
+        case 64: return mask ? bf_coop_kernel<true, SELF, 64> : bf_coop_kernel<false, SELF, 64>;
+        case 128: return mask ? bf_coop_kernel<true, SELF, 128> : bf_coop_kernel<false, SELF, 128>;
+        default: return mask ? bf_coop_kernel<true, SELF, 256> : bf_coop_kernel<false, SELF, 256>;
+    }
+}
+
+constexpr int BF_COOP = 2;  // variant of the workgroup-cooperative kernel (not for tuning entries)
 
 struct BfShape {
     int variant, per_lane, j_split;
 };
+
+// What the cooperative kernel takes: sums small enough that wavefronts walking the affecting
+// bodies alone are bound by their own issue rate (a 1,024-body range takes one 34 us). Measured,
+// alone / cooperative, softened: 1,000 x 1,000 34 / 9 us; 4,096 x 4,096 36 / 15; 64 x 65,536
+// 51 / 17; 8,192 x 8,192 28 / 28 (6.7e7 pairs); 12,000 x 16,384 67 / 96. With few affecting bodies
+// the others have no range to split and it pays up to 2.5e8 pairs (65,536 x 1,000 78 / 28 us); with
+// at most one tile there is nothing to share (50,000 x 64: 4.2 / 7.4 us).
+static bool coop_pays(size_t n, size_t m) {
+    if (m <= 64 || (m <= 256 && n > 32768)) return false;
+    return n * m <= (m < 2048 ? size_t(250000000) : size_t(60000000));
+}
+
+static BfShape default_shape(pnb_ctx* c, size_t n, size_t m) {
+    const size_t cus = c->cu_count > 0 ? size_t(c->cu_count) : 256;
+    int s = 1;
+    if (coop_pays(n, m)) {
+        // workgroups of 16 wavefronts over the affecting range until every CU has one, keeping a
+        // tile of 64 bodies for each wavefront
+        const size_t blocks = div_up(n, 64);
+        while (s < 64 && blocks * s * 2 <= cus && m / (size_t(s) * 2) >= size_t(COOP_WAVES) * 64) s <<= 1;
+        return {BF_COOP, 1, s};
+    }
+    // Otherwise one wavefront per affected tile and range: bodies per lane by the affected count
+    // (register-blocked scalar loads from 131,072 on; below, more and smaller workgroups reading
+    // the affecting bodies from LDS, one per lane where there are few affecting bodies to split), and up to 64 workgroups per CU over the affecting range, of at
+    // least one tile (4 per lane) or two. Softened: 65,536 x 16,384 299 us with 2 per lane from LDS,
+    // 333 with 4 from scalar loads in ranges of 1,024; 500,000 x 20,000 2.53 ms with 4 per lane,
+    // 2.57 with 2.
+    const int r = n >= 131072 && m > 64 ? 4 : n >= 24576 && m >= 8192 ? 2 : 1;
+    const size_t blocks = div_up(n, size_t(BF_BLOCK) * r);
+    const size_t least = (r == 4 ? 1 : 2) * size_t(BF_TILE);
+    while (s < 64 && blocks * s * 2 <= 64 * cus && m / (size_t(s) * 2) >= least) s <<= 1;
+    return {r == 4 ? 1 : 0, r, s};
+}
 
 static BfShape choose_shape(pnb_ctx* c, size_t n, size_t m) {
     if (c->bf_tune) {
@@ -173,32 +228,28 @@ static BfShape choose_shape(pnb_ctx* c, size_t n, size_t m) {
             if (e.n_min <= n && (!best || e.n_min > best->n_min)) best = &e;
         if (best) return {best->variant, best->per_lane, best->j_split};
     }
-    // Default (from autotuning on MI355X): 4 affected bodies per lane with scalar-loaded
-    // affecting bodies once there are at least 64 affected tiles, else 1 per lane from LDS; the
-    // affecting range is split into up to 64 workgroups per CU (small workgroups balance the
-    // load across CUs and XCDs), keeping at least 4 tiles of affecting bodies per split.
-    const size_t cus = c->cu_count > 0 ? size_t(c->cu_count) : 256;
-    const int r = n >= size_t(64) * BF_BLOCK * 4 ? 4 : 1;
-    const int variant = r == 4 ? 1 : 0;
-    const size_t blocks = div_up(n, size_t(BF_BLOCK) * r);
-    int s = 1;
-    while (s < 64 && blocks * s * 2 <= 64 * cus && m / (size_t(s) * 2) >= 4 * size_t(BF_TILE)) s <<= 1;
-    return {variant, r, s};
+    return default_shape(c, n, m);
 }
 
 struct BfPlan {
     BfShape shape;
     uint32_t splits, chunk;
+    int tile;
 };
 
-static BfPlan plan(pnb_ctx* c, size_t n, size_t m) {
-    const BfShape sh = choose_shape(c, n, m);
+// Splits of the affecting range in whole tiles. The cooperative kernel takes smaller tiles for
+// small ranges, so that all its wavefronts get one.
+static BfPlan plan_for(const BfShape& sh, size_t m) {
     uint32_t splits = uint32_t(sh.j_split);
+    const size_t per = m / splits / COOP_WAVES;
+    const int tile = sh.variant != BF_COOP || per >= 256 ? BF_TILE : per >= 128 ? 128 : 64;
     uint32_t chunk = uint32_t(div_up(m, splits));
-    chunk = (chunk + BF_TILE - 1) / BF_TILE * BF_TILE;
+    chunk = (chunk + tile - 1) / tile * tile;
     splits = uint32_t(div_up(m, chunk));
-    return {sh, splits, chunk};
+    return {sh, splits, chunk, tile};
 }
+
+static BfPlan plan(pnb_ctx* c, size_t n, size_t m) { return plan_for(choose_shape(c, n, m), m); }
 
 // Allocates what bf_launch(n, m) will need, so that a later launch inside a graph capture
 // allocates nothing.
@@ -237,16 +288,21 @@ int bf_noalloc_init(pnb_ctx* c) {
 // unused when the plan has one split). No allocation.
 static int bf_launch_with(pnb_ctx* c, const BfPlan& p, const float4* affected, size_t n,
                           const float4* affecting, size_t m, float softening, int checked,
-                          float4* out, float4* partial) {
+                          float4* out, float4* partial, bool self = false) {
     const BfShape sh = p.shape;
     const bool mask = checked && softening == 0.0f;
-    BfKernel k = pick_kernel(sh.variant, sh.per_lane, mask);
+    const bool coop = sh.variant == BF_COOP;
+    BfKernel k;
+    if (coop) k = self ? pick_coop<true>(mask, p.tile) : pick_coop<false>(mask, p.tile);
+    else if (self) k = mask ? pick_self<true>(sh.per_lane) : pick_self<false>(sh.per_lane);
+    else k = sh.variant == 0 ? pick_mask<0>(sh.per_lane, mask) : pick_mask<1>(sh.per_lane, mask);
     const float eps2 = softening * softening;
     const uint32_t splits = p.splits, chunk = p.chunk;
-    dim3 grid(div_up(n, size_t(BF_BLOCK) * sh.per_lane), splits);
+    const unsigned block = coop ? 64 * COOP_WAVES : BF_BLOCK;
+    dim3 grid(div_up(n, coop ? size_t(64) : size_t(BF_BLOCK) * sh.per_lane), splits);
     float4* dst = splits > 1 ? partial : out;
     return timed(c, PNB_PROF_BF, [&]() -> int {
-        k<<<grid, BF_BLOCK, 0, c->stream>>>(affected, uint32_t(n), affecting, uint32_t(m), chunk,
+        k<<<grid, block, 0, c->stream>>>(affected, uint32_t(n), affecting, uint32_t(m), chunk,
                                             eps2, dst);
         PNB_CHECK_LAUNCH(c);
         if (splits > 1) {
@@ -255,6 +311,19 @@ static int bf_launch_with(pnb_ctx* c, const BfPlan& p, const float4* affected, s
         }
         return PNB_OK;
     });
+}
+
+// The sum over all other bodies of one set, for sizes where the pair kernel cannot fill the chip
+// (pairs.hip): a body's term with itself is left out by index, whatever the softening.
+int bf_self_launch(pnb_ctx* c, const float4* p, size_t n, float softening, int checked, float4* out) {
+    const BfPlan pl = plan_for(default_shape(c, n, n), n);
+    if (pl.splits > 1) {
+        const size_t need = size_t(pl.splits) * n * sizeof(float4);
+        if (c->capturing && c->bf_partial.cap < need)
+            return fail(c, PNB_E_STATE, "brute-force scratch not prepared before graph capture");
+        PNB_HIP(c, c->bf_partial.ensure(need));
+    }
+    return bf_launch_with(c, pl, p, n, p, n, softening, checked, out, c->bf_partial.as<float4>(), true);
 }
 
 int bf_launch(pnb_ctx* c, const float4* affected, size_t n, const float4* affecting, size_t m,

@@ -1,0 +1,133 @@
+// The brute-force pair term and the workgroup-cooperative sum over affecting bodies, shared by the
+// single brute force (bf.hip) and the batched ensemble (batch.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+namespace pnb {
+
+// a_i += d * (mu * rsq(r2)^3) for one affecting body q and R affected bodies per lane.
+// MASK: a pair at zero distance adds nothing. SELF: body `self + 64 r` of the affecting array is
+// affected body r itself and adds nothing (whatever its term would be); j is q's index.
+template <int R, bool MASK, bool SELF = false>
+__device__ __forceinline__ void bf_body(const float4 q, const float (&xi)[R], const float (&yi)[R],
+                                        const float (&zi)[R], float eps2, float (&px)[R],
+                                        float (&py)[R], float (&pz)[R], uint32_t j = 0,
+                                        uint32_t self = 0, uint32_t stride = 64) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const float dx = q.x - xi[r];
+        const float dy = q.y - yi[r];
+        const float dz = q.z - zi[r];
+        const float r2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
+        float inv = __builtin_amdgcn_rsqf(r2);
+        if (MASK) inv = (r2 > 0.0f) ? inv : 0.0f;
+        if (SELF) inv = (j != self + uint32_t(r) * stride) ? inv : 0.0f;
+        const float s = (q.w * inv) * (inv * inv);
+        px[r] = fmaf(dx, s, px[r]);
+        py[r] = fmaf(dy, s, py[r]);
+        pz[r] = fmaf(dz, s, pz[r]);
+    }
+}
+
+__device__ __forceinline__ void kahan_add(float& sum, float& comp, float v) {
+    const float y = v - comp;
+    const float t = sum + y;
+    comp = (t - sum) - y;
+    sum = t;
+}
+
+// Shared memory of coop_sum for a workgroup of W wavefronts: every wavefront's sums over its
+// latest tile, and the running compensated sums of each group of J wavefronts (J >= 2).
+template <int R, int W>
+struct CoopLds {
+    float part[W][3 * R][64];
+    float sum[W / 2][3 * R][2][64];
+};
+
+// One affected tile of 64 R bodies summed by J wavefronts together (J a power of two, 1 <= J <= W,
+// the same in every wavefront of the workgroup; wavefronts g J .. g J + J - 1 form group g).
+// The affecting range [jb, je) is taken in tiles of T bodies, J tiles a round, one per wavefront,
+// each read with wave-uniform addresses (scalar loads). A tile's sum is plain FP32; the J sums of
+// a round go through LDS into the group's compensated sums in tile order, so the result is the
+// one a single wavefront gets from the same tiles in order, whatever J is. Folding is spread over
+// the group (wavefront k takes components k, k + J, ...), so a round costs two barriers and
+// a few LDS reads for 256 x R pair terms per lane.
+// Every wavefront of the workgroup calls it the same number of times with the same range (idle
+// groups pass live = false); `ax, ay, az` come back complete in every wavefront of the group.
+// Why the split: one wavefront issues about one instruction per 4.8 cycles however idle its CU is,
+// so a tile of affected bodies walked by one wavefront takes m x R x 13 x 4.8 cycles (1.7 ms for
+// 16,384 affecting bodies and R = 4); J wavefronts divide that by J without another pass over
+// memory.
+template <int R, bool MASK, bool SELF, int T, int W>
+__device__ __forceinline__ void coop_sum(CoopLds<R, W>& lds, const float4* __restrict__ afg,
+                                         uint32_t jb, uint32_t je, int J, int wave, bool live,
+                                         float eps2, uint32_t self, const float (&xi)[R],
+                                         const float (&yi)[R], const float (&zi)[R],
+                                         float (&ax)[R], float (&ay)[R], float (&az)[R]) {
+    const int lane = threadIdx.x & 63;
+    const int slot = wave & (J - 1), g0 = wave - slot, g = g0 / J;
+    float cx[R], cy[R], cz[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) ax[r] = ay[r] = az[r] = cx[r] = cy[r] = cz[r] = 0.0f;
+    if (J > 1) {
+        for (int c = slot; c < 3 * R; c += J) lds.sum[g][c][0][lane] = lds.sum[g][c][1][lane] = 0.0f;
+        __syncthreads();
+    }
+    const uint32_t span = uint32_t(T) * uint32_t(J);
+    for (uint32_t base = jb; base < je; base += span) {
+        const uint32_t j0 = base + uint32_t(T) * uint32_t(slot);
+        float px[R], py[R], pz[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) px[r] = py[r] = pz[r] = 0.0f;
+        if (live && j0 < je) {
+            const float4* q = afg + j0;
+            const uint32_t cnt = min(uint32_t(T), je - j0);
+            if (cnt == uint32_t(T)) {
+#pragma unroll 8
+                for (int j = 0; j < T; ++j)
+                    bf_body<R, MASK, SELF>(q[j], xi, yi, zi, eps2, px, py, pz, j0 + j, self);
+            } else {
+                for (uint32_t j = 0; j < cnt; ++j)
+                    bf_body<R, MASK, SELF>(q[j], xi, yi, zi, eps2, px, py, pz, j0 + j, self);
+            }
+        }
+        if (J == 1) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                kahan_add(ax[r], cx[r], px[r]);
+                kahan_add(ay[r], cy[r], py[r]);
+                kahan_add(az[r], cz[r], pz[r]);
+            }
+            continue;
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            lds.part[wave][3 * r][lane] = px[r];
+            lds.part[wave][3 * r + 1][lane] = py[r];
+            lds.part[wave][3 * r + 2][lane] = pz[r];
+        }
+        __syncthreads();
+        const int tiles = int(min(uint32_t(J), (je - base + uint32_t(T) - 1) / uint32_t(T)));
+        for (int c = slot; c < 3 * R; c += J) {
+            float s = lds.sum[g][c][0][lane], k = lds.sum[g][c][1][lane];
+            for (int t = 0; t < tiles; ++t) kahan_add(s, k, lds.part[g0 + t][c][lane]);
+            lds.sum[g][c][0][lane] = s;
+            lds.sum[g][c][1][lane] = k;
+        }
+        __syncthreads();
+    }
+    if (J > 1) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            ax[r] = lds.sum[g][3 * r][0][lane];
+            ay[r] = lds.sum[g][3 * r + 1][0][lane];
+            az[r] = lds.sum[g][3 * r + 2][0][lane];
+        }
+        __syncthreads();  // the sums are read before the next call clears them
+    }
+}
+
+}  // namespace pnb

@@ -212,6 +212,14 @@ __global__ void pairs_zero_kernel(float4* __restrict__ out, size_t n) {
 // at this size).
 constexpr size_t PR_MAX_N = size_t(1) << 22;
 
+// Below these sizes the one-sided sums over all other bodies are faster: the pair kernel has one
+// workgroup per two super-tiles of 4,096 bodies (36 workgroups at 30,000 bodies, two resident per
+// CU), each a serial pass of 8 x 512 j bodies (2.4 ms alone, 3.7 ms with two on a CU).
+// Measured, pair kernel against one-sided, softened: 4,096 bodies 1,402 / 16 us; 30,011: 2,390 /
+// 288; 131,072: 5,980 / 4,362; 196,608: 9.83 / 9.64 ms; 262,144: 16.6 / 17.0. With the
+// zero-distance mask: 131,072 6.5 / 4.9 ms; 196,608 10.5 / 10.8.
+constexpr size_t PR_MIN_N = 240000, PR_MIN_N_MASKED = 170000;
+
 int pairs_launch(pnb_ctx* c, const float4* p, size_t n, float softening, int checked,
                  float4* out) {
     if (n == 0) return PNB_OK;
@@ -222,6 +230,8 @@ int pairs_launch(pnb_ctx* c, const float4* p, size_t n, float softening, int che
         PNB_CHECK_LAUNCH(c);
         return PNB_OK;
     }
+    const bool mask = checked && softening == 0.0f;
+    if (n < (mask ? PR_MIN_N_MASKED : PR_MIN_N)) return bf_self_launch(c, p, n, softening, checked, out);
     const uint32_t ns = uint32_t(div_up(n, PR_S));
     const uint32_t n_pad = ns * uint32_t(PR_S);
     const size_t need = size_t(ns) * n_pad * sizeof(float4);
@@ -230,7 +240,6 @@ int pairs_launch(pnb_ctx* c, const float4* p, size_t n, float softening, int che
     PNB_HIP(c, c->pairs_part.ensure(need));
     float4* part = c->pairs_part.as<float4>();
     const unsigned blocks = unsigned(size_t(ns) * (ns + 1) / 2);
-    const bool mask = checked && softening == 0.0f;
     const float eps2 = softening * softening;
     return timed(c, PNB_PROF_BF, [&]() -> int {
         if (mask)

@@ -88,6 +88,8 @@ int split_affecting(pnb_ctx* c, const float4* particles, size_t n, float4* dst, 
 // Brute force on device pointers, asynchronous on c->stream.
 int bf_launch(pnb_ctx* c, const float4* affected, size_t n, const float4* affecting, size_t m,
               float softening, int checked, float4* out);
+// Brute force of one set on itself, each body's own term left out by index.
+int bf_self_launch(pnb_ctx* c, const float4* p, size_t n, float softening, int checked, float4* out);
 
 // Folds all recorded event pairs into the per-kernel totals (waits for the last one).
 int prof_resolve(pnb_ctx* c);
