@@ -8,8 +8,10 @@
 // tail. R (affected bodies per lane) is chosen per system-size bucket by the autotuner. Affecting
 // bodies are read with wave-uniform addresses (scalar loads), so wavefronts need no barriers and
 // run independently. The per-lane arithmetic and summation order are those of the brute-force
-// kernel (FP32 tiles of 256 bodies, Kahan across tiles). A step is enqueue-only and can be
+// kernel (FP32 tiles of 256 bodies, Kahan across tiles). Ensembles whose largest systems would
+// outlast the rest take the queue by workgroups, which share an item's affecting bodies. A step is enqueue-only and can be
 // captured into a hipGraph (the queue counter is cleared by a kernel, not a memset).
+#include "bf_common.hpp"
 #include "pnb_internal.hpp"
 
 #include <algorithm>
@@ -18,6 +20,7 @@
 namespace pnb {
 
 constexpr int BT_TILE = 256;
+constexpr int BT_R_MAX = 2;  // bodies per lane of the workgroup form
 
 struct BatchItem {
     uint32_t off;  // first particle of the system
@@ -33,6 +36,7 @@ struct BatchState {
     std::vector<int64_t> offsets;
     std::vector<std::pair<size_t, int>> tuning;  // (n_min, per_lane)
     bool items_dirty = true;
+    bool coop = false;  // items for workgroups (bt_coop_kernel), else for wavefronts
     size_t n_items = 0;
     unsigned long long interactions = 0;
     DevBuf x, v, shadow, acc, items, queue, stage;
@@ -57,13 +61,6 @@ void batch_free(BatchState* s) {
     delete s;
 }
 
-__device__ __forceinline__ void bt_kahan(float& sum, float& comp, float v) {
-    const float y = v - comp;
-    const float t = sum + y;
-    comp = (t - sum) - y;
-    sum = t;
-}
-
 template <int R, bool MASK>
 __device__ __forceinline__ void bt_tile(const float4* __restrict__ sh, const BatchItem w, float eps2,
                                         float4* __restrict__ acc) {
@@ -83,24 +80,13 @@ __device__ __forceinline__ void bt_tile(const float4* __restrict__ sh, const Bat
 #pragma unroll
         for (int r = 0; r < R; ++r) px[r] = py[r] = pz[r] = 0.f;
         for (uint32_t j = 0; j < cnt; ++j) {
-            const float4 q = sys[j0 + j];
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const float dx = q.x - xi[r], dy = q.y - yi[r], dz = q.z - zi[r];
-                const float r2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
-                float inv = __builtin_amdgcn_rsqf(r2);
-                if (MASK) inv = (r2 > 0.0f) ? inv : 0.0f;
-                const float s = (q.w * inv) * (inv * inv);
-                px[r] = fmaf(dx, s, px[r]);
-                py[r] = fmaf(dy, s, py[r]);
-                pz[r] = fmaf(dz, s, pz[r]);
-            }
+            bf_body<R, MASK>(sys[j0 + j], xi, yi, zi, eps2, px, py, pz);
         }
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            bt_kahan(ax[r], cx[r], px[r]);
-            bt_kahan(ay[r], cy[r], py[r]);
-            bt_kahan(az[r], cz[r], pz[r]);
+            kahan_add(ax[r], cx[r], px[r]);
+            kahan_add(ay[r], cy[r], py[r]);
+            kahan_add(az[r], cz[r], pz[r]);
         }
     }
 #pragma unroll
@@ -128,6 +114,69 @@ __global__ __launch_bounds__(256) void bt_force_kernel(const BatchItem* __restri
             case 4: bt_tile<4, MASK>(sh, w, eps2, acc); break;
             case 2: bt_tile<2, MASK>(sh, w, eps2, acc); break;
             default: bt_tile<1, MASK>(sh, w, eps2, acc); break;
+        }
+    }
+}
+
+// The same queue taken by workgroups: BT_WAVES wavefronts share an item, J of them its affecting
+// bodies (coop_sum; the same tiles summed in the same order, so the same bits) and, in systems with
+// fewer than BT_WAVES tiles of affecting bodies, the others neighbouring affected tiles: an item
+// covers BT_WAVES / J tiles of 64 R bodies.
+constexpr int BT_WAVES = 8;
+
+static __host__ __device__ inline int bt_share(uint32_t n) {  // wavefronts per affected tile
+    int j = 1;
+    while (j < BT_WAVES && uint32_t(j) * BT_TILE < n) j <<= 1;
+    return j;
+}
+
+template <int R, bool MASK>
+__device__ __forceinline__ void bt_coop_tile(CoopLds<BT_R_MAX, BT_WAVES>& lds_max,
+                                             const float4* __restrict__ sh, const BatchItem w,
+                                             int wave, float eps2, float4* __restrict__ acc) {
+    // smaller R use a prefix of the same memory
+    CoopLds<R, BT_WAVES>& lds = reinterpret_cast<CoopLds<R, BT_WAVES>&>(lds_max);
+    const uint32_t lane = threadIdx.x & 63;
+    const float4* sys = sh + w.off;
+    const int J = bt_share(w.n);
+    const uint32_t i0 = w.i0 + uint32_t(wave / J) * (64 * R);
+    float xi[R], yi[R], zi[R], ax[R], ay[R], az[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint32_t i = i0 + r * 64 + lane;
+        const float4 p = sys[i < w.n ? i : w.n - 1];
+        xi[r] = p.x; yi[r] = p.y; zi[r] = p.z;
+    }
+    coop_sum<R, MASK, false, BT_TILE, BT_WAVES>(lds, sys, 0, w.n, J, wave, i0 < w.n, eps2, 0, xi, yi,
+                                                zi, ax, ay, az);
+    if (wave % J != 0) return;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint32_t i = i0 + r * 64 + lane;
+        if (i < w.n) acc[w.off + i] = make_float4(ax[r], ay[r], az[r], 0.f);
+    }
+}
+
+template <bool MASK>
+__global__ __launch_bounds__(64 * BT_WAVES) void bt_coop_kernel(const BatchItem* __restrict__ items,
+                                                                uint32_t n_items,
+                                                                uint32_t* __restrict__ queue,
+                                                                const float4* __restrict__ sh,
+                                                                float eps2,
+                                                                float4* __restrict__ acc) {
+    __shared__ CoopLds<BT_R_MAX, BT_WAVES> lds;
+    __shared__ uint32_t next;
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+    while (true) {
+        if (threadIdx.x == 0) next = atomicAdd(queue, 1u);
+        __syncthreads();
+        const uint32_t it = __builtin_amdgcn_readfirstlane(next);
+        __syncthreads();  // everyone has read it before the next round's write
+        if (it >= n_items) break;
+        const BatchItem w = items[it];
+        switch (w.r) {
+            case 2: bt_coop_tile<2, MASK>(lds, sh, w, wave, eps2, acc); break;
+            default: bt_coop_tile<1, MASK>(lds, sh, w, wave, eps2, acc); break;
         }
     }
 }
@@ -196,17 +245,34 @@ static int per_lane_for(const BatchState* s, size_t n) {
     return n >= 256 ? 4 : 1;  // untuned default (what autotuning picks on MI355X)
 }
 
+// Whether a step's force pass is better taken by workgroups than by wavefronts: a wavefront needs
+// n r 13 instructions of 4.8 cycles for an item, and the first ones share their SIMDs with others,
+// so once a few times the longest item exceeds the whole pass at full rate the heavy items are
+// its tail. Measured with sizes log-uniform in 64 .. 16,384 (force pass, wavefronts / workgroups):
+// 128 systems 3.60 / 1.18 ms (4 x longest / pass = 8), 512 5.46 / 4.34 (2.0), 1,024 8.25 / 8.42
+// (1.0); one system of 16,384: 3.10 / 0.37 ms; 2,000 of 64 .. 500: 187 / 95 us.
+static bool use_coop(const BatchState* s) {
+    double longest = 0.0, pairs = 0.0;
+    for (size_t k = 0; k < s->systems; ++k) {
+        const double n = double(s->offsets[k + 1] - s->offsets[k]);
+        if (n > 0) longest = std::max(longest, n * per_lane_for(s, size_t(n)));
+        pairs += n * n;
+    }
+    return 3.5 * longest * 13 * 4.8 / 2.4e9 > pairs / 3.7e12;
+}
+
 static int build_items(pnb_ctx* c, BatchState* s) {
     std::vector<BatchItem> items;
-    std::vector<uint64_t> cost;
     s->interactions = 0;
+    s->coop = use_coop(s);
     for (size_t k = 0; k < s->systems; ++k) {
         const uint32_t off = uint32_t(s->offsets[k]);
         const uint32_t n = uint32_t(s->offsets[k + 1] - s->offsets[k]);
         if (n == 0) continue;
         s->interactions += (unsigned long long)n * n;
-        const uint32_t r = uint32_t(per_lane_for(s, n));
-        const uint32_t tile = 64 * r;
+        uint32_t r = uint32_t(per_lane_for(s, n));
+        if (s->coop) r = std::min<uint32_t>(r, BT_R_MAX);
+        const uint32_t tile = 64 * r * (s->coop ? uint32_t(BT_WAVES / bt_share(n)) : 1u);
         for (uint32_t i0 = 0; i0 < n; i0 += tile) items.push_back({off, n, i0, r});
     }
     std::stable_sort(items.begin(), items.end(), [](const BatchItem& a, const BatchItem& b) {
@@ -225,22 +291,18 @@ static int build_items(pnb_ctx* c, BatchState* s) {
 static int force(pnb_ctx* c, BatchState* s) {
     const bool mask = s->checked && s->softening == 0.0f;
     const float eps2 = s->softening * s->softening;
+    auto k = s->coop ? (mask ? bt_coop_kernel<true> : bt_coop_kernel<false>)
+                     : (mask ? bt_force_kernel<true> : bt_force_kernel<false>);
+    const unsigned block = s->coop ? 64 * BT_WAVES : 256;
     int occ = 0;
-    hipError_t e = mask ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, bt_force_kernel<true>, 256, 0)
-                        : hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, bt_force_kernel<false>, 256, 0);
-    if (e != hipSuccess || occ < 1) occ = 2;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k, int(block), 0) != hipSuccess || occ < 1) occ = 2;
     const unsigned grid = unsigned(std::max(1, c->cu_count) * occ);
     bt_queue_reset_kernel<<<1, 1, 0, c->stream>>>(s->queue.as<uint32_t>());
     PNB_CHECK_LAUNCH(c);
     return timed(c, PNB_PROF_BATCH, [&]() -> int {
-        if (mask)
-            bt_force_kernel<true><<<grid, 256, 0, c->stream>>>(s->items.as<BatchItem>(), uint32_t(s->n_items),
-                                                              s->queue.as<uint32_t>(), s->shadow.as<float4>(),
-                                                              eps2, s->acc.as<float4>());
-        else
-            bt_force_kernel<false><<<grid, 256, 0, c->stream>>>(s->items.as<BatchItem>(), uint32_t(s->n_items),
-                                                               s->queue.as<uint32_t>(), s->shadow.as<float4>(),
-                                                               eps2, s->acc.as<float4>());
+        k<<<grid, block, 0, c->stream>>>(s->items.as<BatchItem>(), uint32_t(s->n_items),
+                                         s->queue.as<uint32_t>(), s->shadow.as<float4>(), eps2,
+                                         s->acc.as<float4>());
         PNB_CHECK_LAUNCH(c);
         return PNB_OK;
     });

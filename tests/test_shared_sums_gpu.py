@@ -60,3 +60,30 @@ def test_pairs_own_term_only_is_left_out(res):
     p[8000] = p[17]
     bad = ~np.isfinite(pa.BruteForcePairs(res, pa.Acceleration.unchecked()).compute(p)).all(1)
     assert set(np.nonzero(bad)[0]) == {17, 8000}
+
+
+def test_ensemble_by_workgroups_equals_single_systems(res):
+    """Systems at the edges of tiles and groups, one large enough that the queue is taken by
+    workgroups: the bits of the brute-force kernel on each system alone."""
+    sizes = [1, 2, 63, 64, 65, 127, 255, 256, 257, 511, 513, 1025, 2047, 2049, 9001]
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
+    n = int(off[-1])
+    pos, vel = workloads.plummer(n, 5)
+    mu = np.random.default_rng(5).uniform(0.5, 1.5, n).astype(np.float32) / n
+    L = _lib.lib()
+    for eps in (0.0, 1e-3):
+        res.reset_stream()
+        res.check(L.pnb_batch_init(res.handle, pos.ctypes.data, vel.ctypes.data, mu.ctypes.data,
+                                   off.ctypes.data, len(sizes), eps, 1))
+        acc = np.zeros((n, 4), np.float32)
+        res.check(L.pnb_batch_read(res.handle, None, None, acc.ctypes.data))
+        res.set_bf_tuning(0, 1, 2, 1)
+        try:
+            for b, e in zip(off[:-1], off[1:]):
+                p = workloads.pack(pos[b:e], mu[b:e])
+                out = np.zeros((e - b, 4), np.float32)
+                res.check(L.pnb_bf_accel_f32(res.handle, p.ctypes.data, e - b, p.ctypes.data, e - b,
+                                             ctypes.c_float(eps), 1, out.ctypes.data))
+                np.testing.assert_array_equal(acc[b:e], out)
+        finally:
+            res.clear_bf_tuning()
