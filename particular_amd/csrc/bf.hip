@@ -81,7 +81,7 @@ __global__ __launch_bounds__(BF_BLOCK) void bf_kernel(const float4* __restrict__
         } else if (cnt == BF_TILE) {
 #pragma unroll 8
             for (int j = 0; j < BF_TILE; ++j)
-                bf_body<R, MASK>(LDS ? tile[j] : afg[j0 + j], xi, yi, zi, eps2, px, py, pz);
+                bf_body<R, MASK, false, R == 1>(LDS ? tile[j] : afg[j0 + j], xi, yi, zi, eps2, px, py, pz);
         } else {
             for (uint32_t j = 0; j < cnt; ++j)
                 bf_body<R, MASK>(LDS ? tile[j] : afg[j0 + j], xi, yi, zi, eps2, px, py, pz);
@@ -166,12 +166,6 @@ static BfKernel pick_mask(int r, bool mask) {
     return mask ? pick_r<true, VAR>(r) : pick_r<false, VAR>(r);
 }
 
-// One set on itself: the default shapes only (tuning entries are for two sets).
-template <bool MASK>
-static BfKernel pick_self(int r) {
-    return r == 4 ? bf_kernel<4, MASK, 1, true> : r == 2 ? bf_kernel<2, MASK, 0, true> : bf_kernel<1, MASK, 0, true>;
-}
-
 template <bool SELF>
 static BfKernel pick_coop(bool mask, int tile) {
     switch (tile) {
@@ -188,14 +182,16 @@ struct BfShape {
 };
 
 // What the cooperative kernel takes: sums small enough that wavefronts walking the affecting
-// bodies alone are bound by their own issue rate (a 1,024-body range takes one 34 us). Measured,
-// alone / cooperative, softened: 1,000 x 1,000 34 / 9 us; 4,096 x 4,096 36 / 15; 64 x 65,536
-// 51 / 17; 8,192 x 8,192 28 / 28 (6.7e7 pairs); 12,000 x 16,384 67 / 96. With few affecting bodies
-// the others have no range to split and it pays up to 2.5e8 pairs (65,536 x 1,000 78 / 28 us); with
-// at most one tile there is nothing to share (50,000 x 64: 4.2 / 7.4 us).
+// bodies alone are bound by their own issue rate (a 1,024-body range takes one 34 us), and sums
+// with few bodies on one side, which leave the others too few ranges or tiles. Measured, the best
+// split of the plain kernel / cooperative, softened: 1,000 x 1,000 34 / 8 us; 4,096 x 4,096 36 / 11;
+// 1,000 x 65,536 91 / 28; 4,096 x 65,536 102 / 96; 8,192 x 8,192 28 / 27 (6.7e7 pairs); 12,000 x
+// 16,384 67 / 92; 32,768 x 4,096 45 / 42; 300,000 x 5,000 385 / 430; 65,536 x 1,000 78 / 21;
+// 1,000,000 x 1,000 291 / 273; 50,000 x 64 4.2 / 7.4 (one tile: nothing to share).
 static bool coop_pays(size_t n, size_t m) {
     if (m <= 64 || (m <= 256 && n > 32768)) return false;
-    return n * m <= (m < 2048 ? size_t(250000000) : size_t(60000000));
+    const double pairs = double(n) * double(m);
+    return pairs <= (m < 2048 ? 1e9 : n <= 4096 ? 3e8 : m <= 4096 ? 1.5e8 : 7e7);
 }
 
 static BfShape default_shape(pnb_ctx* c, size_t n, size_t m) {
@@ -208,17 +204,19 @@ static BfShape default_shape(pnb_ctx* c, size_t n, size_t m) {
         while (s < 64 && blocks * s * 2 <= cus && m / (size_t(s) * 2) >= size_t(COOP_WAVES) * 64) s <<= 1;
         return {BF_COOP, 1, s};
     }
-    // Otherwise one wavefront per affected tile and range: bodies per lane by the affected count
-    // (register-blocked scalar loads from 131,072 on; below, more and smaller workgroups reading
-    // the affecting bodies from LDS, one per lane where there are few affecting bodies to split), and up to 64 workgroups per CU over the affecting range, of at
-    // least one tile (4 per lane) or two. Softened: 65,536 x 16,384 299 us with 2 per lane from LDS,
-    // 333 with 4 from scalar loads in ranges of 1,024; 500,000 x 20,000 2.53 ms with 4 per lane,
-    // 2.57 with 2.
-    const int r = n >= 131072 && m > 64 ? 4 : n >= 24576 && m >= 8192 ? 2 : 1;
-    const size_t blocks = div_up(n, size_t(BF_BLOCK) * r);
-    const size_t least = (r == 4 ? 1 : 2) * size_t(BF_TILE);
-    while (s < 64 && blocks * s * 2 <= 64 * cus && m / (size_t(s) * 2) >= least) s <<= 1;
-    return {r == 4 ? 1 : 0, r, s};
+    // Otherwise one body per lane and one wavefront per affected tile and range, the affecting
+    // bodies from scalar loads (from LDS below 32,768 affected bodies, where few wavefronts hide
+    // their latency, 12,000 x 16,384 67 / 70 us, and for at most a tile, 65,536 x 64 4 / 9 us), the affecting range split into up to 64 workgroups
+    // per CU of at least one tile each, up to 256 per CU while ranges stay at 1,024 bodies
+    // (small workgroups balance the load across CUs and XCDs). 1,048,576 x 65,536 16.1 ms, with four
+    // bodies per lane 17.1; 65,536 x 16,384 286 us, 333.
+    const size_t blocks = div_up(n, size_t(BF_BLOCK));
+    while (s < 64 && blocks * s * 2 <= 256 * cus) {
+        const size_t per = m / (size_t(s) * 2);
+        if (per < (blocks * s * 2 <= 64 * cus ? size_t(BF_TILE) : size_t(1024))) break;
+        s <<= 1;
+    }
+    return {n < 32768 || m <= 256 ? 0 : 1, 1, s};
 }
 
 static BfShape choose_shape(pnb_ctx* c, size_t n, size_t m) {
@@ -294,7 +292,8 @@ static int bf_launch_with(pnb_ctx* c, const BfPlan& p, const float4* affected, s
     const bool coop = sh.variant == BF_COOP;
     BfKernel k;
     if (coop) k = self ? pick_coop<true>(mask, p.tile) : pick_coop<false>(mask, p.tile);
-    else if (self) k = mask ? pick_self<true>(sh.per_lane) : pick_self<false>(sh.per_lane);
+    else if (self && sh.variant == 0) k = mask ? bf_kernel<1, true, 0, true> : bf_kernel<1, false, 0, true>;
+    else if (self) k = mask ? bf_kernel<1, true, 1, true> : bf_kernel<1, false, 1, true>;
     else k = sh.variant == 0 ? pick_mask<0>(sh.per_lane, mask) : pick_mask<1>(sh.per_lane, mask);
     const float eps2 = softening * softening;
     const uint32_t splits = p.splits, chunk = p.chunk;
