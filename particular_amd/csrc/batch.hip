@@ -2,15 +2,15 @@
 //
 // Every system is its own Between(system, system) brute force (all bodies massive within a
 // system), integrated with kick-drift-kick leapfrog in FP64 like the single-system loop. The force
-// pass of a step is ONE persistent launch: a few workgroups per CU whose wavefronts pull work
-// items (system, tile of 64*R affected bodies) from a queue until it is empty. Items are ordered by
-// decreasing cost (system size x tile size), so large systems start first and small ones fill the
-// tail. R (affected bodies per lane) is chosen per system-size bucket by the autotuner. Affecting
-// bodies are read with wave-uniform addresses (scalar loads), so wavefronts need no barriers and
-// run independently. The per-lane arithmetic and summation order are those of the brute-force
-// kernel (FP32 tiles of 256 bodies, Kahan across tiles). Ensembles whose largest systems would
-// outlast the rest take the queue by workgroups, which share an item's affecting bodies. A step is enqueue-only and can be
-// captured into a hipGraph (the queue counter is cleared by a kernel, not a memset).
+// pass of a step is ONE persistent launch: a few workgroups per CU that pull work items (system,
+// tiles of 64*R affected bodies) from a queue until it is empty, the wavefronts of a workgroup
+// sharing an item's affecting bodies (coop_sum), which they read with wave-uniform addresses
+// (scalar loads). Items are ordered by decreasing cost (system size x bodies per lane), so large
+// systems start first and small ones fill the tail. Tuning entries that ask for more than two
+// bodies per lane take the queue by single wavefronts, which need no barriers. The per-lane
+// arithmetic and summation order are those of the brute-force kernel either way (FP32 tiles of 256
+// bodies, Kahan across tiles). A step is enqueue-only and can be captured into a hipGraph (the queue
+// counter is cleared by a kernel, not a memset).
 #include "bf_common.hpp"
 #include "pnb_internal.hpp"
 
@@ -130,7 +130,7 @@ static __host__ __device__ inline int bt_share(uint32_t n) {  // wavefronts per 
     return j;
 }
 
-template <int R, bool MASK>
+template <int R, bool MASK, bool SEQ>
 __device__ __forceinline__ void bt_coop_tile(CoopLds<BT_R_MAX, BT_WAVES>& lds_max,
                                              const float4* __restrict__ sh, const BatchItem w,
                                              int wave, float eps2, float4* __restrict__ acc) {
@@ -147,7 +147,7 @@ __device__ __forceinline__ void bt_coop_tile(CoopLds<BT_R_MAX, BT_WAVES>& lds_ma
         const float4 p = sys[i < w.n ? i : w.n - 1];
         xi[r] = p.x; yi[r] = p.y; zi[r] = p.z;
     }
-    coop_sum<R, MASK, false, BT_TILE, BT_WAVES>(lds, sys, 0, w.n, J, wave, i0 < w.n, eps2, 0, xi, yi,
+    coop_sum<R, MASK, false, BT_TILE, BT_WAVES, SEQ>(lds, sys, 0, w.n, J, wave, i0 < w.n, eps2, 0, xi, yi,
                                                 zi, ax, ay, az);
     if (wave % J != 0) return;
 #pragma unroll
@@ -157,7 +157,7 @@ __device__ __forceinline__ void bt_coop_tile(CoopLds<BT_R_MAX, BT_WAVES>& lds_ma
     }
 }
 
-template <bool MASK>
+template <bool MASK, bool SEQ>
 __global__ __launch_bounds__(64 * BT_WAVES) void bt_coop_kernel(const BatchItem* __restrict__ items,
                                                                 uint32_t n_items,
                                                                 uint32_t* __restrict__ queue,
@@ -175,8 +175,8 @@ __global__ __launch_bounds__(64 * BT_WAVES) void bt_coop_kernel(const BatchItem*
         if (it >= n_items) break;
         const BatchItem w = items[it];
         switch (w.r) {
-            case 2: bt_coop_tile<2, MASK>(lds, sh, w, wave, eps2, acc); break;
-            default: bt_coop_tile<1, MASK>(lds, sh, w, wave, eps2, acc); break;
+            case 2: bt_coop_tile<2, MASK, SEQ>(lds, sh, w, wave, eps2, acc); break;
+            default: bt_coop_tile<1, MASK, SEQ>(lds, sh, w, wave, eps2, acc); break;
         }
     }
 }
@@ -233,7 +233,8 @@ __global__ void bt_unpack_kernel(const double4* __restrict__ x, const double4* _
     out[3 * (n + i)] = b.x; out[3 * (n + i) + 1] = b.y; out[3 * (n + i) + 2] = b.z;
 }
 
-static int per_lane_for(const BatchState* s, size_t n) {
+// A tuning entry's bodies per lane for systems of n bodies, 0 without one.
+static int tuned_per_lane(const BatchState* s, size_t n) {
     int r = 0;
     size_t best = 0;
     for (const auto& t : s->tuning)
@@ -241,37 +242,32 @@ static int per_lane_for(const BatchState* s, size_t n) {
             best = t.first;
             r = t.second;
         }
-    if (r) return r;
-    return n >= 256 ? 4 : 1;  // untuned default (what autotuning picks on MI355X)
+    return r;
 }
 
-// Whether a step's force pass is better taken by workgroups than by wavefronts: a wavefront needs
-// n r 13 instructions of 4.8 cycles for an item, and the first ones share their SIMDs with others,
-// so once a few times the longest item exceeds the whole pass at full rate the heavy items are
-// its tail. Measured with sizes log-uniform in 64 .. 16,384 (force pass, wavefronts / workgroups):
-// 128 systems 3.60 / 1.18 ms (4 x longest / pass = 8), 512 5.46 / 4.34 (2.0), 1,024 8.25 / 8.42
-// (1.0); one system of 16,384: 3.10 / 0.37 ms; 2,000 of 64 .. 500: 187 / 95 us.
-static bool use_coop(const BatchState* s) {
-    double longest = 0.0, pairs = 0.0;
-    for (size_t k = 0; k < s->systems; ++k) {
-        const double n = double(s->offsets[k + 1] - s->offsets[k]);
-        if (n > 0) longest = std::max(longest, n * per_lane_for(s, size_t(n)));
-        pairs += n * n;
-    }
-    return 3.5 * longest * 13 * 4.8 / 2.4e9 > pairs / 3.7e12;
+// Bodies per lane of a system's items. Untuned: two, one for systems with at most half a
+// workgroup's lanes.
+static uint32_t per_lane_for(const BatchState* s, size_t n) {
+    const int r = tuned_per_lane(s, n);
+    return uint32_t(r ? r : n >= 256 ? 2 : 1);
 }
 
 static int build_items(pnb_ctx* c, BatchState* s) {
     std::vector<BatchItem> items;
     s->interactions = 0;
-    s->coop = use_coop(s);
+    // Workgroups share the items unless a tuning entry asks for more bodies per lane than they
+    // hold. Force pass, wavefronts with 4 per lane / workgroups with 2: one system of 16,384 bodies
+    // 3.10 / 0.37 ms; sizes log-uniform in 64 .. 16,384: 128 systems 3.60 / 1.09, 1,024 8.25 /
+    // 7.00, 2,048 13.9 / 13.4; 512 of 64 .. 65,536 45.4 / 41.5; 2,000 of 64 .. 500 187 / 90 us.
+    s->coop = true;
+    for (size_t k = 0; k < s->systems && s->coop; ++k)
+        s->coop = tuned_per_lane(s, size_t(s->offsets[k + 1] - s->offsets[k])) <= BT_R_MAX;
     for (size_t k = 0; k < s->systems; ++k) {
         const uint32_t off = uint32_t(s->offsets[k]);
         const uint32_t n = uint32_t(s->offsets[k + 1] - s->offsets[k]);
         if (n == 0) continue;
         s->interactions += (unsigned long long)n * n;
-        uint32_t r = uint32_t(per_lane_for(s, n));
-        if (s->coop) r = std::min<uint32_t>(r, BT_R_MAX);
+        const uint32_t r = per_lane_for(s, n);
         const uint32_t tile = 64 * r * (s->coop ? uint32_t(BT_WAVES / bt_share(n)) : 1u);
         for (uint32_t i0 = 0; i0 < n; i0 += tile) items.push_back({off, n, i0, r});
     }
@@ -291,8 +287,12 @@ static int build_items(pnb_ctx* c, BatchState* s) {
 static int force(pnb_ctx* c, BatchState* s) {
     const bool mask = s->checked && s->softening == 0.0f;
     const float eps2 = s->softening * s->softening;
-    auto k = s->coop ? (mask ? bt_coop_kernel<true> : bt_coop_kernel<false>)
-                     : (mask ? bt_force_kernel<true> : bt_force_kernel<false>);
+    // terms in source order once the items give every SIMD four wavefronts (bf_body); below that
+    // 16 systems of 64 .. 500 bodies take 41 us so, 32 us otherwise
+    const bool seq = s->n_items * BT_WAVES >= size_t(16) * std::max(1, c->cu_count);
+    auto k = !s->coop ? (mask ? bt_force_kernel<true> : bt_force_kernel<false>)
+             : seq    ? (mask ? bt_coop_kernel<true, true> : bt_coop_kernel<false, true>)
+                      : (mask ? bt_coop_kernel<true, false> : bt_coop_kernel<false, false>);
     const unsigned block = s->coop ? 64 * BT_WAVES : 256;
     int occ = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k, int(block), 0) != hipSuccess || occ < 1) occ = 2;
