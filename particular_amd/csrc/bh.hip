@@ -51,7 +51,7 @@ namespace pnb {
 int radix_sort_pairs(pnb_ctx* c, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
                      uint32_t* vals_alt, size_t n, int key_bits, DevBuf& hist_buf,
                      DevBuf& bits_buf, uint64_t** keys_out, uint32_t** vals_out,
-                     bool all_digits = false);
+                     bool all_digits = false, int low_bit = 0);
 int split_affecting(pnb_ctx* c, const float4* particles, size_t n, float4* dst, uint32_t* m_host);
 
 constexpr int KEY_LEVELS = 21;
@@ -2318,9 +2318,13 @@ static int accel_dev(pnb_ctx* c, const float4* affected, size_t n, const float4*
     PNB_CHECK_LAUNCH(c);
     uint64_t* sk;
     uint32_t* si;
+    // Only neighbours together: thirteen levels of the key (39 bits, five digits instead of eight)
+    // put 64 particles into cells 2^-13 of the box apart; below that any order serves, and none
+    // changes a result.
+    constexpr int AFFECTED_LOW_BIT = 23;
     if (int rc = radix_sort_pairs(c, s->akeys.as<uint64_t>(), s->aidx.as<uint32_t>(),
                                   s->akeys_alt.as<uint64_t>(), s->aidx_alt.as<uint32_t>(), n, 63,
-                                  s->hist, s->bits, &sk, &si, dd))
+                                  s->hist, s->bits, &sk, &si, dd, AFFECTED_LOW_BIT))
         return rc;
     bh_gather_kernel<<<g, 256, 0, c->stream>>>(affected, n, si, s->apts.as<float4>());
     PNB_CHECK_LAUNCH(c);

@@ -94,6 +94,120 @@ __global__ __launch_bounds__(RS_BLOCK) void rs_scatter_kernel(
     }
 }
 
+// Middle sizes, up to MID_SORT pairs: one launch per digit. A launch's cost there is its latency (the
+// five launches a digit takes below come to 25 us for 100,000 keys, 0.2 ms for the eight digits),
+// so the histograms of a digit are counted by the previous digit's scatter (a key's next tile is
+// known once its place is; atomics on a tile's 256 counters) and every workgroup adds up the
+// tiles' counters itself: tiles x 256 counters, at most 256 KiB, read from L2 in two halves.
+// Measured with its launches: 100,003 keys 99 us, 222 with the five launches a digit; 262,144: 170 / 251.
+constexpr size_t MID_SORT = 262144;
+constexpr int MS_BLOCK = 512;
+constexpr int MS_WAVES = MS_BLOCK / 64;
+constexpr int MS_ROUNDS = 2;                   // 64-key rounds per wave
+constexpr int MS_TILE = MS_BLOCK * MS_ROUNDS;  // 1024 keys per workgroup
+
+// Histograms (tile-major) of the first digit, and zeros for the later digits' (hist + k tiles 256).
+__global__ __launch_bounds__(256) void ms_hist_kernel(const uint64_t* __restrict__ keys, size_t n,
+                                                      int shift, uint32_t* __restrict__ hist,
+                                                      uint32_t tiles, int digits) {
+    __shared__ uint32_t h[256];
+    h[threadIdx.x] = 0;
+    __syncthreads();
+    const size_t base = size_t(blockIdx.x) * MS_TILE;
+#pragma unroll
+    for (int k = 0; k < MS_TILE / 256; ++k) {
+        const size_t i = base + size_t(k) * 256 + threadIdx.x;
+        if (i < n) atomicAdd(&h[(keys[i] >> shift) & 0xffu], 1u);
+    }
+    __syncthreads();
+    const size_t at = size_t(blockIdx.x) * 256 + threadIdx.x;
+    hist[at] = h[threadIdx.x];
+    for (int k = 1; k < digits; ++k) hist[size_t(k) * tiles * 256 + at] = 0u;
+}
+
+__global__ __launch_bounds__(MS_BLOCK) void ms_pass_kernel(
+    const uint64_t* __restrict__ keys, const uint32_t* __restrict__ vals, size_t n, int shift,
+    const uint32_t* __restrict__ hist, uint32_t* __restrict__ next, uint32_t tiles,
+    uint64_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out) {
+    __shared__ uint32_t wcnt[MS_WAVES][256];
+    __shared__ uint32_t sum[2][2][256];  // per half of the tiles: all of them, those before this one
+    __shared__ uint32_t wsum[4];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int d = threadIdx.x & 255, half = threadIdx.x >> 8;
+    const uint32_t mine = blockIdx.x, mid = (tiles + 1) / 2;
+    // this tile's keys are requested before the counters, so that their latencies overlap
+    const size_t seg = size_t(mine) * MS_TILE + size_t(w) * (64 * MS_ROUNDS);
+    uint64_t key[MS_ROUNDS];
+    uint32_t val[MS_ROUNDS], rank[MS_ROUNDS];
+#pragma unroll
+    for (int r = 0; r < MS_ROUNDS; ++r) {
+        const size_t i = seg + size_t(r) * 64 + lane;
+        key[r] = i < n ? keys[i] : 0ull;
+        val[r] = i < n ? vals[i] : 0u;
+    }
+    uint32_t all = 0, before = 0;
+    const uint32_t t0 = half ? mid : 0u, t1 = half ? tiles : mid;
+#pragma unroll 16
+    for (uint32_t t = t0; t < t1; ++t) {
+        const uint32_t c = hist[size_t(t) * 256 + d];
+        all += c;
+        before += t < mine ? c : 0u;
+    }
+    sum[half][0][d] = all;
+    sum[half][1][d] = before;
+    for (int q = lane; q < 256; q += 64) wcnt[w][q] = 0;
+    __syncthreads();
+    // exclusive scan of the digits' totals over the first four wavefronts
+    uint32_t total = 0, incl = 0;
+    if (half == 0) {
+        total = sum[0][0][d] + sum[1][0][d];
+        incl = total;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += y;
+        }
+        if (lane == 63) wsum[w] = incl;
+    }
+    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+    for (int r = 0; r < MS_ROUNDS; ++r) {
+        const bool valid = seg + size_t(r) * 64 + lane < n;
+        const uint32_t dg = uint32_t(key[r] >> shift) & 0xffu;
+        uint64_t peers = __ballot(valid);
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            const uint64_t bal = __ballot((dg >> b) & 1u);
+            peers &= ((dg >> b) & 1u) ? bal : ~bal;
+        }
+        const uint32_t run = wcnt[w][dg];
+        rank[r] = run + uint32_t(__popcll(peers & lt_mask));
+        if (valid && (peers & lt_mask) == 0) wcnt[w][dg] = run + uint32_t(__popcll(peers));
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    if (half == 0) {
+        uint32_t run = incl - total + sum[0][1][d] + sum[1][1][d];
+        for (int q = 0; q < w; ++q) run += wsum[q];
+#pragma unroll
+        for (int ww = 0; ww < MS_WAVES; ++ww) {
+            const uint32_t c = wcnt[ww][d];
+            wcnt[ww][d] = run;
+            run += c;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < MS_ROUNDS; ++r) {
+        if (seg + size_t(r) * 64 + lane >= n) continue;
+        const uint32_t pos = wcnt[w][uint32_t(key[r] >> shift) & 0xffu] + rank[r];
+        keys_out[pos] = key[r];
+        vals_out[pos] = val[r];
+        if (next)
+            atomicAdd(&next[size_t(pos / MS_TILE) * 256 + (uint32_t(key[r] >> (shift + 8)) & 0xffu)], 1u);
+    }
+}
+
 __global__ __launch_bounds__(256) void rs_bits_kernel(const uint64_t* __restrict__ keys, size_t n,
                                                       unsigned long long* __restrict__ or_and) {
     unsigned long long o = 0ull, a = ~0ull;
@@ -207,14 +321,15 @@ __global__ __launch_bounds__(256) void rank_scatter_kernel(const uint64_t* __res
 }
 
 // Sorts keys[0..n) with their values, stably; the result ends in (*keys_out, *vals_out), which is
-// either the input pair or the alternate pair. Only bits [0, key_bits) are considered. Up to
+// either the input pair or the alternate pair. Only bits [0, key_bits) are considered, and above
+// SMALL_SORT pairs only bits from low_bit on (a caller that wants neighbours together, not an order). Up to
 // SMALL_SORT pairs (keys of at most 63 bits) are ranked by counting, into the alternate pair;
 // either way equal keys keep their input order.
 // Digits no two keys differ in are skipped after one read-back to the host, unless all_digits.
 int radix_sort_pairs(pnb_ctx* c, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
                      uint32_t* vals_alt, size_t n, int key_bits, DevBuf& hist_buf,
                      DevBuf& bits_buf, uint64_t** keys_out, uint32_t** vals_out,
-                     bool all_digits) {
+                     bool all_digits, int low_bit) {
     *keys_out = keys;
     *vals_out = vals;
     if (n <= 1) return PNB_OK;
@@ -240,6 +355,26 @@ int radix_sort_pairs(pnb_ctx* c, uint64_t* keys, uint32_t* vals, uint64_t* keys_
         return PNB_OK;
     }
     if (n > 0xffffffffu) return fail(c, PNB_E_ARG, "radix sort supports at most 2^32-1 keys");
+    if (n <= MID_SORT) {
+        const uint32_t tiles = div_up(n, MS_TILE);
+        const int digits = (key_bits - low_bit + 7) / 8;
+        PNB_HIP(c, hist_buf.ensure(size_t(digits) * tiles * 256 * sizeof(uint32_t)));
+        uint32_t* hist = hist_buf.as<uint32_t>();
+        ms_hist_kernel<<<tiles, 256, 0, c->stream>>>(keys, n, low_bit, hist, tiles, digits);
+        PNB_CHECK_LAUNCH(c);
+        for (int k = 0; k < digits; ++k) {
+            uint32_t* h = hist + size_t(k) * tiles * 256;
+            ms_pass_kernel<<<tiles, MS_BLOCK, 0, c->stream>>>(
+                keys, vals, n, low_bit + 8 * k, h, k + 1 < digits ? h + size_t(tiles) * 256 : nullptr,
+                tiles, keys_alt, vals_alt);
+            PNB_CHECK_LAUNCH(c);
+            std::swap(keys, keys_alt);
+            std::swap(vals, vals_alt);
+        }
+        *keys_out = keys;
+        *vals_out = vals;
+        return PNB_OK;
+    }
     const uint32_t tiles = div_up(n, RS_TILE);
     PNB_HIP(c, hist_buf.ensure((size_t(256) * tiles + 1) * sizeof(uint32_t)));
     // one digit: sorted in one pass, no need to look for it first; all_digits: every pass runs
@@ -261,7 +396,7 @@ int radix_sort_pairs(pnb_ctx* c, uint64_t* keys, uint32_t* vals, uint64_t* keys_
     uint32_t* hist = hist_buf.as<uint32_t>();
     uint64_t *kin = keys, *kout = keys_alt;
     uint32_t *vin = vals, *vout = vals_alt;
-    for (int shift = 0; shift < key_bits; shift += 8) {
+    for (int shift = low_bit; shift < key_bits; shift += 8) {
         if (((varying >> shift) & 0xffull) == 0) continue;
         rs_hist_kernel<<<tiles, RS_BLOCK, 0, c->stream>>>(kin, n, shift, hist, tiles);
         PNB_CHECK_LAUNCH(c);
