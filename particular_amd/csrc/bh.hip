@@ -129,6 +129,7 @@ struct BhState {
     const uint32_t* sidx = nullptr;   // tree order -> original index
     DevBuf keys, keys_alt, idx, idx_alt, sp, lcp, cnt, ip, key2, rec, sums, level, width;
     DevBuf skipv;            // per node: the skip pointer alone (the bottom-up pass's child walk)
+    DevBuf kids;             // per internal node: its children's indices (the batched walk)
     DevBuf ilist;            // internal nodes grouped by level (bottom-up pass)
     DevBuf lvl;              // padded per-level counts and list cursors (2 x LVL_SLOTS lines)
     DevBuf mom, quad, desc;  // second moments (FP64), normalised quadrupoles, child shares
@@ -146,7 +147,7 @@ struct BhState {
     DevBuf info, bbox_part, hist, bits, afg_tmp;
     // capturable builds (pnb_bh_set_capturable): sized once by an ordinary build, then no host
     // round trip; dd_last: the last build's node count and status are only on the device
-    bool dd_mode = false, dd_last = false, dd_mlp = false;
+    bool dd_mode = false, dd_last = false, dd_mlp = false, dd_kids = false;
     size_t dd_m = 0, dd_n = 0, dd_cap = 0;
     int dd_levels = 0;
     std::vector<uint32_t> last_lvl;  // internal nodes per level of the last ordinary build
@@ -165,7 +166,7 @@ struct BhState {
 void bh_free(BhState* s) {
     if (!s) return;
     for (DevBuf* b : {&s->keys, &s->keys_alt, &s->idx, &s->idx_alt, &s->sp, &s->lcp, &s->cnt,
-                      &s->ip, &s->key2, &s->rec, &s->sums, &s->level, &s->width, &s->skipv,
+                      &s->ip, &s->key2, &s->rec, &s->sums, &s->level, &s->width, &s->skipv, &s->kids,
                       &s->ilist, &s->lvl, &s->mom, &s->quad, &s->desc, &s->qh, &s->oh, &s->rrec, &s->est,
                       &s->cen, &s->cen_spread, &s->est_spread, &s->wkey, &s->wkey_alt, &s->wval, &s->wval_alt,
                       &s->info, &s->bbox_part, &s->hist, &s->bits, &s->afg_tmp, &s->akeys,
@@ -678,6 +679,7 @@ __global__ __launch_bounds__(256) void bh_node_kernel(
 // (impls/mod.rs:126-131: mass-weighted mean, or the plain mean when the total mass is 0).
 // With `mom`, also the second moments by the parallel-axis rule
 // T = sum over children of (T_c + M_c (c_c - c)(c_c - c)^T), and the normalised quadrupole.
+// With `kids`, also the child table the batched walk reads (bh_list.hpp).
 // One internal node k: its sums from its children's (and, with moments, its second and third
 // moments, normalised quadrupole and octupole), its record's centre of mass and mass.
 __device__ __forceinline__ void up_node(uint32_t k, NodeRec* __restrict__ rec,
@@ -687,9 +689,11 @@ __device__ __forceinline__ void up_node(uint32_t k, NodeRec* __restrict__ rec,
                                         NodeDesc* __restrict__ desc,
                                         const float* __restrict__ width,
                                         const uint32_t* __restrict__ skipv,
-                                        const float4* __restrict__ sp) {
+                                        const float4* __restrict__ sp,
+                                        uint32_t* __restrict__ kids) {
     {
         const NodeRec r = rec[k];
+        int nkids = 0;
         double4 a = make_double4(0, 0, 0, 0);
         // with moments, in the same pass over the children: the second and third moments about
         // o (the first massive child's centre of mass) by the parallel-axis rule, with
@@ -704,6 +708,7 @@ __device__ __forceinline__ void up_node(uint32_t k, NodeRec* __restrict__ rec,
             const double4 s1 = sums[c].m;
             a.x += s1.x; a.y += s1.y; a.z += s1.z; a.w += s1.w;
             const uint32_t nx = skipv[c];
+            if (kids) kids[8 * size_t(k) + nkids++] = uint32_t(c);
             if (mom) {
                 if (s1.x > 0.0) {
                     const NodeMoments tc = nx == c + 1 ? NodeMoments{} : mom[c];
@@ -737,6 +742,7 @@ __device__ __forceinline__ void up_node(uint32_t k, NodeRec* __restrict__ rec,
             }
             c = nx > c ? nx : c + 1;
         }
+        if (kids) kids[8 * size_t(k)] = (k + 1) | (uint32_t(nkids - 1) << 28);
         sums[k].m = a;
         float cx, cy, cz;
         if (a.x != 0.0) {
@@ -842,10 +848,11 @@ __global__ __launch_bounds__(256) void bh_up_kernel(NodeRec* __restrict__ rec,
                                                     NodeDesc* __restrict__ desc,
                                                     const float* __restrict__ width,
                                                     const uint32_t* __restrict__ skipv,
-                                                    const float4* __restrict__ sp) {
+                                                    const float4* __restrict__ sp,
+                                                    uint32_t* __restrict__ kids) {
     for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < count;
          t += gridDim.x * blockDim.x)
-        up_node(nodes_at_level[t], rec, sums, MOM ? mom : nullptr, quad, desc, width, skipv, sp);
+        up_node(nodes_at_level[t], rec, sums, MOM ? mom : nullptr, quad, desc, width, skipv, sp, kids);
 }
 
 // Consecutive small levels (deepest first) in one workgroup: a barrier between levels makes one
@@ -867,11 +874,12 @@ __global__ __launch_bounds__(1024) void bh_up_run_kernel(NodeRec* __restrict__ r
                                                          NodeDesc* __restrict__ desc,
                                                          const float* __restrict__ width,
                                                          const uint32_t* __restrict__ skipv,
-                                                         const float4* __restrict__ sp) {
+                                                         const float4* __restrict__ sp,
+                                                         uint32_t* __restrict__ kids) {
     for (int j = 0; j < run.levels; ++j) {
         for (uint32_t t = threadIdx.x; t < run.cnt[j]; t += blockDim.x)
             up_node(ilist[run.off[j] + t], rec, sums, MOM ? mom : nullptr, quad, desc, width, skipv,
-                    sp);
+                    sp, kids);
         __syncthreads();
     }
 }
@@ -900,11 +908,12 @@ __global__ __launch_bounds__(256) void bh_up_level_dd_kernel(NodeRec* __restrict
                                                              NodeMoments* __restrict__ mom,
                                                              NodeQuad* __restrict__ quad,
                                                              NodeDesc* __restrict__ desc,
-                                                             const float* __restrict__ width) {
+                                                             const float* __restrict__ width,
+                                                             uint32_t* __restrict__ kids) {
     if (info->flags) return;
     const uint32_t cnt = info->lvl_count[level], off = info->lvl_off[level];
     for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < cnt; t += gridDim.x * blockDim.x)
-        up_node(ilist[off + t], rec, sums, MOM ? mom : nullptr, quad, desc, width, skipv, sp);
+        up_node(ilist[off + t], rec, sums, MOM ? mom : nullptr, quad, desc, width, skipv, sp, kids);
 }
 
 // A run of levels hi, hi - 1, ..., lo in one workgroup, a barrier between levels (levels the tree
@@ -920,13 +929,14 @@ __global__ __launch_bounds__(1024) void bh_up_levels_dd_kernel(NodeRec* __restri
                                                                NodeMoments* __restrict__ mom,
                                                                NodeQuad* __restrict__ quad,
                                                                NodeDesc* __restrict__ desc,
-                                                               const float* __restrict__ width) {
+                                                               const float* __restrict__ width,
+                                                               uint32_t* __restrict__ kids) {
     if (info->flags) return;  // uniform: every thread returns, or none
     for (int L = hi; L >= lo; --L) {
         const uint32_t cnt = info->lvl_count[L], off = info->lvl_off[L];
         for (uint32_t t = threadIdx.x; t < cnt; t += blockDim.x)
             up_node(ilist[off + t], rec, sums, MOM ? mom : nullptr, quad, desc, width, skipv,
-                    sp);
+                    sp, kids);
         __syncthreads();
     }
 }
@@ -1627,10 +1637,12 @@ __global__ __launch_bounds__(256) void bh_walk_kernel(const NodeRec* __restrict_
     }
 }
 
+#include "bh_list.hpp"
+
 // ---- host side --------------------------------------------------------------------------------
 
 static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = false,
-                      bool moments = false) {
+                      bool moments = false, bool children = false) {
     if (!c->bh) c->bh = new BhState();
     BhState* s = c->bh;
     s->built = false;
@@ -1728,6 +1740,11 @@ static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = fa
         NodeRec* rec = s->rec.as<NodeRec>();
         PNB_HIP(c, s->skipv.ensure(size_t(total) * sizeof(uint32_t)));
         uint32_t* skipv = s->skipv.as<uint32_t>();
+        uint32_t* kids = nullptr;
+        if (children) {
+            PNB_HIP(c, s->kids.ensure(size_t(total) * 8 * sizeof(uint32_t)));
+            kids = s->kids.as<uint32_t>();
+        }
         bh_node_kernel<<<g, 256, 0, c->stream>>>(sk, s->sp.as<float4>(), lcp, s->ip.as<int>(),
                                                  cnt, m, info, rec, s->sums.as<NodeSums>(),
                                                  s->level.as<uint8_t>(),
@@ -1750,7 +1767,7 @@ static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = fa
                 (mom ? bh_up_kernel<true> : bh_up_kernel<false>)<<<div_up(n_l, 256), 256, 0,
                                                                    c->stream>>>(
                     rec, s->sums.as<NodeSums>(), ilist + off[L], n_l, mom, quad,
-                    desc, s->width.as<float>(), skipv, s->sp.as<float4>());
+                    desc, s->width.as<float>(), skipv, s->sp.as<float4>(), kids);
                 PNB_CHECK_LAUNCH(c);
                 --L;
                 continue;
@@ -1763,7 +1780,7 @@ static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = fa
             }
             (mom ? bh_up_run_kernel<true> : bh_up_run_kernel<false>)<<<1, 1024, 0, c->stream>>>(
                 rec, s->sums.as<NodeSums>(), ilist, run, mom, quad, desc, s->width.as<float>(),
-                skipv, s->sp.as<float4>());
+                skipv, s->sp.as<float4>(), kids);
             PNB_CHECK_LAUNCH(c);
         }
         s->has_moments = moments;
@@ -1807,7 +1824,7 @@ static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = fa
 // Capacities of a capturable build from an ordinary build of the same size (its node count and
 // depth known on the host): a quarter more nodes and 8 more levels, so that later trees of
 // similar inputs fit.
-static int dd_size(pnb_ctx* c, size_t m, bool mlp) {
+static int dd_size(pnb_ctx* c, size_t m, bool mlp, bool children) {
     BhState* s = c->bh;
     const size_t cap = s->nodes + s->nodes / 4 + 1024;
     if (cap + 1 >= (size_t(1) << 27))
@@ -1817,6 +1834,7 @@ static int dd_size(pnb_ctx* c, size_t m, bool mlp) {
     PNB_HIP(c, s->level.ensure(cap));
     PNB_HIP(c, s->width.ensure(cap * sizeof(float)));
     PNB_HIP(c, s->skipv.ensure(cap * sizeof(uint32_t)));
+    if (children) PNB_HIP(c, s->kids.ensure(cap * 8 * sizeof(uint32_t)));
     PNB_HIP(c, s->ilist.ensure(cap * sizeof(uint32_t)));
     if (mlp) {  // the learned correction's node data and walk entries
         PNB_HIP(c, s->mom.ensure(cap * sizeof(NodeMoments)));
@@ -1826,6 +1844,7 @@ static int dd_size(pnb_ctx* c, size_t m, bool mlp) {
         PNB_HIP(c, s->oh.ensure((cap + 1) * sizeof(OctH)));
     }
     s->dd_mlp = mlp;
+    s->dd_kids = children;
     s->dd_cap = cap;
     s->dd_levels = std::min(std::max(s->max_level, 0) + 8, MAX_LEVEL + 1);
     s->dd_plan = s->last_lvl;
@@ -1836,7 +1855,7 @@ static int dd_size(pnb_ctx* c, size_t m, bool mlp) {
 // The octree of a capturable build: the ordinary build's kernels with no host round trip (every
 // digit of the sort, the node count checked and used on the device, the bottom-up sums launched
 // for every level up to the sized depth). Buffers were sized by dd_size for these m.
-static int build_tree_dd(pnb_ctx* c, const float4* afg, size_t m, bool moments) {
+static int build_tree_dd(pnb_ctx* c, const float4* afg, size_t m, bool moments, bool children) {
     BhState* s = c->bh;
     s->built = false;
     s->has_moments = false;
@@ -1897,6 +1916,7 @@ static int build_tree_dd(pnb_ctx* c, const float4* afg, size_t m, bool moments) 
         NodeQuad* quad = moments ? s->quad.as<NodeQuad>() : nullptr;
         NodeDesc* desc = moments ? s->desc.as<NodeDesc>() : nullptr;
         const float* width = s->width.as<float>();
+        uint32_t* kids = children ? s->kids.as<uint32_t>() : nullptr;
         bh_node_kernel<<<g, 256, 0, c->stream>>>(sk, sp, lcp, s->ip.as<int>(), cnt, m, info, rec,
                                                  s->sums.as<NodeSums>(), s->level.as<uint8_t>(),
                                                  s->width.as<float>(), mom, quad, skipv);
@@ -1919,7 +1939,7 @@ static int build_tree_dd(pnb_ctx* c, const float4* afg, size_t m, bool moments) 
                 const unsigned ug = std::min<unsigned>(div_up(n_l + n_l / 4, 256u), max_grid);
                 (mom ? bh_up_level_dd_kernel<true> : bh_up_level_dd_kernel<false>)<<<
                     ug, 256, 0, c->stream>>>(rec, s->sums.as<NodeSums>(), ilist, info, L, skipv,
-                                             sp, mom, quad, desc, width);
+                                             sp, mom, quad, desc, width, kids);
                 PNB_CHECK_LAUNCH(c);
                 --L;
                 continue;
@@ -1928,7 +1948,7 @@ static int build_tree_dd(pnb_ctx* c, const float4* afg, size_t m, bool moments) 
             while (L >= 0 && planned(L) <= UP_RUN_NODES / 2) --L;
             (mom ? bh_up_levels_dd_kernel<true> : bh_up_levels_dd_kernel<false>)<<<
                 1, 1024, 0, c->stream>>>(rec, s->sums.as<NodeSums>(), ilist, info, hi, L + 1, skipv,
-                                         sp, mom, quad, desc, width);
+                                         sp, mom, quad, desc, width, kids);
             PNB_CHECK_LAUNCH(c);
         }
         s->has_moments = moments;
@@ -2086,6 +2106,21 @@ static uint32_t walk_lanes(const pnb_ctx* c, size_t n) {
     return lanes;
 }
 
+// Particles per wavefront of the batched walk (bh_list_kernel), or 0 for the stackless one.
+// It pays while the stackless walk's wavefronts are too few to hide its latency; with more, the
+// work per particle decides, and a batched wavefront has fewer particles to share its rounds.
+// Walk at theta = 0.5, stackless / 4 / 16 particles per wavefront (us): plain, 1,000 bodies 71 /
+// 47 / 73; 4,096: 182 / 106 / 159; 20,000: 379 / 246 / 282; 30,000: - / 336 / 310; 50,000: 601 / 540
+// / 477; 100,003: 750 / 1,043 / 805. Corrected (no ordered sum, so nearly as cheap as plain):
+// 1,000: 100 / 45 / 99; 4,096: 321 / 100 / 226; 20,000: 739 / 241 / 416; 100,003: 1,605 / 1,047 /
+// 1,192; 262,144: 2,357 / 2,938 / 3,183.
+// PNB_WALK_LANES and PNB_WIDE_WALK name forms of the stackless walk.
+static int list_lanes(size_t n, bool mlp) {
+    if (std::getenv("PNB_WALK_LANES") || std::getenv("PNB_WIDE_WALK")) return 0;
+    if (mlp) return n <= 160000 ? 4 : 0;
+    return n <= 20000 ? 4 : n <= 75000 ? 16 : 0;
+}
+
 // quad: add the learned correction (the per-node moments in s->qh). rel: the relative criterion
 // in addition to the geometric one: an estimate pass (plain walk at s->rel_theta_est) gives
 // alpha |a~| per particle or, by default, per wavefront at the centroid of its 64 particles; then
@@ -2093,7 +2128,7 @@ static uint32_t walk_lanes(const pnb_ctx* c, size_t n) {
 // passes count in the walk's time and in the step/accepted counters.
 static int walk(pnb_ctx* c, const float4* pts, const uint32_t* perm, size_t n, float theta,
                 float softening, float4* out, const WalkRows* rows = nullptr, bool quad = false,
-                bool rel = false, bool dd = false) {
+                bool rel = false, bool dd = false, int list = 0) {
     BhState* s = c->bh;
     const float theta2 = theta * theta;  // (self.theta * self.theta), sequential.rs:491
     const float eps2 = softening * softening;
@@ -2201,6 +2236,14 @@ static int walk(pnb_ctx* c, const float4* pts, const uint32_t* perm, size_t n, f
         } else if (rows) {
             launch_walk<WALK_ROWS, false>(wide, grid, c->stream, nr, total, pts, perm, uint32_t(n),
                                           theta2, eps2, out, info, *rows, nullptr);
+        } else if (list && total > 0 && !wide) {
+            auto go = [&](auto k) {
+                k<<<div_up(n, size_t(list)), 64, 0, c->stream>>>(
+                    nr, s->kids.as<uint4>(), total, pts, perm, uint32_t(n), theta2, eps2, out, info,
+                    s->qh.as<QuadH>(), s->oh.as<OctH>(), dd ? 1 : 0);
+            };
+            if (quad) mlp_octupole(c) ? go(bh_list_kernel<WALK_OCT, 4>) : go(bh_list_kernel<WALK_QUAD, 4>);
+            else list == 4 ? go(bh_list_kernel<WALK_PLAIN, 4>) : go(bh_list_kernel<WALK_PLAIN, 16>);
         } else {
             const uint32_t lanes = walk_lanes(c, n);
             const unsigned pgrid = unsigned(div_up(div_up(n, size_t(lanes)) * 64, size_t(256)));
@@ -2259,13 +2302,14 @@ static int accel_dev(pnb_ctx* c, const float4* affected, size_t n, const float4*
         return fail(c, PNB_E_STATE, "PNB_BH_MLP needs an initialised MLP (pnb_mlp_init)");
     if (!c->bh) c->bh = new BhState();
     bool dd = false;
+    const int list = rel ? 0 : list_lanes(n, mlp);
     if (c->bh->dd_mode) {
         if (ref_com || rel)
             return fail(c, PNB_E_ARG, "capturable Barnes-Hut takes neither PNB_BH_REF_COM nor "
                                       "PNB_BH_RELATIVE");
         BhState* s = c->bh;
         const bool sized = s->dd_cap > 0 && s->dd_m == m && s->dd_mlp == mlp &&
-                           ((affected == afg && n == m) || s->dd_n == n);
+                           (s->dd_kids || !list) && ((affected == afg && n == m) || s->dd_n == n);
         if (sized) {
             dd = true;
         } else if (stream_capturing(c)) {
@@ -2283,17 +2327,17 @@ static int accel_dev(pnb_ctx* c, const float4* affected, size_t n, const float4*
         ~Restore() { c->capturing = v; }
     } restore{c, was_capturing};
     if (dd) {
-        if (int rc = build_tree_dd(c, afg, m, mlp)) return rc;
+        if (int rc = build_tree_dd(c, afg, m, mlp, list != 0)) return rc;
     } else {
-        if (int rc = build_tree(c, afg, m, ref_com, mlp)) return rc;
+        if (int rc = build_tree(c, afg, m, ref_com, mlp, list != 0)) return rc;
         if (c->bh->dd_mode) {
             // The sizing call of a capturable build: capacities from this tree, then the tree
             // again in the sized buffers (growing a buffer discards its contents, so the tree
             // just built may be gone), built the capturable way.
-            if (int rc = dd_size(c, m, mlp)) return rc;
+            if (int rc = dd_size(c, m, mlp, list != 0)) return rc;
             c->bh->dd_n = n;
             dd = true;
-            if (int rc = build_tree_dd(c, afg, m, mlp)) return rc;
+            if (int rc = build_tree_dd(c, afg, m, mlp, list != 0)) return rc;
         }
     }
     BhState* s = c->bh;
@@ -2302,7 +2346,7 @@ static int accel_dev(pnb_ctx* c, const float4* affected, size_t n, const float4*
         if (int rc = node_network(c)) return rc;
     if (affected == afg && n == m)
         return walk(c, s->sp.as<float4>(), s->sidx, n, theta, softening, out, nullptr, quad, rel,
-                    dd);
+                    dd, list);
     const unsigned g = div_up(n, 256);
     PNB_HIP(c, s->akeys.ensure(n * 8));
     PNB_HIP(c, s->akeys_alt.ensure(n * 8));
@@ -2328,7 +2372,7 @@ static int accel_dev(pnb_ctx* c, const float4* affected, size_t n, const float4*
         return rc;
     bh_gather_kernel<<<g, 256, 0, c->stream>>>(affected, n, si, s->apts.as<float4>());
     PNB_CHECK_LAUNCH(c);
-    return walk(c, s->apts.as<float4>(), si, n, theta, softening, out, nullptr, quad, rel, dd);
+    return walk(c, s->apts.as<float4>(), si, n, theta, softening, out, nullptr, quad, rel, dd, list);
 }
 
 static int copy_h2d(pnb_ctx* c, DevBuf& b, const float* src, size_t count) {
