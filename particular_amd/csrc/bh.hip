@@ -51,7 +51,8 @@ namespace pnb {
 int radix_sort_pairs(pnb_ctx* c, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
                      uint32_t* vals_alt, size_t n, int key_bits, DevBuf& hist_buf,
                      DevBuf& bits_buf, uint64_t** keys_out, uint32_t** vals_out,
-                     bool all_digits = false, int low_bit = 0);
+                     bool all_digits = false, int low_bit = 0,
+                     const float4* src = nullptr, float4* dst = nullptr);
 int split_affecting(pnb_ctx* c, const float4* particles, size_t n, float4* dst, uint32_t* m_host);
 
 constexpr int KEY_LEVELS = 21;
@@ -159,6 +160,7 @@ struct BhState {
     DevBuf c_starts, c_pts, c_bh, c_bf, c_list, c_count, c_target, c_wgt, c_rows, c_rwave,
         c_cfeats, c_cgeom, c_cmask, c_lanes;
     DevBuf feat_out;  // pnb_bh_node_features
+    BhInfo* host_info = nullptr;  // pinned: the ordinary build's read-back
     float last_theta = 0.f;
     unsigned long long last_steps = 0, last_accepted = 0;
 };
@@ -175,6 +177,7 @@ void bh_free(BhState* s) {
                       &s->c_count, &s->c_target, &s->c_wgt, &s->c_rows, &s->c_rwave, &s->c_cfeats,
                       &s->c_cgeom, &s->c_cmask, &s->c_lanes, &s->feat_out})
         b->release();
+    if (s->host_info) hipHostFree(s->host_info);
     delete s;
 }
 
@@ -259,6 +262,20 @@ __global__ __launch_bounds__(256) void bh_bbox_kernel(const float4* __restrict__
 
 // square_with (partition.rs:136-153): centre = (min+max)/2, half = max(0, sizes...)/2,
 // box = centre -+ half, all in f32.
+__device__ __forceinline__ void write_root_box(const float (&mn)[3], const float (&mx)[3],
+                                               BhInfo* __restrict__ info) {
+    float centre[3], big = 0.0f;
+    for (int a = 0; a < 3; ++a) {
+        centre[a] = midpoint(mn[a], mx[a]);
+        big = fmaxf(big, sub_rn(mx[a], mn[a]));
+    }
+    const float half = midpoint(big, 0.0f);
+    for (int a = 0; a < 3; ++a) {
+        info->mn[a] = sub_rn(centre[a], half);
+        info->mx[a] = add_rn(centre[a], half);
+    }
+}
+
 // One wavefront: the partial boxes strided over the lanes, then a lane reduction (min and max
 // are exact, so the order does not matter).
 __global__ void bh_root_kernel(const float* __restrict__ part, int blocks, BhInfo* __restrict__ info) {
@@ -273,17 +290,7 @@ __global__ void bh_root_kernel(const float* __restrict__ part, int blocks, BhInf
             mn[a] = fminf(mn[a], __shfl_xor(mn[a], off, 64));
             mx[a] = fmaxf(mx[a], __shfl_xor(mx[a], off, 64));
         }
-    if (threadIdx.x != 0) return;
-    float centre[3], big = 0.0f;
-    for (int a = 0; a < 3; ++a) {
-        centre[a] = midpoint(mn[a], mx[a]);
-        big = fmaxf(big, sub_rn(mx[a], mn[a]));
-    }
-    const float half = midpoint(big, 0.0f);
-    for (int a = 0; a < 3; ++a) {
-        info->mn[a] = sub_rn(centre[a], half);
-        info->mx[a] = add_rn(centre[a], half);
-    }
+    if (threadIdx.x == 0) write_root_box(mn, mx, info);
 }
 
 __global__ void bh_info_init_kernel(BhInfo* info, uint32_t* __restrict__ lvl) {
@@ -299,6 +306,73 @@ __global__ void bh_info_init_kernel(BhInfo* info, uint32_t* __restrict__ lvl) {
     for (int l = threadIdx.x; l < MAX_LEVEL + 2; l += blockDim.x) info->lvl_count[l] = 0;
 }
 
+// The three steps above for small sets in one workgroup: there each launch is all latency (4.5 us).
+constexpr size_t BOX_SMALL = 16384;
+
+__global__ __launch_bounds__(1024) void bh_small_box_kernel(const float4* __restrict__ p, uint32_t m,
+                                                            BhInfo* __restrict__ info,
+                                                            uint32_t* __restrict__ lvl) {
+    __shared__ float red[16][6];
+    __shared__ uint32_t flags;
+    for (int l = threadIdx.x; l < 2 * LVL_SLOTS; l += blockDim.x) lvl[l * LVL_STRIDE] = 0;
+    for (int l = threadIdx.x; l < MAX_LEVEL + 2; l += blockDim.x) info->lvl_count[l] = 0;
+    if (threadIdx.x == 0) flags = 0;
+    float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
+    bool bad = false;
+    for (uint32_t i = threadIdx.x; i < m; i += blockDim.x) {
+        const float4 q = p[i];
+        bad |= !(isfinite(q.x) && isfinite(q.y) && isfinite(q.z));
+        mn[0] = fminf(mn[0], q.x); mx[0] = fmaxf(mx[0], q.x);
+        mn[1] = fminf(mn[1], q.y); mx[1] = fmaxf(mx[1], q.y);
+        mn[2] = fminf(mn[2], q.z); mx[2] = fmaxf(mx[2], q.z);
+    }
+    for (int off = 32; off > 0; off >>= 1)
+        for (int a = 0; a < 3; ++a) {
+            mn[a] = fminf(mn[a], __shfl_xor(mn[a], off, 64));
+            mx[a] = fmaxf(mx[a], __shfl_xor(mx[a], off, 64));
+        }
+    if ((threadIdx.x & 63) == 0)
+        for (int a = 0; a < 3; ++a) {
+            red[threadIdx.x >> 6][a] = mn[a];
+            red[threadIdx.x >> 6][3 + a] = mx[a];
+        }
+    __syncthreads();
+    if (bad) atomicOr(&flags, FLAG_NONFINITE);
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int w = 0; w < 16; ++w)
+        for (int a = 0; a < 3; ++a) {
+            mn[a] = fminf(mn[a], red[w][a]);
+            mx[a] = fmaxf(mx[a], red[w][3 + a]);
+        }
+    info->flags = flags;
+    info->max_level = -1;
+    info->total = 0;
+    info->max_rows = 0;
+    info->steps = 0;
+    info->accepted = 0;
+    write_root_box(mn, mx, info);
+}
+
+// Info cleared and the root box of the bodies.
+static int root_box(pnb_ctx* c, BhState* s, const float4* afg, size_t m) {
+    BhInfo* info = s->info.as<BhInfo>();
+    uint32_t* lvl = s->lvl.as<uint32_t>();
+    if (m <= BOX_SMALL) {
+        bh_small_box_kernel<<<1, 1024, 0, c->stream>>>(afg, uint32_t(m), info, lvl);
+        PNB_CHECK_LAUNCH(c);
+        return PNB_OK;
+    }
+    bh_info_init_kernel<<<1, 256, 0, c->stream>>>(info, lvl);
+    PNB_CHECK_LAUNCH(c);
+    const int bb = int(std::min<size_t>(BB_BLOCKS, div_up(m, 256)));
+    bh_bbox_kernel<<<bb, 256, 0, c->stream>>>(afg, m, s->bbox_part.as<float>(), info);
+    PNB_CHECK_LAUNCH(c);
+    bh_root_kernel<<<1, 64, 0, c->stream>>>(s->bbox_part.as<float>(), bb, info);
+    PNB_CHECK_LAUNCH(c);
+    return PNB_OK;
+}
+
 // ---- 2. keys ------------------------------------------------------------------------------------
 
 __global__ __launch_bounds__(256) void bh_keys_kernel(const float4* __restrict__ p, size_t m,
@@ -312,13 +386,6 @@ __global__ __launch_bounds__(256) void bh_keys_kernel(const float4* __restrict__
     float mx[3] = {info->mx[0], info->mx[1], info->mx[2]};
     keys[i] = descend_key(q.x, q.y, q.z, mn, mx, KEY_LEVELS);
     idx[i] = uint32_t(i);
-}
-
-__global__ __launch_bounds__(256) void bh_gather_kernel(const float4* __restrict__ src, size_t m,
-                                                        const uint32_t* __restrict__ idx,
-                                                        float4* __restrict__ dst) {
-    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < m) dst[i] = src[idx[i]];
 }
 
 // ---- 3. common prefixes and deep runs -----------------------------------------------------------
@@ -503,26 +570,39 @@ __global__ __launch_bounds__(256) void bh_count_kernel(const int* __restrict__ l
         if (hist[l]) atomicAdd(&lvl_count[l * LVL_STRIDE], hist[l]);
 }
 
-// Copies the per-level counts into info (for the host) and sets the list cursors to their
-// exclusive scan.
+// Copies the per-level counts and the node count (S[m], the scan's total) into info and sets the
+// list cursors to the counts' exclusive scan. cap > 0 (a capturable build): a tree that needs more
+// nodes or levels than an earlier ordinary build sized flags the build; every later kernel of it
+// then returns at once and the walk writes NaN.
 __global__ __launch_bounds__(256) void bh_level_offsets_kernel(BhInfo* __restrict__ info,
                                                                const uint32_t* __restrict__ lvl_count,
-                                                               uint32_t* __restrict__ lvl_cur) {
-    __shared__ uint32_t v[LVL_SLOTS];
-    for (int l = threadIdx.x; l < LVL_SLOTS; l += blockDim.x) v[l] = lvl_count[l * LVL_STRIDE];
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t acc = 0;
-        for (int l = 0; l < LVL_SLOTS; ++l) {
-            const uint32_t n_l = v[l];
-            v[l] = acc;
-            info->lvl_count[l] = n_l;
-            info->lvl_off[l] = acc;
-            acc += n_l;
-        }
+                                                               uint32_t* __restrict__ lvl_cur,
+                                                               const uint32_t* __restrict__ S,
+                                                               size_t m, uint32_t cap, int levels) {
+    static_assert(LVL_SLOTS <= 256, "one thread per level");
+    __shared__ uint32_t wsum[4];
+    const int l = threadIdx.x, lane = l & 63, w = l >> 6;
+    const uint32_t n_l = l < LVL_SLOTS ? lvl_count[l * LVL_STRIDE] : 0u;
+    uint32_t incl = n_l;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += y;
     }
+    if (lane == 63) wsum[w] = incl;
     __syncthreads();
-    for (int l = threadIdx.x; l < LVL_SLOTS; l += blockDim.x) lvl_cur[l * LVL_STRIDE] = v[l];
+    uint32_t off = incl - n_l;
+    for (int q = 0; q < w; ++q) off += wsum[q];
+    if (l < LVL_SLOTS) {
+        info->lvl_count[l] = n_l;
+        info->lvl_off[l] = off;
+        lvl_cur[l * LVL_STRIDE] = off;
+    }
+    if (l == 0) {
+        const uint32_t total = S[m];
+        info->total = total;
+        if (cap && (total > cap || info->max_level > levels)) atomicOr(&info->flags, FLAG_CAPACITY);
+    }
 }
 
 // ilist: the internal nodes of each level together (level l from the exclusive scan of the
@@ -885,15 +965,6 @@ __global__ __launch_bounds__(1024) void bh_up_run_kernel(NodeRec* __restrict__ r
 }
 
 // ---- capturable builds: node count and status stay on the device ----------------------------
-// The scan's total against the capacities sized by an earlier ordinary build; a tree that does
-// not fit flags the build (every later kernel of it then returns at once and the walk writes NaN).
-__global__ void bh_dd_check_kernel(const uint32_t* __restrict__ S, size_t m, uint32_t cap,
-                                   int levels, BhInfo* __restrict__ info) {
-    const uint32_t total = S[m];
-    info->total = total;
-    if (total > cap || info->max_level > levels) atomicOr(&info->flags, FLAG_CAPACITY);
-}
-
 // The bottom-up sums of one level, its count and place in the level-grouped list read from the
 // device (the host launches every level up to the sized depth; levels the tree lacks are empty).
 // With `mom` (the learned correction), also the node moments, as in the ordinary build.
@@ -1659,9 +1730,9 @@ static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = fa
     PNB_HIP(c, s->lvl.ensure(size_t(2) * LVL_SLOTS * LVL_STRIDE * sizeof(uint32_t)));
     uint32_t* lvl_count = s->lvl.as<uint32_t>();
     uint32_t* lvl_cur = lvl_count + LVL_SLOTS * LVL_STRIDE;
-    bh_info_init_kernel<<<1, 256, 0, c->stream>>>(info, lvl_count);
-    PNB_CHECK_LAUNCH(c);
     if (m == 0) {
+        bh_info_init_kernel<<<1, 256, 0, c->stream>>>(info, lvl_count);
+        PNB_CHECK_LAUNCH(c);
         s->built = true;
         return PNB_OK;
     }
@@ -1679,11 +1750,7 @@ static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = fa
     PNB_HIP(c, s->key2.ensure(m * 8));
 
     return timed(c, PNB_PROF_BH_BUILD, [&]() -> int {
-        const int bb = int(std::min<size_t>(BB_BLOCKS, div_up(m, 256)));
-        bh_bbox_kernel<<<bb, 256, 0, c->stream>>>(afg, m, s->bbox_part.as<float>(), info);
-        PNB_CHECK_LAUNCH(c);
-        bh_root_kernel<<<1, 64, 0, c->stream>>>(s->bbox_part.as<float>(), bb, info);
-        PNB_CHECK_LAUNCH(c);
+        if (int rc = root_box(c, s, afg, m)) return rc;
         bh_keys_kernel<<<g, 256, 0, c->stream>>>(afg, m, info, s->keys.as<uint64_t>(), s->idx.as<uint32_t>());
         PNB_CHECK_LAUNCH(c);
         uint64_t* sk;
@@ -1691,13 +1758,11 @@ static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = fa
         int rc = timed(c, PNB_PROF_SORT, [&]() -> int {
             return radix_sort_pairs(c, s->keys.as<uint64_t>(), s->idx.as<uint32_t>(),
                                     s->keys_alt.as<uint64_t>(), s->idx_alt.as<uint32_t>(), m, 63,
-                                    s->hist, s->bits, &sk, &si);
+                                    s->hist, s->bits, &sk, &si, false, 0, afg, s->sp.as<float4>());
         });
         if (rc) return rc;
         s->skeys = sk;
         s->sidx = si;
-        bh_gather_kernel<<<g, 256, 0, c->stream>>>(afg, m, si, s->sp.as<float4>());
-        PNB_CHECK_LAUNCH(c);
         int* lcp = s->lcp.as<int>();
         bh_lcp_kernel<<<g, 256, 0, c->stream>>>(sk, s->sp.as<float4>(), m, lcp);
         PNB_CHECK_LAUNCH(c);
@@ -1708,14 +1773,14 @@ static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = fa
         const unsigned lg = std::min<unsigned>(g, 4 * std::max(c->cu_count, 1));
         bh_count_kernel<<<lg, 256, 0, c->stream>>>(lcp, m, cnt, s->ip.as<int>(), info, lvl_count);
         PNB_CHECK_LAUNCH(c);
-        bh_level_offsets_kernel<<<1, 256, 0, c->stream>>>(info, lvl_count, lvl_cur);
-        PNB_CHECK_LAUNCH(c);
         if ((rc = scan_u32(c, cnt, cnt, m, true))) return rc;
-        BhInfo h;
-        PNB_HIP(c, hipMemcpyAsync(&h, info, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-        uint32_t total = 0;
-        PNB_HIP(c, hipMemcpyAsync(&total, cnt + m, 4, hipMemcpyDeviceToHost, c->stream));
+        bh_level_offsets_kernel<<<1, 256, 0, c->stream>>>(info, lvl_count, lvl_cur, cnt, m, 0, 0);
+        PNB_CHECK_LAUNCH(c);
+        if (!s->host_info) PNB_HIP(c, hipHostMalloc(reinterpret_cast<void**>(&s->host_info), sizeof(BhInfo)));
+        PNB_HIP(c, hipMemcpyAsync(s->host_info, info, sizeof(BhInfo), hipMemcpyDeviceToHost, c->stream));
         PNB_HIP(c, hipStreamSynchronize(c->stream));
+        const BhInfo& h = *s->host_info;
+        const uint32_t total = h.total;
         if (h.flags & FLAG_NONFINITE) return fail(c, PNB_E_ARG, "non-finite affecting position");
         if (h.flags & FLAG_DEPTH)
             return fail(c, PNB_E_DEPTH, "octree deeper than %d levels", MAX_LEVEL);
@@ -1864,23 +1929,19 @@ static int build_tree_dd(pnb_ctx* c, const float4* afg, size_t m, bool moments, 
     BhInfo* info = s->info.as<BhInfo>();
     uint32_t* lvl_count = s->lvl.as<uint32_t>();
     uint32_t* lvl_cur = lvl_count + LVL_SLOTS * LVL_STRIDE;
-    bh_info_init_kernel<<<1, 256, 0, c->stream>>>(info, lvl_count);
-    PNB_CHECK_LAUNCH(c);
     s->nodes = s->dd_cap;  // an upper bound; the count itself is info->total
     s->max_level = s->dd_levels;
     s->internal = 0;
     s->dd_last = true;
     if (m == 0) {
+        bh_info_init_kernel<<<1, 256, 0, c->stream>>>(info, lvl_count);
+        PNB_CHECK_LAUNCH(c);
         s->built = true;
         return PNB_OK;
     }
     const unsigned g = div_up(m, 256);
     return timed(c, PNB_PROF_BH_BUILD, [&]() -> int {
-        const int bb = int(std::min<size_t>(BB_BLOCKS, div_up(m, 256)));
-        bh_bbox_kernel<<<bb, 256, 0, c->stream>>>(afg, m, s->bbox_part.as<float>(), info);
-        PNB_CHECK_LAUNCH(c);
-        bh_root_kernel<<<1, 64, 0, c->stream>>>(s->bbox_part.as<float>(), bb, info);
-        PNB_CHECK_LAUNCH(c);
+        if (int rc = root_box(c, s, afg, m)) return rc;
         bh_keys_kernel<<<g, 256, 0, c->stream>>>(afg, m, info, s->keys.as<uint64_t>(), s->idx.as<uint32_t>());
         PNB_CHECK_LAUNCH(c);
         uint64_t* sk;
@@ -1888,14 +1949,12 @@ static int build_tree_dd(pnb_ctx* c, const float4* afg, size_t m, bool moments, 
         int rc = timed(c, PNB_PROF_SORT, [&]() -> int {
             return radix_sort_pairs(c, s->keys.as<uint64_t>(), s->idx.as<uint32_t>(),
                                     s->keys_alt.as<uint64_t>(), s->idx_alt.as<uint32_t>(), m, 63,
-                                    s->hist, s->bits, &sk, &si, true);
+                                    s->hist, s->bits, &sk, &si, true, 0, afg, s->sp.as<float4>());
         });
         if (rc) return rc;
         s->skeys = sk;
         s->sidx = si;
         float4* sp = s->sp.as<float4>();
-        bh_gather_kernel<<<g, 256, 0, c->stream>>>(afg, m, si, sp);
-        PNB_CHECK_LAUNCH(c);
         int* lcp = s->lcp.as<int>();
         bh_lcp_kernel<<<g, 256, 0, c->stream>>>(sk, sp, m, lcp);
         PNB_CHECK_LAUNCH(c);
@@ -1905,10 +1964,9 @@ static int build_tree_dd(pnb_ctx* c, const float4* afg, size_t m, bool moments, 
         const unsigned lg = std::min<unsigned>(g, 4 * std::max(c->cu_count, 1));
         bh_count_kernel<<<lg, 256, 0, c->stream>>>(lcp, m, cnt, s->ip.as<int>(), info, lvl_count);
         PNB_CHECK_LAUNCH(c);
-        bh_level_offsets_kernel<<<1, 256, 0, c->stream>>>(info, lvl_count, lvl_cur);
-        PNB_CHECK_LAUNCH(c);
         if ((rc = scan_u32(c, cnt, cnt, m, true))) return rc;
-        bh_dd_check_kernel<<<1, 1, 0, c->stream>>>(cnt, m, uint32_t(s->dd_cap), s->dd_levels, info);
+        bh_level_offsets_kernel<<<1, 256, 0, c->stream>>>(info, lvl_count, lvl_cur, cnt, m,
+                                                          uint32_t(s->dd_cap), s->dd_levels);
         PNB_CHECK_LAUNCH(c);
         NodeRec* rec = s->rec.as<NodeRec>();
         uint32_t* skipv = s->skipv.as<uint32_t>();
@@ -2368,10 +2426,9 @@ static int accel_dev(pnb_ctx* c, const float4* affected, size_t n, const float4*
     constexpr int AFFECTED_LOW_BIT = 23;
     if (int rc = radix_sort_pairs(c, s->akeys.as<uint64_t>(), s->aidx.as<uint32_t>(),
                                   s->akeys_alt.as<uint64_t>(), s->aidx_alt.as<uint32_t>(), n, 63,
-                                  s->hist, s->bits, &sk, &si, dd, AFFECTED_LOW_BIT))
+                                  s->hist, s->bits, &sk, &si, dd, AFFECTED_LOW_BIT, affected,
+                                  s->apts.as<float4>()))
         return rc;
-    bh_gather_kernel<<<g, 256, 0, c->stream>>>(affected, n, si, s->apts.as<float4>());
-    PNB_CHECK_LAUNCH(c);
     return walk(c, s->apts.as<float4>(), si, n, theta, softening, out, nullptr, quad, rel, dd, list);
 }
 

@@ -135,6 +135,34 @@ __global__ __launch_bounds__(SCAN_BLOCK) void scan_apply_kernel(const uint32_t* 
     if (with_total && blockIdx.x == gridDim.x - 1 && threadIdx.x == SCAN_BLOCK - 1) out[n] = run;
 }
 
+// Small inputs in one launch: a workgroup of 16 wavefronts, 16 consecutive values per thread.
+constexpr size_t SCAN_SMALL = 16384;
+
+__global__ __launch_bounds__(1024) void scan_small_kernel(const uint32_t* in, uint32_t n, uint32_t* out,
+                                                          int with_total) {
+    __shared__ uint32_t wsum[16];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const uint32_t per = (n + 1023) / 1024, b = min(n, threadIdx.x * per), e = min(n, b + per);
+    uint32_t s = 0;
+    for (uint32_t i = b; i < e; ++i) s += in[i];
+    uint32_t x = s;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+    }
+    if (lane == 63) wsum[wid] = x;
+    __syncthreads();
+    uint32_t run = x - s;
+    for (int w = 0; w < wid; ++w) run += wsum[w];
+    for (uint32_t i = b; i < e; ++i) {
+        const uint32_t v = in[i];
+        out[i] = run;
+        run += v;
+    }
+    if (with_total && threadIdx.x == 1023) out[n] = run;
+}
+
 static int scan_rec(pnb_ctx* c, const uint32_t* in, uint32_t* out, size_t n, bool with_total,
                     uint32_t* tmp, size_t tmp_cap) {
     unsigned blocks = div_up(n, SCAN_TILE);
@@ -162,6 +190,11 @@ int scan_u32(pnb_ctx* c, const uint32_t* in, uint32_t* out, size_t n, bool with_
             zero_u32_kernel<<<1, 1, 0, c->stream>>>(out);
             PNB_CHECK_LAUNCH(c);
         }
+        return PNB_OK;
+    }
+    if (n > SCAN_TILE && n <= SCAN_SMALL) {
+        scan_small_kernel<<<1, 1024, 0, c->stream>>>(in, uint32_t(n), out, with_total ? 1 : 0);
+        PNB_CHECK_LAUNCH(c);
         return PNB_OK;
     }
     size_t need = 0, level = n;

@@ -128,7 +128,8 @@ __global__ __launch_bounds__(256) void ms_hist_kernel(const uint64_t* __restrict
 __global__ __launch_bounds__(MS_BLOCK) void ms_pass_kernel(
     const uint64_t* __restrict__ keys, const uint32_t* __restrict__ vals, size_t n, int shift,
     const uint32_t* __restrict__ hist, uint32_t* __restrict__ next, uint32_t tiles,
-    uint64_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out) {
+    uint64_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out,
+    const float4* __restrict__ src, float4* __restrict__ dst) {
     __shared__ uint32_t wcnt[MS_WAVES][256];
     __shared__ uint32_t sum[2][2][256];  // per half of the tiles: all of them, those before this one
     __shared__ uint32_t wsum[4];
@@ -203,6 +204,7 @@ __global__ __launch_bounds__(MS_BLOCK) void ms_pass_kernel(
         const uint32_t pos = wcnt[w][uint32_t(key[r] >> shift) & 0xffu] + rank[r];
         keys_out[pos] = key[r];
         vals_out[pos] = val[r];
+        if (dst) dst[pos] = src[val[r]];
         if (next)
             atomicAdd(&next[size_t(pos / MS_TILE) * 256 + (uint32_t(key[r] >> (shift + 8)) & 0xffu)], 1u);
     }
@@ -246,9 +248,10 @@ __global__ void rs_bits_init_kernel(unsigned long long* or_and) {
 // before it in the input, which is exactly the stable order of the radix path. One thread per
 // key; a wavefront reads the keys it counts against 64 at a time (one per lane, coalesced) and
 // broadcasts them lane by lane with v_readlane into scalar registers, so each compare is a
-// vector-scalar compare with no memory access. A workgroup counts against at most RANK_SPAN keys:
-// inputs above it split the count over blockIdx.y and add the parts with atomics before a
-// scatter launch.
+// vector-scalar compare with no memory access. A workgroup counts against at most RANK_SPAN keys (a
+// quarter of that from 1,025 to 8,192 keys, where there are few workgroups and each is bound by its
+// wavefronts' issue rate: 4,096 keys 17 -> 6 us): inputs above it split the count over blockIdx.y
+// and add the parts with atomics before a scatter launch.
 constexpr uint32_t SMALL_SORT = 16384;
 constexpr uint32_t RANK_SPAN = 1024;
 
@@ -262,15 +265,17 @@ __device__ __forceinline__ uint64_t lane_key(uint64_t v, int k) {
 // ki + 1 and the others below ki; positions past the span read as ~0, which counts for neither.
 __global__ __launch_bounds__(256) void rank_count_kernel(const uint64_t* __restrict__ keys,
                                                          const uint32_t* __restrict__ vals,
-                                                         uint32_t n, uint64_t mask,
+                                                         uint32_t n, uint32_t span, uint64_t mask,
                                                          uint32_t* __restrict__ rank,
                                                          uint64_t* __restrict__ keys_out,
-                                                         uint32_t* __restrict__ vals_out) {
+                                                         uint32_t* __restrict__ vals_out,
+                                                         const float4* __restrict__ src,
+                                                         float4* __restrict__ dst) {
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t wbase = i - lane;  // the wavefront's first position
     const uint64_t ki = i < n ? (keys[i] & mask) : 0ull;
-    const uint32_t j0 = blockIdx.y * RANK_SPAN, j1 = min(n, j0 + RANK_SPAN);
+    const uint32_t j0 = blockIdx.y * span, j1 = min(n, j0 + span);
     uint32_t cc[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // independent counts: no carry chain
     uint64_t next = j0 + lane < j1 ? (keys[j0 + lane] & mask) : ~0ull;
     for (uint32_t t0 = j0; t0 < j1; t0 += 64) {
@@ -301,6 +306,7 @@ __global__ __launch_bounds__(256) void rank_count_kernel(const uint64_t* __restr
     }
     keys_out[c] = keys[i];
     vals_out[c] = vals[i];
+    if (dst) dst[c] = src[vals[i]];
 }
 
 __global__ __launch_bounds__(256) void rank_zero_kernel(uint32_t* __restrict__ rank, uint32_t n) {
@@ -313,29 +319,47 @@ __global__ __launch_bounds__(256) void rank_scatter_kernel(const uint64_t* __res
                                                            uint32_t n,
                                                            const uint32_t* __restrict__ rank,
                                                            uint64_t* __restrict__ keys_out,
-                                                           uint32_t* __restrict__ vals_out) {
+                                                           uint32_t* __restrict__ vals_out,
+                                                           const float4* __restrict__ src,
+                                                           float4* __restrict__ dst) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     keys_out[rank[i]] = keys[i];
     vals_out[rank[i]] = vals[i];
+    if (dst) dst[rank[i]] = src[vals[i]];
+}
+
+__global__ __launch_bounds__(256) void rs_gather_kernel(const float4* __restrict__ src, size_t n,
+                                                        const uint32_t* __restrict__ vals,
+                                                        float4* __restrict__ dst) {
+    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < n) dst[i] = src[vals[i]];
 }
 
 // Sorts keys[0..n) with their values, stably; the result ends in (*keys_out, *vals_out), which is
 // either the input pair or the alternate pair. Only bits [0, key_bits) are considered, and above
-// SMALL_SORT pairs only bits from low_bit on (a caller that wants neighbours together, not an order). Up to
+// SMALL_SORT pairs only bits from low_bit on (a caller that wants neighbours together, not an order).
+// dst (optional): dst[i] = src[i-th value], written by the sort's last launch below MID_SORT pairs. Up to
 // SMALL_SORT pairs (keys of at most 63 bits) are ranked by counting, into the alternate pair;
 // either way equal keys keep their input order.
 // Digits no two keys differ in are skipped after one read-back to the host, unless all_digits.
 int radix_sort_pairs(pnb_ctx* c, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
                      uint32_t* vals_alt, size_t n, int key_bits, DevBuf& hist_buf,
                      DevBuf& bits_buf, uint64_t** keys_out, uint32_t** vals_out,
-                     bool all_digits, int low_bit) {
+                     bool all_digits, int low_bit, const float4* src, float4* dst) {
     *keys_out = keys;
     *vals_out = vals;
-    if (n <= 1) return PNB_OK;
+    auto gather = [&](const uint32_t* v) -> int {
+        if (!dst || n == 0) return PNB_OK;
+        rs_gather_kernel<<<div_up(n, 256), 256, 0, c->stream>>>(src, n, v, dst);
+        PNB_CHECK_LAUNCH(c);
+        return PNB_OK;
+    };
+    if (n <= 1) return gather(vals);
     if (n <= SMALL_SORT && key_bits <= 63) {
         const uint64_t mask = key_bits >= 64 ? ~0ull : ((1ull << key_bits) - 1);
-        const uint32_t nn = uint32_t(n), g = div_up(nn, 256u), parts = div_up(nn, RANK_SPAN);
+        const uint32_t nn = uint32_t(n), span = n > RANK_SPAN && n <= 8192 ? RANK_SPAN / 4 : RANK_SPAN;
+        const uint32_t g = div_up(nn, 256u), parts = div_up(nn, span);
         uint32_t* rank = nullptr;
         if (parts > 1) {
             PNB_HIP(c, hist_buf.ensure(size_t(nn) * sizeof(uint32_t)));
@@ -343,11 +367,11 @@ int radix_sort_pairs(pnb_ctx* c, uint64_t* keys, uint32_t* vals, uint64_t* keys_
             rank_zero_kernel<<<g, 256, 0, c->stream>>>(rank, nn);
             PNB_CHECK_LAUNCH(c);
         }
-        rank_count_kernel<<<dim3(g, parts), 256, 0, c->stream>>>(keys, vals, nn, mask, rank,
-                                                                keys_alt, vals_alt);
+        rank_count_kernel<<<dim3(g, parts), 256, 0, c->stream>>>(keys, vals, nn, span, mask, rank,
+                                                                keys_alt, vals_alt, src, dst);
         PNB_CHECK_LAUNCH(c);
         if (parts > 1) {
-            rank_scatter_kernel<<<g, 256, 0, c->stream>>>(keys, vals, nn, rank, keys_alt, vals_alt);
+            rank_scatter_kernel<<<g, 256, 0, c->stream>>>(keys, vals, nn, rank, keys_alt, vals_alt, src, dst);
             PNB_CHECK_LAUNCH(c);
         }
         *keys_out = keys_alt;
@@ -366,7 +390,7 @@ int radix_sort_pairs(pnb_ctx* c, uint64_t* keys, uint32_t* vals, uint64_t* keys_
             uint32_t* h = hist + size_t(k) * tiles * 256;
             ms_pass_kernel<<<tiles, MS_BLOCK, 0, c->stream>>>(
                 keys, vals, n, low_bit + 8 * k, h, k + 1 < digits ? h + size_t(tiles) * 256 : nullptr,
-                tiles, keys_alt, vals_alt);
+                tiles, keys_alt, vals_alt, src, k + 1 < digits ? nullptr : dst);
             PNB_CHECK_LAUNCH(c);
             std::swap(keys, keys_alt);
             std::swap(vals, vals_alt);
@@ -408,7 +432,7 @@ int radix_sort_pairs(pnb_ctx* c, uint64_t* keys, uint32_t* vals, uint64_t* keys_
     }
     *keys_out = kin;
     *vals_out = vin;
-    return PNB_OK;
+    return gather(vin);
 }
 
 }  // namespace pnb
