@@ -14,8 +14,8 @@
 //   mlp_rowgrad_kernel per row: g_y = sum over its lanes of the scaled (d field / d y)^T g_pred
 //                     (quad_field_grad, oct_field_grad)
 //   mlp_bwd_kernel    recomputes the forward per 16-row tile and back-propagates with MFMA;
-//                     weight gradients accumulate in registers, one partial per wavefront
-//   mlp_reduce_kernel fixed-order sum of the partials (deterministic)
+//                     weight gradients accumulate in registers, one partial per workgroup
+//   mlp_reduce_kernel fixed-order sum of the partials (deterministic), and of the loss
 //   mlp_adam_kernel   Adam on the FP32 master weights, then mlp_pack_kernel
 // The loss and its gradients are those of oracle/mlp_oracle.py with the same BF16 rounding points.
 #include "pnb_internal.hpp"
@@ -163,7 +163,10 @@ __global__ __launch_bounds__(256) void mlp_fwd_kernel(const float* __restrict__ 
 // All sums run in a fixed order, so the loss and the gradients do not depend on scheduling.
 constexpr uint32_t MLP_CHUNK = 128;
 
-__global__ __launch_bounds__(64) void mlp_pred_kernel(const float* __restrict__ y,
+// One wavefront per chunk adds the rows in order. Their outputs and geometry come to LDS first, in
+// coalesced loads, and are read from there as broadcasts: scalar loads row by row inside the mask's
+// branch left the wavefront waiting (256,000 rows of 128 wavefronts: 74 -> 50 us).
+__global__ __launch_bounds__(64) void mlp_pred_kernel(const float4* __restrict__ y,
                                                       const uint32_t* __restrict__ wave_rows,
                                                       const uint32_t* __restrict__ chunk_wave,
                                                       const uint32_t* __restrict__ chunk_rb,
@@ -171,25 +174,44 @@ __global__ __launch_bounds__(64) void mlp_pred_kernel(const float* __restrict__ 
                                                       const float4* __restrict__ geom,
                                                       const float4* __restrict__ lanes,
                                                       float4* __restrict__ part) {
+    static_assert(MLP_YS == 16 && MLP_GEOM == 8, "rows of four and two float4");
+    __shared__ float4 yl[MLP_CHUNK * 4], gl[MLP_CHUNK * 2];
     const uint32_t c = blockIdx.x;
     const int lane = threadIdx.x;
     const uint32_t w = chunk_wave[c], rb = chunk_rb[c];
     const uint32_t re = min(rb + MLP_CHUNK, wave_rows[w + 1]);
+    const uint32_t rows = re > rb ? re - rb : 0u;
+    unsigned long long mk[MLP_CHUNK / 64];
+#pragma unroll
+    for (uint32_t q = 0; q < MLP_CHUNK / 64; ++q)
+        mk[q] = 64 * q + lane < rows ? mask[rb + 64 * q + lane] : 0ull;
+#pragma unroll
+    for (uint32_t q = 0; q < MLP_CHUNK * 4 / 64; ++q)
+        if (64 * q + lane < 4 * rows) yl[64 * q + lane] = y[4 * size_t(rb) + 64 * q + lane];
+#pragma unroll
+    for (uint32_t q = 0; q < MLP_CHUNK * 2 / 64; ++q)
+        if (64 * q + lane < 2 * rows) gl[64 * q + lane] = geom[2 * size_t(rb) + 64 * q + lane];
+    wave_lds_sync();
     const float4 p = lanes[size_t(w) * 64 + lane];  // w = softening^2
     float px = 0.f, py = 0.f, pz = 0.f;
-    for (uint32_t r = rb; r < re; ++r) {
-        if ((mask[r] >> lane) & 1ull) {
-            const float4 gm = geom[2 * size_t(r)];
-            const float mw3 = geom[2 * size_t(r) + 1].x;
-            const float dx = gm.x - p.x, dy = gm.y - p.y, dz = gm.z - p.z;
-            const float inv = rsqrtf(dx * dx + dy * dy + dz * dz + p.w);
-            float q[6], o[7];
 #pragma unroll
-            for (int j = 0; j < 6; ++j) q[j] = y[size_t(r) * MLP_YS + j];
-#pragma unroll
-            for (int j = 0; j < 7; ++j) o[j] = y[size_t(r) * MLP_YS + MLP_QOUT + j];
-            quad_field(q, dx, dy, dz, inv, gm.w, px, py, pz);
-            oct_field(o, dx, dy, dz, inv, mw3, px, py, pz);
+    for (uint32_t q = 0; q < MLP_CHUNK / 64; ++q) {
+        const uint32_t mlo = uint32_t(mk[q]), mhi = uint32_t(mk[q] >> 32);
+        const uint32_t end = min(rows, 64 * q + 64);
+#pragma unroll 2
+        for (uint32_t r = 64 * q; r < end; ++r) {
+            const float4 y0 = yl[4 * r], y1 = yl[4 * r + 1], y2 = yl[4 * r + 2], gm = gl[2 * r];
+            const float y3 = yl[4 * r + 3].x, mw3 = gl[2 * r + 1].x;
+            const uint64_t m = uint64_t(uint32_t(__builtin_amdgcn_readlane(int(mlo), int(r & 63)))) |
+                               uint64_t(uint32_t(__builtin_amdgcn_readlane(int(mhi), int(r & 63)))) << 32;
+            if ((m >> lane) & 1ull) {
+                const float dx = gm.x - p.x, dy = gm.y - p.y, dz = gm.z - p.z;
+                const float inv = rsqrtf(fmaf(dz, dz, fmaf(dx, dx, dy * dy)) + p.w);
+                const float qd[6] = {y0.x, y0.y, y0.z, y0.w, y1.x, y1.y};
+                const float o[7] = {y1.z, y1.w, y2.x, y2.y, y2.z, y2.w, y3};
+                quad_field(qd, dx, dy, dz, inv, gm.w, px, py, pz);
+                oct_field(o, dx, dy, dz, inv, mw3, px, py, pz);
+            }
         }
     }
     part[size_t(c) * 64 + lane] = make_float4(px, py, pz, 0.f);
@@ -267,11 +289,26 @@ __global__ __launch_bounds__(256) void mlp_rowgrad_kernel(size_t rows,
 // from memory in both layouts), G_h1 in the grad layout (from G_z2 in the chain layout);
 // gradients: gW3 += H2^T g_y, gW2 += H1^T G_z2, gW1 += X^T G_z1, bias gradients summed from the
 // grad layouts (rows 4g..4g+3 per lane, then across the four row groups).
-__global__ __launch_bounds__(256) void mlp_bwd_kernel(const float* __restrict__ feats,
-                                                      const float* __restrict__ gyin, size_t rows,
-                                                      const MlpWeights* __restrict__ wg,
-                                                      float* __restrict__ partial) {
-    __shared__ MlpWeights w;
+//
+// Eight wavefronts per workgroup (two per SIMD: one alone waited on LDS and on each product's
+// result most of the time, 6,500 cycles a tile against 1,400 of MFMA), whose gradients are added in
+// LDS before one set per workgroup is written, an eighth of the bytes for mlp_reduce_kernel. The
+// weights' fragments are read from LDS for every tile (kept in registers, as one wavefront per SIMD
+// could, they leave no room for a second). 256,000 rows: 47 -> 38 us, and mlp_reduce_kernel 38 -> 6.
+constexpr int MLP_BWD_WAVES = 8;
+constexpr int MLP_BWD_SETS = 27;  // f32x4 of gradients per lane: 16 gw2, 4 gw1, 4 gw3, gb1, gb2, gb3
+constexpr int MLP_BWD_HALF = (MLP_BWD_SETS + 1) / 2;
+
+__global__ __launch_bounds__(64 * MLP_BWD_WAVES) void mlp_bwd_kernel(
+    const float* __restrict__ feats, const float* __restrict__ gyin, size_t rows,
+    const MlpWeights* __restrict__ wg, float* __restrict__ partial) {
+    union Lds {
+        MlpWeights w;
+        f32x4_t sums[MLP_BWD_WAVES / 2][MLP_BWD_HALF][64];
+        __device__ Lds() {}
+    };
+    __shared__ Lds lds;
+    MlpWeights& w = lds.w;
     load_weights(w, wg);
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r16 = lane & 15, g = lane >> 4;
@@ -285,10 +322,10 @@ __global__ __launch_bounds__(256) void mlp_bwd_kernel(const float* __restrict__ 
 #pragma unroll
         for (int b = 0; b < 4; ++b) gw2[a][b] = zero;
     }
-    const size_t gwave = size_t(blockIdx.x) * MLP_WAVES_PER_BLOCK + wv;
-    const size_t nw = size_t(gridDim.x) * MLP_WAVES_PER_BLOCK;
-    // A tile's inputs, read one tile ahead (one wavefront per SIMD here: the loads' latency is
-    // hidden behind the previous tile's products): x and g_y of row r, columns 4g..4g+3 (chain
+    const size_t gwave = size_t(blockIdx.x) * MLP_BWD_WAVES + wv;
+    const size_t nw = size_t(gridDim.x) * MLP_BWD_WAVES;
+    // A tile's inputs, read one tile ahead (the loads' latency is hidden behind the previous
+    // tile's products): x and g_y of row r, columns 4g..4g+3 (chain
     // layout / A fragment of the row-major matrix) and of rows 4g..4g+3, column r (grad layout).
     float4 nxv, ngv;
     float nxs[4], ngs[4];
@@ -318,6 +355,8 @@ __global__ __launch_bounds__(256) void mlp_bwd_kernel(const float* __restrict__ 
             gs[i] = ngs[i];
         }
         fetch(tile + nw);  // past the last tile: zeros, nothing read
+        // keeps the weights' fragments out of registers
+        asm volatile("" ::: "memory");
         bf16x4_t bx, gyc;
         {
             const float xa[4] = {xv.x, xv.y, xv.z, xv.w}, ga[4] = {gv.x, gv.y, gv.z, gv.w};
@@ -421,7 +460,35 @@ __global__ __launch_bounds__(256) void mlp_bwd_kernel(const float* __restrict__ 
             for (int nt = 0; nt < 4; ++nt) gw2[mt][nt] = mfma16(h1g[mt], g2g[nt], gw2[mt][nt]);
         }
     }
-    float* out = partial + gwave * MLP_NPARAM;
+    // the workgroup's sum: the upper half of the wavefronts to the lower, three times, half of the
+    // values at a time
+    f32x4_t bias[3];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        bias[0][i] = gb1[i];
+        bias[1][i] = gb2[i];
+        bias[2][i] = i == 0 ? gb3 : 0.f;
+    }
+    const auto value = [&](int v) -> f32x4_t& {
+        return v < 16 ? gw2[v >> 2][v & 3] : v < 20 ? gw1[v - 16] : v < 24 ? gw3[v - 20] : bias[v - 24];
+    };
+#pragma unroll
+    for (int half = MLP_BWD_WAVES / 2; half > 0; half >>= 1)
+#pragma unroll
+        for (int v0 = 0; v0 < MLP_BWD_SETS; v0 += MLP_BWD_HALF) {
+            __syncthreads();  // the weights, or the values before these, have been read
+            if (wv >= half && wv < 2 * half)
+#pragma unroll
+                for (int v = v0; v < min(v0 + MLP_BWD_HALF, MLP_BWD_SETS); ++v)
+                    lds.sums[wv - half][v - v0][lane] = value(v);
+            __syncthreads();
+            if (wv < half)
+#pragma unroll
+                for (int v = v0; v < min(v0 + MLP_BWD_HALF, MLP_BWD_SETS); ++v)
+                    value(v) += lds.sums[wv][v - v0][lane];
+        }
+    if (wv != 0) return;
+    float* out = partial + size_t(blockIdx.x) * MLP_NPARAM;
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
@@ -444,7 +511,7 @@ __global__ __launch_bounds__(256) void mlp_bwd_kernel(const float* __restrict__ 
     // bias gradients: each lane's sums over its rows 4g..4g+3, then over the four row groups
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
-        float a = gb1[nt], b = gb2[nt];
+        float a = bias[0][nt], b = bias[1][nt];
         a += __shfl_xor(a, 16, 64);
         a += __shfl_xor(a, 32, 64);
         b += __shfl_xor(b, 16, 64);
@@ -454,6 +521,7 @@ __global__ __launch_bounds__(256) void mlp_bwd_kernel(const float* __restrict__ 
             out[MLP_OFF_B2 + 16 * nt + r16] = b;
         }
     }
+    gb3 = bias[2][0];
     gb3 += __shfl_xor(gb3, 16, 64);
     gb3 += __shfl_xor(gb3, 32, 64);
     if (g == 0 && r16 < MLP_OUT) out[MLP_OFF_B3 + r16] = gb3;
@@ -462,15 +530,32 @@ __global__ __launch_bounds__(256) void mlp_bwd_kernel(const float* __restrict__ 
 // grads[k] = sum over the partials in a fixed order: 8 groups of 32 threads per workgroup, group
 // g summing its contiguous eighth of the partials for 32 parameters, then the eight group sums
 // added in group order.
+// One more workgroup sums the wavefronts' loss shares.
 constexpr int MLP_RED_PARAMS = 32;
 __global__ __launch_bounds__(256) void mlp_reduce_kernel(const float* __restrict__ partial,
-                                                         int parts, float* __restrict__ grads) {
+                                                         int parts, float* __restrict__ grads,
+                                                         const float* __restrict__ loss_part,
+                                                         size_t waves, float* __restrict__ loss) {
     __shared__ float acc[8][MLP_RED_PARAMS];
     const int g = threadIdx.x / MLP_RED_PARAMS, t = threadIdx.x % MLP_RED_PARAMS;
+    if (blockIdx.x == gridDim.x - 1) {
+        __shared__ float red[256];
+        float s = 0.f;
+        for (size_t i = threadIdx.x; i < waves; i += 256) s += loss_part[i];
+        red[threadIdx.x] = s;
+        __syncthreads();
+        for (int w = 128; w > 0; w >>= 1) {
+            if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) *loss = red[0];
+        return;
+    }
     const int k = blockIdx.x * MLP_RED_PARAMS + t;
     const int per = (parts + 7) / 8, p0 = g * per, p1 = min(parts, p0 + per);
     float s = 0.f;
     if (k < MLP_NPARAM)
+#pragma unroll 8
         for (int p = p0; p < p1; ++p) s += partial[size_t(p) * MLP_NPARAM + k];
     acc[g][t] = s;
     __syncthreads();
@@ -493,19 +578,6 @@ __global__ void mlp_adam_kernel(float* __restrict__ p, const float* __restrict__
     m[k] = mk;
     v[k] = vk;
     p[k] -= lr * (mk / c1) / (sqrtf(vk / c2) + 1e-8f);
-}
-
-__global__ void mlp_loss_sum_kernel(const float* __restrict__ part, size_t n, float* __restrict__ out) {
-    __shared__ float red[256];
-    float s = 0.f;
-    for (size_t i = threadIdx.x; i < n; i += 256) s += part[i];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *out = red[0];
 }
 
 // ---- host helpers ------------------------------------------------------------------------------
@@ -615,7 +687,7 @@ static int step_grads(pnb_ctx* c, float* loss_dev) {
     PNB_HIP(c, s->y.ensure(std::max<size_t>(1, s->rows) * MLP_YS * 4));
     PNB_HIP(c, s->gy.ensure(std::max<size_t>(1, s->rows) * MLP_YS * 4));
     PNB_HIP(c, s->loss_part.ensure(s->waves * 4));
-    PNB_HIP(c, s->partial.ensure(size_t(MLP_BWD_BLOCKS) * MLP_WAVES_PER_BLOCK * MLP_NPARAM * 4));
+    PNB_HIP(c, s->partial.ensure(size_t(MLP_BWD_BLOCKS) * MLP_NPARAM * 4));
     if (!s->chunks_ok) {
         // once per training set: lanes with a positive weight, and the row chunks
         std::vector<float> hw(s->waves * 64);
@@ -660,7 +732,7 @@ static int step_grads(pnb_ctx* c, float* loss_dev) {
             PNB_CHECK_LAUNCH(c);
         }
         mlp_pred_kernel<<<unsigned(s->chunks), 64, 0, c->stream>>>(
-            s->y.as<float>(), s->wave_rows.as<uint32_t>(), s->chunk_wave.as<uint32_t>(),
+            s->y.as<float4>(), s->wave_rows.as<uint32_t>(), s->chunk_wave.as<uint32_t>(),
             s->chunk_rb.as<uint32_t>(), s->mask.as<unsigned long long>(), s->geom.as<float4>(),
             s->lanes.as<float4>(), s->part.as<float4>());
         PNB_CHECK_LAUNCH(c);
@@ -675,13 +747,13 @@ static int step_grads(pnb_ctx* c, float* loss_dev) {
                 s->gy.as<float>());
             PNB_CHECK_LAUNCH(c);
         }
-        mlp_loss_sum_kernel<<<1, 256, 0, c->stream>>>(s->loss_part.as<float>(), s->waves, loss_dev);
+        const int blocks = int(std::min<unsigned>(MLP_BWD_BLOCKS, div_up(tiles, MLP_BWD_WAVES)));
+        mlp_bwd_kernel<<<blocks, 64 * MLP_BWD_WAVES, 0, c->stream>>>(
+            s->feats.as<float>(), s->gy.as<float>(), s->rows, wg, s->partial.as<float>());
         PNB_CHECK_LAUNCH(c);
-        mlp_bwd_kernel<<<MLP_BWD_BLOCKS, 256, 0, c->stream>>>(s->feats.as<float>(), s->gy.as<float>(),
-                                                             s->rows, wg, s->partial.as<float>());
-        PNB_CHECK_LAUNCH(c);
-        mlp_reduce_kernel<<<div_up(MLP_NPARAM, MLP_RED_PARAMS), 256, 0, c->stream>>>(
-            s->partial.as<float>(), MLP_BWD_BLOCKS * MLP_WAVES_PER_BLOCK, s->grads.as<float>());
+        mlp_reduce_kernel<<<div_up(MLP_NPARAM, MLP_RED_PARAMS) + 1, 256, 0, c->stream>>>(
+            s->partial.as<float>(), blocks, s->grads.as<float>(), s->loss_part.as<float>(), s->waves,
+            loss_dev);
         PNB_CHECK_LAUNCH(c);
         return PNB_OK;
     });
