@@ -1304,15 +1304,17 @@ struct WalkRows {
 };
 
 // Advances the wavefront's cursor: (k, r) = (open != 0) ? (kn, rn) : (ks, rs), with the
-// operands and results in SGPRs (one scalar compare and four scalar selects). Left to itself the
-// compiler copies both candidate records into VGPRs and selects them with v_cndmask.
+// operands and results in SGPRs (four scalar selects on the scalar condition code). Left to itself
+// the compiler copies both candidate records into VGPRs and selects them with v_cndmask. open is
+// live & crit, made here because the AND sets that condition code; with SEL3 (the relative criterion,
+// whose buckets can clear it) it is the caller's.
 __device__ __forceinline__ uint64_t pack2(uint32_t lo, uint32_t hi) {
     return uint64_t(lo) | (uint64_t(hi) << 32);
 }
 
 template <typename Off, bool SEL3>
-__device__ __forceinline__ void advance(uint64_t open, Off kn, Off ks, Off& k, NodeRec& r,
-                                        const NodeRec& rn, const NodeRec& rs) {
+__device__ __forceinline__ void advance(uint64_t& open, uint64_t live, uint64_t crit, Off kn, Off ks,
+                                        Off& k, NodeRec& r, const NodeRec& rn, const NodeRec& rs) {
     const uint64_t n0 = pack2(__float_as_uint(rn.cx), __float_as_uint(rn.cy));
     const uint64_t s0 = pack2(__float_as_uint(rs.cx), __float_as_uint(rs.cy));
     const uint64_t n1 = pack2(__float_as_uint(rn.cz), __float_as_uint(rn.mass));
@@ -1352,25 +1354,25 @@ __device__ __forceinline__ void advance(uint64_t open, Off kn, Off ks, Off& k, N
         }
     } else if constexpr (sizeof(Off) == 4) {
         asm volatile(
-            "s_cmp_lg_u64 %4, 0\n\t"
+            "s_and_b64 %4, %15, %16\n\t"
             "s_cselect_b64 %0, %5, %6\n\t"
             "s_cselect_b64 %1, %7, %8\n\t"
             "s_cselect_b64 %2, %9, %10\n\t"
             "s_cselect_b32 %3, %11, %12"
-            : "=&s"(o0), "=&s"(o1), "=&s"(o2), "=&s"(ok)
-            : "s"(open), "s"(n0), "s"(s0), "s"(n1), "s"(s1), "s"(n2), "s"(s2), "s"(kn), "s"(ks),
-              "s"(n3), "s"(s3)
+            : "=&s"(o0), "=&s"(o1), "=&s"(o2), "=&s"(ok), "=&s"(open)
+            : "s"(n0), "s"(s0), "s"(n1), "s"(s1), "s"(n2), "s"(s2), "s"(kn), "s"(ks),
+              "s"(n3), "s"(s3), "s"(live), "s"(crit)
             : "scc");
     } else {
         asm volatile(
-            "s_cmp_lg_u64 %4, 0\n\t"
+            "s_and_b64 %4, %15, %16\n\t"
             "s_cselect_b64 %0, %5, %6\n\t"
             "s_cselect_b64 %1, %7, %8\n\t"
             "s_cselect_b64 %2, %9, %10\n\t"
             "s_cselect_b64 %3, %11, %12"
-            : "=&s"(o0), "=&s"(o1), "=&s"(o2), "=&s"(ok)
-            : "s"(open), "s"(n0), "s"(s0), "s"(n1), "s"(s1), "s"(n2), "s"(s2), "s"(kn), "s"(ks),
-              "s"(n3), "s"(s3)
+            : "=&s"(o0), "=&s"(o1), "=&s"(o2), "=&s"(ok), "=&s"(open)
+            : "s"(n0), "s"(s0), "s"(n1), "s"(s1), "s"(n2), "s"(s2), "s"(kn), "s"(ks),
+              "s"(n3), "s"(s3), "s"(live), "s"(crit)
             : "scc");
     }
     r.cx = __uint_as_float(uint32_t(o0));
@@ -1410,12 +1412,14 @@ __device__ __forceinline__ float half_hi(uint32_t v) {
 
 // One wavefront walks the pre-order node records with one cursor (k, in SGPRs); lane decisions
 // are the reference's (see the file comment). The walk is bound by its instruction stream as a
-// whole (about 33 VALU, 15 SALU and 2 scalar loads per step for the plain walk, and the latency
-// of those loads), so the step keeps everything wave-uniform in SGPRs: the records of both
+// whole (about 34 VALU, 13 SALU and 2 scalar loads per step for the plain walk: 98 cycles of a SIMD
+// each, with eight wavefronts on it), so the step keeps everything wave-uniform in SGPRs: the records of both
 // possible next nodes (k + 1, skip) are requested at the top of the step and picked with scalar
 // selects at its end, and the corrected walks fetch the learned entry of node k only when some
 // lane accepts it as an internal node (prefetching it for both candidates costs more
-// scalar-cache misses than it hides).
+// scalar-cache misses than it hides). With theta^2 and eps^2 on vector registers and the masks
+// combined as scalars a pass over 4,194,304 bodies at theta 0.5 went from 12.40 to 12.15 ms in the
+// walk, the corrected one over 1,048,576 from 6.53 to 6.38 ms.
 // WIDE: 64-bit byte offsets, for trees whose records span 4 GiB or more (2^27 nodes).
 // REL: the relative criterion. Each lane holds A = alpha |a~| (est_in[i >> est_shift], from an
 // estimate pass per particle, est_shift = 0, or per wavefront, est_shift = 6) and
@@ -1500,6 +1504,9 @@ __global__ __launch_bounds__(256) void bh_walk_kernel(const NodeRec* __restrict_
     Off ko = 0;
     NodeRec r{};
     if (total > 0) r = nodes[0];  // no tree (m = 0): nodes may not even be allocated
+    // A VALU instruction with a scalar operand issues at half the rate of one on vector registers
+    // alone: these two are used in every step.
+    asm volatile("" : "+v"(theta2), "+v"(eps2));
     while (ko < end) {
         // in bounds: k + 1 <= total and skip <= total, and the array holds total + 1 records
         const Off so = Off(r.skip) * Off(sizeof(NodeRec));
@@ -1519,17 +1526,16 @@ __global__ __launch_bounds__(256) void bh_walk_kernel(const NodeRec* __restrict_
         const float lhs = REL ? (REL_INV ? mul_rn(OCT ? mul_rn(K, inv_rel) : K, inv_rel) : K)
                               : 0.f;
         const float rhs = REL ? mul_rn(mul_rn(A, r2_rel), r2_rel) : 0.f;
-        const bool crit = mul_rn(theta2, d2) < r.w2 || (REL && rhs < lhs);
-        bool open = active && nz && crit;
-        const bool acc = active && nz && !crit;
-        // the wavefront's open mask from the compares' own lane masks (a ballot of the combined
-        // bool would first copy it into a VGPR)
+        // the open and accepting masks from the compares' own lane masks, combined as scalars (of
+        // bools the compiler made two more scalar instructions and a branch)
         const uint64_t live_mask = __builtin_amdgcn_ballot_w64(active) &
                                    __builtin_amdgcn_ballot_w64(nz);
         uint64_t crit_mask = __builtin_amdgcn_fcmpf(mul_rn(theta2, d2), r.w2, 4 /*olt*/);
         if constexpr (REL) crit_mask |= __builtin_amdgcn_fcmpf(rhs, lhs, 4 /*olt*/);
-        uint64_t open_mask = live_mask & crit_mask;
+        uint64_t open_mask = REL ? live_mask & crit_mask : 0;  // without REL: from advance()
+        bool open = REL && __builtin_amdgcn_inverse_ballot_w64(open_mask);
         const uint64_t acc_mask = live_mask & ~crit_mask;
+        const bool acc = __builtin_amdgcn_inverse_ballot_w64(acc_mask);
         if constexpr (REL) {
             const uint32_t bucket = r.end;
             if (bucket != 0 && open_mask != 0) {  // a small node that some lanes open
@@ -1681,12 +1687,13 @@ __global__ __launch_bounds__(256) void bh_walk_kernel(const NodeRec* __restrict_
                 ++nrows;
             }
         }
+        ++steps;
+        // skip > k for every node, and skip = k + 1 for a leaf, so the two candidates agree there
+        advance<Off, REL>(open_mask, live_mask, crit_mask, ko + Off(32), so, ko, r, r_next, r_skip);
+        if constexpr (!REL) open = __builtin_amdgcn_inverse_ballot_w64(open_mask);
         // active && !open: resume at skip. An inactive lane sits inside a skipped subtree that
         // contains node k, so its resume point is already >= skip(k) and the max keeps it.
         if (!open) resume = max(resume, so);
-        ++steps;
-        // skip > k for every node, and skip = k + 1 for a leaf, so the two candidates agree there
-        advance<Off, REL>(open_mask, ko + Off(32), so, ko, r, r_next, r_skip);
     }
     if constexpr (PARTIAL) fold_partial(ax, ay, az, cx, cy, cz, px, py, pz);
     if (MODE == WALK_ROWS && lane == 0 && wave_slot * 64 < n) {  // wavefronts holding particles
