@@ -193,16 +193,25 @@ __global__ void bt_pack_kernel(const double* __restrict__ x3, const double* __re
     sh[i] = make_float4(float(x3[3 * i]), float(x3[3 * i + 1]), float(x3[3 * i + 2]), mu[i]);
 }
 
+// A step's drift with the half kick before it and, TWO, the previous step's last half kick (the
+// same two additions to v, from the same a); also resets the queue for the step's force launch.
+template <bool TWO>
 __global__ void bt_kick_drift_kernel(double4* __restrict__ x, double4* __restrict__ v,
                                      const float4* __restrict__ acc, float4* __restrict__ sh,
-                                     size_t n, double h, double dt) {
+                                     size_t n, double h, double dt, uint32_t* __restrict__ queue) {
     size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n) return;
+    if (i == 0) *queue = 0u;
     const float4 a = acc[i];
     double4 vi = v[i];
     vi.x += double(a.x) * h;
     vi.y += double(a.y) * h;
     vi.z += double(a.z) * h;
+    if (TWO) {
+        vi.x += double(a.x) * h;
+        vi.y += double(a.y) * h;
+        vi.z += double(a.z) * h;
+    }
     double4 xi = x[i];
     xi.x += vi.x * dt;
     xi.y += vi.y * dt;
@@ -284,6 +293,7 @@ static int build_items(pnb_ctx* c, BatchState* s) {
     return PNB_OK;
 }
 
+// The queue has to be 0 (bt_queue_reset_kernel, bt_kick_drift_kernel).
 static int force(pnb_ctx* c, BatchState* s) {
     const bool mask = s->checked && s->softening == 0.0f;
     const float eps2 = s->softening * s->softening;
@@ -297,8 +307,6 @@ static int force(pnb_ctx* c, BatchState* s) {
     int occ = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k, int(block), 0) != hipSuccess || occ < 1) occ = 2;
     const unsigned grid = unsigned(std::max(1, c->cu_count) * occ);
-    bt_queue_reset_kernel<<<1, 1, 0, c->stream>>>(s->queue.as<uint32_t>());
-    PNB_CHECK_LAUNCH(c);
     return timed(c, PNB_PROF_BATCH, [&]() -> int {
         k<<<grid, block, 0, c->stream>>>(s->items.as<BatchItem>(), uint32_t(s->n_items),
                                          s->queue.as<uint32_t>(), s->shadow.as<float4>(), eps2,
@@ -312,11 +320,13 @@ static int enqueue(pnb_ctx* c, BatchState* s, size_t steps, double dt) {
     const unsigned g = div_up(s->total, 256);
     const double h = 0.5 * dt;
     for (size_t k = 0; k < steps; ++k) {
-        bt_kick_drift_kernel<<<g, 256, 0, c->stream>>>(s->x.as<double4>(), s->v.as<double4>(),
-                                                       s->acc.as<float4>(), s->shadow.as<float4>(),
-                                                       s->total, h, dt);
+        (k == 0 ? bt_kick_drift_kernel<false> : bt_kick_drift_kernel<true>)<<<g, 256, 0, c->stream>>>(
+            s->x.as<double4>(), s->v.as<double4>(), s->acc.as<float4>(), s->shadow.as<float4>(),
+            s->total, h, dt, s->queue.as<uint32_t>());
         PNB_CHECK_LAUNCH(c);
         if (int rc = force(c, s)) return rc;
+    }
+    if (steps) {
         bt_kick_kernel<<<g, 256, 0, c->stream>>>(s->v.as<double4>(), s->acc.as<float4>(), s->total, h);
         PNB_CHECK_LAUNCH(c);
     }
@@ -379,6 +389,8 @@ int pnb_batch_init(pnb_ctx* c, const double* pos3, const double* vel3, const flo
                                                               s->v.as<double4>(), s->shadow.as<float4>());
     PNB_CHECK_LAUNCH(c);
     if (int rc = build_items(c, s)) return rc;
+    bt_queue_reset_kernel<<<1, 1, 0, c->stream>>>(s->queue.as<uint32_t>());
+    PNB_CHECK_LAUNCH(c);
     if (int rc = force(c, s)) return rc;
     PNB_HIP(c, hipStreamSynchronize(c->stream));
     return PNB_OK;

@@ -8,7 +8,8 @@
 // compacted once, in their original order, by a precomputed rank (Ordered::new,
 // particular/src/storage.rs:85-95).
 //
-// One step: v += a dt/2; x += v dt; refresh the shadows; a = brute force; v += a dt/2.
+// One step: v += a dt/2; x += v dt; refresh the shadows; a = brute force; v += a dt/2 (the last with
+// the next step's first, in one launch).
 // The steps can be captured once into a hipGraph and replayed (no memset nodes, no allocation
 // inside the capture).
 #include "pnb_internal.hpp"
@@ -62,6 +63,9 @@ __global__ void lf_compact_kernel(const float4* __restrict__ shadow, const uint3
     if (i < n && shadow[i].w != 0.0f) afg[rank[i]] = shadow[i];
 }
 
+// A step's drift with the half kick before it and, TWO, the previous step's last half kick (the
+// same two additions to v, from the same a): one launch and one pass over v fewer per step.
+template <bool TWO>
 __global__ void lf_kick_drift_kernel(double4* __restrict__ x, double4* __restrict__ v,
                                      const float4* __restrict__ acc, float4* __restrict__ shadow,
                                      const uint32_t* __restrict__ rank, float4* __restrict__ afg,
@@ -73,6 +77,11 @@ __global__ void lf_kick_drift_kernel(double4* __restrict__ x, double4* __restric
     vi.x += double(a.x) * h;
     vi.y += double(a.y) * h;
     vi.z += double(a.z) * h;
+    if (TWO) {
+        vi.x += double(a.x) * h;
+        vi.y += double(a.y) * h;
+        vi.z += double(a.z) * h;
+    }
     double4 xi = x[i];
     xi.x += vi.x * dt;
     xi.y += vi.y * dt;
@@ -111,7 +120,7 @@ static int enqueue_steps(pnb_ctx* c, StepState* s, size_t steps, double dt) {
     const double h = 0.5 * dt;
     for (size_t k = 0; k < steps; ++k) {
         int rc = timed(c, PNB_PROF_DRIFT, [&]() -> int {
-            lf_kick_drift_kernel<<<g, 256, 0, c->stream>>>(
+            (k == 0 ? lf_kick_drift_kernel<false> : lf_kick_drift_kernel<true>)<<<g, 256, 0, c->stream>>>(
                 s->x.as<double4>(), s->v.as<double4>(), s->acc.as<float4>(), s->shadow.as<float4>(),
                 s->rank.as<uint32_t>(), s->afg.as<float4>(), s->n, h, dt);
             PNB_CHECK_LAUNCH(c);
@@ -121,6 +130,8 @@ static int enqueue_steps(pnb_ctx* c, StepState* s, size_t steps, double dt) {
         rc = bf_launch(c, s->shadow.as<float4>(), s->n, s->afg.as<float4>(), s->m, s->softening,
                        s->checked, s->acc.as<float4>());
         if (rc) return rc;
+    }
+    if (steps) {
         lf_kick_kernel<<<g, 256, 0, c->stream>>>(s->v.as<double4>(), s->acc.as<float4>(), s->n, h);
         PNB_CHECK_LAUNCH(c);
     }
