@@ -187,9 +187,10 @@ struct BfShape {
 // split of the plain kernel / cooperative, softened: 1,000 x 1,000 34 / 8 us; 4,096 x 4,096 36 / 11;
 // 1,000 x 65,536 91 / 28; 4,096 x 65,536 102 / 96; 8,192 x 8,192 28 / 27 (6.7e7 pairs); 12,000 x
 // 16,384 67 / 92; 32,768 x 4,096 45 / 42; 300,000 x 5,000 385 / 430; 65,536 x 1,000 78 / 21;
-// 1,000,000 x 1,000 291 / 273; 50,000 x 64 4.2 / 7.4 (one tile: nothing to share).
+// 1,000,000 x 1,000 291 / 273; 256 x 100 6.0 / 8.8, 256 x 128 6.9 / 7.6, 256 x 200 9.8 / 8.7 (two
+// tiles: little to share).
 static bool coop_pays(size_t n, size_t m) {
-    if (m <= 64 || (m <= 256 && n > 32768)) return false;
+    if (m <= 128 || (m <= 256 && n > 32768)) return false;
     const double pairs = double(n) * double(m);
     return pairs <= (m < 2048 ? 1e9 : n <= 4096 ? 3e8 : m <= 4096 ? 1.5e8 : 7e7);
 }
@@ -206,12 +207,13 @@ static BfShape default_shape(pnb_ctx* c, size_t n, size_t m) {
     }
     // Otherwise one body per lane and one wavefront per affected tile and range, the affecting
     // bodies from scalar loads (from LDS below 32,768 affected bodies, where few wavefronts hide
-    // their latency, 12,000 x 16,384 67 / 70 us, and for at most a tile, 65,536 x 64 4 / 9 us), the affecting range split into up to 64 workgroups
-    // per CU of at least one tile each, up to 256 per CU while ranges stay at 1,024 bodies
-    // (small workgroups balance the load across CUs and XCDs). 1,048,576 x 65,536 16.1 ms, with four
+    // their latency, 12,000 x 16,384 67 / 70 us, and for at most a tile, 65,536 x 64 4 / 9 us), the
+    // affecting range from 2,048 bodies on split into up to 64 workgroups per CU of at least one
+    // tile each, up to 256 per CU while ranges stay at 1,024 bodies (small workgroups balance the
+    // load across CUs and XCDs; what is left below 2,048 has enough of them unsplit). 1,048,576 x 65,536 16.1 ms, with four
     // bodies per lane 17.1; 65,536 x 16,384 286 us, 333.
     const size_t blocks = div_up(n, size_t(BF_BLOCK));
-    while (s < 64 && blocks * s * 2 <= 256 * cus) {
+    while (m >= 2048 && s < 64 && blocks * s * 2 <= 256 * cus) {
         const size_t per = m / (size_t(s) * 2);
         if (per < (blocks * s * 2 <= 64 * cus ? size_t(BF_TILE) : size_t(1024))) break;
         s <<= 1;
@@ -260,7 +262,7 @@ int bf_prepare(pnb_ctx* c, size_t n, size_t m) {
 
 // Scratch of the allocation-free entry point (pnb_bf_accel_f32_dev_noalloc): the partial sums of
 // the affecting split, splits * n records. 256 MiB: the default shapes need at most
-// 64 * CUs * BF_BLOCK * 4 records (16,777,216 on 256 CUs). Every GPU the library runs on holds its
+// 256 * CUs * BF_BLOCK records (16,777,216 on 256 CUs). Every GPU the library runs on holds its
 // own copy until the process ends; every call on that GPU shares it.
 constexpr size_t BF_SCRATCH_RECORDS = size_t(1) << 24;
 static __device__ __align__(256) float4 scratch[BF_SCRATCH_RECORDS];
