@@ -460,18 +460,13 @@ __global__ __launch_bounds__(64) void bf64_reduce_kernel(const double4* __restri
     out[i] = make_double4(ax, ay, az, 0.0);
 }
 
-static int copy_in(pnb_ctx* c, DevBuf& b, const float* src, size_t count) {
-    PNB_HIP(c, b.ensure(count * sizeof(float4)));
-    if (count)
-        PNB_HIP(c, hipMemcpyAsync(b.ptr, src, count * sizeof(float4), hipMemcpyHostToDevice, c->stream));
-    return PNB_OK;
-}
-
-static int copy_out(pnb_ctx* c, float* dst, const DevBuf& b, size_t count) {
-    if (count)
-        PNB_HIP(c, hipMemcpyAsync(dst, b.ptr, count * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
-    PNB_HIP(c, hipStreamSynchronize(c->stream));
-    return PNB_OK;
+// Both sides of a sum over host arrays. A set on itself, or on its own first m bodies, passes one
+// pointer twice and is uploaded once.
+static int upload_sides(pnb_ctx* c, const void* affected, size_t n, const void* affecting, size_t m,
+                        size_t record) {
+    if (affecting == affected) return stage_in(c, c->h_affected, affected, std::max(n, m) * record);
+    if (int rc = stage_in(c, c->h_affected, affected, n * record)) return rc;
+    return stage_in(c, c->h_affecting, affecting, m * record, 1);
 }
 
 }  // namespace pnb
@@ -530,13 +525,14 @@ int pnb_bf_accel_f32(pnb_ctx* c, const float* affected, size_t n, const float* a
     if (!(softening >= 0.0f)) return fail(c, PNB_E_ARG, "softening must be >= 0");
     if (n == 0) return PNB_OK;
     if (int rc = activate(c)) return rc;
-    if (int rc = copy_in(c, c->h_affected, affected, n)) return rc;
-    if (int rc = copy_in(c, c->h_affecting, affecting, m)) return rc;
-    PNB_HIP(c, c->h_out.ensure(n * sizeof(float4)));
-    if (int rc = bf_launch(c, c->h_affected.as<float4>(), n, c->h_affecting.as<float4>(), m,
-                           softening, checked, c->h_out.as<float4>()))
+    void* o;
+    if (int rc = upload_sides(c, affected, n, affecting, m, sizeof(float4))) return rc;
+    if (int rc = stage_out(c, c->h_out, n * sizeof(float4), &o)) return rc;
+    const DevBuf& b = affecting == affected ? c->h_affected : c->h_affecting;
+    if (int rc = bf_launch(c, c->h_affected.as<float4>(), n, b.as<float4>(), m, softening, checked,
+                           static_cast<float4*>(o)))
         return rc;
-    return copy_out(c, out, c->h_out, n);
+    return stage_done(c, out, o, n * sizeof(float4));
 }
 
 int pnb_reordered_bf_accel_f32_dev(pnb_ctx* c, const float* particles, size_t n, float softening,
@@ -561,12 +557,13 @@ int pnb_reordered_bf_accel_f32(pnb_ctx* c, const float* particles, size_t n, flo
     if (!(softening >= 0.0f)) return fail(c, PNB_E_ARG, "softening must be >= 0");
     if (n == 0) return PNB_OK;
     if (int rc = activate(c)) return rc;
-    if (int rc = copy_in(c, c->h_affected, particles, n)) return rc;
-    PNB_HIP(c, c->h_out.ensure(n * sizeof(float4)));
+    void* o;
+    if (int rc = stage_in(c, c->h_affected, particles, n * sizeof(float4))) return rc;
+    if (int rc = stage_out(c, c->h_out, n * sizeof(float4), &o)) return rc;
     if (int rc = pnb_reordered_bf_accel_f32_dev(c, c->h_affected.as<float>(), n, softening,
-                                                checked, c->h_out.as<float>()))
+                                                checked, static_cast<float*>(o)))
         return rc;
-    return copy_out(c, out, c->h_out, n);
+    return stage_done(c, out, o, n * sizeof(float4));
 }
 
 int pnb_bf_set_tuning(pnb_ctx* c, size_t n_min, int variant, int per_lane, int j_split) {
@@ -655,17 +652,14 @@ int pnb_bf_accel_f64(pnb_ctx* c, const double* affected, size_t n, const double*
         return fail(c, PNB_E_ARG, "null pointer with non-zero length");
     if (n == 0) return PNB_OK;
     if (int rc = activate(c)) return rc;
-    PNB_HIP(c, c->h_affected.ensure(n * 32));
-    PNB_HIP(c, c->h_affecting.ensure(std::max<size_t>(m, 1) * 32));
-    PNB_HIP(c, c->h_out.ensure(n * 32));
-    PNB_HIP(c, hipMemcpyAsync(c->h_affected.ptr, affected, n * 32, hipMemcpyHostToDevice, c->stream));
-    if (m) PNB_HIP(c, hipMemcpyAsync(c->h_affecting.ptr, affecting, m * 32, hipMemcpyHostToDevice, c->stream));
-    if (int rc = pnb_bf_accel_f64_dev(c, c->h_affected.as<double>(), n, c->h_affecting.as<double>(), m,
-                                      softening, checked, c->h_out.as<double>()))
+    void* o;
+    if (int rc = upload_sides(c, affected, n, affecting, m, sizeof(double4))) return rc;
+    if (int rc = stage_out(c, c->h_out, n * sizeof(double4), &o)) return rc;
+    const DevBuf& b = affecting == affected ? c->h_affected : c->h_affecting;
+    if (int rc = pnb_bf_accel_f64_dev(c, c->h_affected.as<double>(), n, b.as<double>(), m, softening,
+                                      checked, static_cast<double*>(o)))
         return rc;
-    PNB_HIP(c, hipMemcpyAsync(out, c->h_out.ptr, n * 32, hipMemcpyDeviceToHost, c->stream));
-    PNB_HIP(c, hipStreamSynchronize(c->stream));
-    return PNB_OK;
+    return stage_done(c, out, o, n * sizeof(double4));
 }
 
 }  // extern "C"

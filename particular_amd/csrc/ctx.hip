@@ -1,6 +1,8 @@
 // Context, errors, profiling, device-wide scan and the massive/massless split.
 #include "pnb_internal.hpp"
 
+#include <cstring>
+
 #include <new>
 
 namespace pnb {
@@ -55,6 +57,48 @@ int prof_resolve(pnb_ctx* c) {
         c->prof_count[c->ev_kernel[k]] += 1;
     }
     c->ev_used = 0;
+    return PNB_OK;
+}
+
+__global__ __launch_bounds__(256) void stage_kernel(const uint4* __restrict__ src, size_t n,
+                                                    uint4* __restrict__ dst) {
+    const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
+int stage_in(pnb_ctx* c, DevBuf& dst, const void* src, size_t bytes, int slot) {
+    PNB_HIP(c, dst.ensure(std::max<size_t>(bytes, 16)));
+    if (bytes == 0) return PNB_OK;
+    if (bytes > HOST_STAGE) {
+        PNB_HIP(c, hipMemcpyAsync(dst.ptr, src, bytes, hipMemcpyHostToDevice, c->stream));
+        return PNB_OK;
+    }
+    if (!c->pin_in) PNB_HIP(c, hipHostMalloc(&c->pin_in, 2 * HOST_STAGE));
+    char* pin = static_cast<char*>(c->pin_in) + slot * HOST_STAGE;
+    std::memcpy(pin, src, bytes);
+    stage_kernel<<<div_up(bytes / 16, 256), 256, 0, c->stream>>>(
+        reinterpret_cast<const uint4*>(pin), bytes / 16, dst.as<uint4>());
+    PNB_CHECK_LAUNCH(c);
+    return PNB_OK;
+}
+
+int stage_out(pnb_ctx* c, DevBuf& dev, size_t bytes, void** where) {
+    if (bytes > HOST_STAGE) {
+        PNB_HIP(c, dev.ensure(bytes));
+        *where = dev.ptr;
+        return PNB_OK;
+    }
+    if (!c->pin_out) PNB_HIP(c, hipHostMalloc(&c->pin_out, HOST_STAGE));
+    *where = c->pin_out;
+    return PNB_OK;
+}
+
+int stage_done(pnb_ctx* c, void* out, const void* where, size_t bytes) {
+    const bool pinned = where == c->pin_out;
+    if (!pinned && bytes)
+        PNB_HIP(c, hipMemcpyAsync(out, where, bytes, hipMemcpyDeviceToHost, c->stream));
+    PNB_HIP(c, hipStreamSynchronize(c->stream));
+    if (pinned) std::memcpy(out, where, bytes);
     return PNB_OK;
 }
 
@@ -299,6 +343,8 @@ void pnb_destroy(pnb_ctx* c) {
     pnb::step_free(c->step);
     pnb::batch_free(c->batch);
     pnb::mlp_free(c->mlp);
+    for (void* p : {c->pin_in, c->pin_out})
+        if (p) (void)hipHostFree(p);
     for (pnb::DevBuf* b : {&c->h_affected, &c->h_affecting, &c->h_out, &c->split_tmp,
                            &c->split_flags, &c->bf_partial, &c->scan_tmp, &c->pairs_part, &c->d2_raw_a,
                            &c->d2_raw_b, &c->d2_a, &c->d2_b, &c->d2_out4, &c->d2_out2})

@@ -279,17 +279,13 @@ int pnb_bf_pairs_accel_f32(pnb_ctx* c, const float* particles, size_t n, float s
     if (n > PR_MAX_N)
         return fail(c, PNB_E_ARG, "pair brute force takes at most %zu particles", PR_MAX_N);
     if (int rc = activate(c)) return rc;
-    PNB_HIP(c, c->h_affected.ensure(n * sizeof(float4)));
-    PNB_HIP(c, c->h_out.ensure(n * sizeof(float4)));
-    PNB_HIP(c, hipMemcpyAsync(c->h_affected.ptr, particles, n * sizeof(float4),
-                              hipMemcpyHostToDevice, c->stream));
+    void* o;
+    if (int rc = stage_in(c, c->h_affected, particles, n * sizeof(float4))) return rc;
+    if (int rc = stage_out(c, c->h_out, n * sizeof(float4), &o)) return rc;
     if (int rc = pairs_launch(c, c->h_affected.as<float4>(), n, softening, checked,
-                              c->h_out.as<float4>()))
+                              static_cast<float4*>(o)))
         return rc;
-    PNB_HIP(c, hipMemcpyAsync(out, c->h_out.ptr, n * sizeof(float4), hipMemcpyDeviceToHost,
-                              c->stream));
-    PNB_HIP(c, hipStreamSynchronize(c->stream));
-    return PNB_OK;
+    return stage_done(c, out, o, n * sizeof(float4));
 }
 
 }  // extern "C"
