@@ -177,7 +177,7 @@ void bh_free(BhState* s) {
                       &s->c_count, &s->c_target, &s->c_wgt, &s->c_rows, &s->c_rwave, &s->c_cfeats,
                       &s->c_cgeom, &s->c_cmask, &s->c_lanes, &s->feat_out})
         b->release();
-    if (s->host_info) hipHostFree(s->host_info);
+    if (s->host_info) (void)hipHostFree(s->host_info);
     delete s;
 }
 
@@ -513,9 +513,44 @@ __device__ __forceinline__ void chunk_range(size_t m, size_t& c0, size_t& c1) {
     c1 = min(chunks, c0 + per);
 }
 
-// Node counts per particle: a run of equal positions starting at p (lcp[p] != LCP_SAME) starts
-// the nodes of levels lcp[p] + 1 .. I + 1 (I + 1 is its leaf); also the deepest level and the
-// number of internal nodes per level.
+// The number of nodes that start at particle p (none for p >= m), whose ip it writes: a run of equal
+// positions starting at p (lcp[p] != LCP_SAME) starts the nodes of levels lcp[p] + 1 .. I + 1 (I + 1
+// is its leaf). The wavefront's internal nodes per level are added to hist (in LDS), `deepest` is
+// raised to its deepest level.
+__device__ __forceinline__ uint32_t count_nodes(const int* __restrict__ lcp, size_t p, size_t m,
+                                                int* __restrict__ ip, uint32_t* hist, int& deepest) {
+    int top = -1, lo = MAX_LEVEL + 1;
+    uint32_t n_p = 0;
+    if (p < m) {
+        const int lp = lcp[p];  // -1 at p = 0
+        if (lp != LCP_SAME) {
+            size_t r1 = p + 1;
+            while (r1 < m && lcp[r1] == LCP_SAME) ++r1;
+            const int nxt = r1 < m ? lcp[r1] : -1;
+            const int I = max(lp, nxt);
+            n_p = uint32_t(I + 1 - lp);
+            ip[p] = I;
+            top = I + 1;
+            lo = lp + 1;
+        }
+    }
+    const int hi = top - 1;  // internal levels lo .. hi
+    int wlo = lo, wtop = top;
+    for (int off = 32; off > 0; off >>= 1) {
+        wtop = max(wtop, __shfl_xor(wtop, off, 64));
+        wlo = min(wlo, __shfl_xor(wlo, off, 64));
+    }
+    deepest = max(deepest, wtop);
+    // levels above MAX_LEVEL are not counted: the build fails on such a tree
+    const int whi = min(wtop - 1, MAX_LEVEL);
+    for (int l = wlo; l <= whi; ++l) {
+        const uint64_t in = __ballot(lo <= l && l <= hi);
+        if ((threadIdx.x & 63) == 0 && in) atomicAdd(&hist[l], uint32_t(__popcll(in)));
+    }
+    return n_p;
+}
+
+// Node counts per particle, the deepest level and the number of internal nodes per level.
 __global__ __launch_bounds__(256) void bh_count_kernel(const int* __restrict__ lcp, size_t m,
                                                        uint32_t* __restrict__ cnt,
                                                        int* __restrict__ ip,
@@ -530,35 +565,8 @@ __global__ __launch_bounds__(256) void bh_count_kernel(const int* __restrict__ l
     int deepest = -1;
     for (size_t ch = c0; ch < c1; ++ch) {
         const size_t p = ch * BH_CHUNK + threadIdx.x;
-        int top = -1, lo = MAX_LEVEL + 1;
-        if (p < m) {
-            const int lp = lcp[p];  // -1 at p = 0
-            if (lp == LCP_SAME) {
-                cnt[p] = 0;
-            } else {
-                size_t r1 = p + 1;
-                while (r1 < m && lcp[r1] == LCP_SAME) ++r1;
-                const int nxt = r1 < m ? lcp[r1] : -1;
-                const int I = max(lp, nxt);
-                cnt[p] = uint32_t(I + 1 - lp);
-                ip[p] = I;
-                top = I + 1;
-                lo = lp + 1;
-            }
-        }
-        const int hi = top - 1;  // internal levels lo .. hi
-        int wlo = lo, wtop = top;
-        for (int off = 32; off > 0; off >>= 1) {
-            wtop = max(wtop, __shfl_xor(wtop, off, 64));
-            wlo = min(wlo, __shfl_xor(wlo, off, 64));
-        }
-        deepest = max(deepest, wtop);
-        // levels above MAX_LEVEL are not counted: the build fails on such a tree
-        const int whi = min(wtop - 1, MAX_LEVEL);
-        for (int l = wlo; l <= whi; ++l) {
-            const uint64_t in = __ballot(lo <= l && l <= hi);
-            if (lead && in) atomicAdd(&hist[l], uint32_t(__popcll(in)));
-        }
+        const uint32_t n_p = count_nodes(lcp, p, m, ip, hist, deepest);
+        if (p < m) cnt[p] = n_p;
     }
     if (lead && deepest >= 0) {  // only when it raises the maximum seen so far
         if (deepest > __atomic_load_n(&info->max_level, __ATOMIC_RELAXED))
@@ -570,39 +578,114 @@ __global__ __launch_bounds__(256) void bh_count_kernel(const int* __restrict__ l
         if (hist[l]) atomicAdd(&lvl_count[l * LVL_STRIDE], hist[l]);
 }
 
-// Copies the per-level counts and the node count (S[m], the scan's total) into info and sets the
-// list cursors to the counts' exclusive scan. cap > 0 (a capturable build): a tree that needs more
-// nodes or levels than an earlier ordinary build sized flags the build; every later kernel of it
-// then returns at once and the walk writes NaN.
-__global__ __launch_bounds__(256) void bh_level_offsets_kernel(BhInfo* __restrict__ info,
-                                                               const uint32_t* __restrict__ lvl_count,
-                                                               uint32_t* __restrict__ lvl_cur,
-                                                               const uint32_t* __restrict__ S,
-                                                               size_t m, uint32_t cap, int levels) {
+// The per-level counts (n_l of thread l) and the node count into info, and the list cursors set to
+// the counts' exclusive scan; called by the first 256 threads of a workgroup and, for the barrier,
+// by all others. cap > 0 (a capturable build): a tree that needs more nodes or levels than an
+// earlier ordinary build sized flags the build; every later kernel of it then returns at once and
+// the walk writes NaN.
+__device__ __forceinline__ void level_offsets(BhInfo* __restrict__ info, uint32_t n_l, uint32_t total,
+                                              int max_level, uint32_t* __restrict__ lvl_cur, uint32_t cap,
+                                              int levels) {
     static_assert(LVL_SLOTS <= 256, "one thread per level");
     __shared__ uint32_t wsum[4];
     const int l = threadIdx.x, lane = l & 63, w = l >> 6;
-    const uint32_t n_l = l < LVL_SLOTS ? lvl_count[l * LVL_STRIDE] : 0u;
     uint32_t incl = n_l;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
         const uint32_t y = __shfl_up(incl, o, 64);
         if (lane >= o) incl += y;
     }
-    if (lane == 63) wsum[w] = incl;
+    if (lane == 63 && w < 4) wsum[w] = incl;
     __syncthreads();
+    if (l >= LVL_SLOTS) return;
     uint32_t off = incl - n_l;
     for (int q = 0; q < w; ++q) off += wsum[q];
-    if (l < LVL_SLOTS) {
-        info->lvl_count[l] = n_l;
-        info->lvl_off[l] = off;
-        lvl_cur[l * LVL_STRIDE] = off;
-    }
+    info->lvl_count[l] = n_l;
+    info->lvl_off[l] = off;
+    lvl_cur[l * LVL_STRIDE] = off;
     if (l == 0) {
-        const uint32_t total = S[m];
         info->total = total;
-        if (cap && (total > cap || info->max_level > levels)) atomicOr(&info->flags, FLAG_CAPACITY);
+        if (cap && (total > cap || max_level > levels)) atomicOr(&info->flags, FLAG_CAPACITY);
     }
+}
+
+__global__ __launch_bounds__(256) void bh_level_offsets_kernel(BhInfo* __restrict__ info,
+                                                               const uint32_t* __restrict__ lvl_count,
+                                                               uint32_t* __restrict__ lvl_cur,
+                                                               const uint32_t* __restrict__ S,
+                                                               size_t m, uint32_t cap, int levels) {
+    level_offsets(info, threadIdx.x < LVL_SLOTS ? lvl_count[threadIdx.x * LVL_STRIDE] : 0u, S[m],
+                  info->max_level, lvl_cur, cap, levels);
+}
+
+// The counts, their scan and the level offsets for small sets in one workgroup, in place of three
+// launches of 4.5 us: a pass over 200 bodies takes 80 us so and 89 with the three, 1,000 133 and 138,
+// 4,096 the same, 16,000 396 and 391 (one CU then works longer than the launches take). S[p]: the
+// nodes that start before particle p, S[m] their number.
+constexpr size_t COUNT_SMALL = 2048;
+
+__global__ __launch_bounds__(1024) void bh_small_count_kernel(const int* __restrict__ lcp, uint32_t m,
+                                                              uint32_t* __restrict__ S,
+                                                              int* __restrict__ ip,
+                                                              BhInfo* __restrict__ info,
+                                                              uint32_t* __restrict__ lvl_cur,
+                                                              uint32_t cap, int levels) {
+    __shared__ uint32_t hist[256], wsum[2][16];
+    __shared__ int wdeep[16];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (threadIdx.x < 256) hist[threadIdx.x] = 0;
+    __syncthreads();
+    int deepest = -1;
+    uint32_t carry = 0;
+    for (uint32_t p0 = 0, turn = 0; p0 < m; p0 += 1024, turn ^= 1) {
+        const uint32_t p = p0 + threadIdx.x;
+        const uint32_t n_p = count_nodes(lcp, p, m, ip, hist, deepest);
+        uint32_t incl = n_p;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += y;
+        }
+        if (lane == 63) wsum[turn][w] = incl;
+        __syncthreads();  // the other half of wsum is written next, after everyone's reads of it
+        uint32_t all = 0;
+        for (int q = 0; q < 16; ++q) {
+            if (q == w && p < m) S[p] = carry + all + incl - n_p;
+            all += wsum[turn][q];
+        }
+        carry += all;
+    }
+    if (lane == 0) wdeep[w] = deepest;
+    __syncthreads();
+    for (int q = 0; q < 16; ++q) deepest = max(deepest, wdeep[q]);
+    if (threadIdx.x == 0) {
+        S[m] = carry;
+        info->max_level = deepest;
+        if (deepest > MAX_LEVEL) atomicOr(&info->flags, FLAG_DEPTH);
+    }
+    level_offsets(info, threadIdx.x < LVL_SLOTS ? hist[threadIdx.x] : 0u, carry, deepest, lvl_cur, cap,
+                  levels);
+}
+
+// Counts, scan (S = cnt) and offsets. Info's max_level starts at -1 and the level counters at 0.
+static int count_levels(pnb_ctx* c, BhState* s, size_t m, uint32_t cap, int levels) {
+    BhInfo* info = s->info.as<BhInfo>();
+    uint32_t* lvl_count = s->lvl.as<uint32_t>();
+    uint32_t* lvl_cur = lvl_count + LVL_SLOTS * LVL_STRIDE;
+    uint32_t* cnt = s->cnt.as<uint32_t>();
+    if (m <= COUNT_SMALL) {
+        bh_small_count_kernel<<<1, 1024, 0, c->stream>>>(s->lcp.as<int>(), uint32_t(m), cnt, s->ip.as<int>(),
+                                                         info, lvl_cur, cap, levels);
+        PNB_CHECK_LAUNCH(c);
+        return PNB_OK;
+    }
+    const unsigned lg = std::min<unsigned>(div_up(m, 256), 4 * std::max(c->cu_count, 1));
+    bh_count_kernel<<<lg, 256, 0, c->stream>>>(s->lcp.as<int>(), m, cnt, s->ip.as<int>(), info, lvl_count);
+    PNB_CHECK_LAUNCH(c);
+    if (int rc = scan_u32(c, cnt, cnt, m, true)) return rc;
+    bh_level_offsets_kernel<<<1, 256, 0, c->stream>>>(info, lvl_count, lvl_cur, cnt, m, cap, levels);
+    PNB_CHECK_LAUNCH(c);
+    return PNB_OK;
 }
 
 // ilist: the internal nodes of each level together (level l from the exclusive scan of the
@@ -1777,12 +1860,7 @@ static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = fa
                                                  s->key2.as<uint64_t>(), info);
         PNB_CHECK_LAUNCH(c);
         uint32_t* cnt = s->cnt.as<uint32_t>();
-        const unsigned lg = std::min<unsigned>(g, 4 * std::max(c->cu_count, 1));
-        bh_count_kernel<<<lg, 256, 0, c->stream>>>(lcp, m, cnt, s->ip.as<int>(), info, lvl_count);
-        PNB_CHECK_LAUNCH(c);
-        if ((rc = scan_u32(c, cnt, cnt, m, true))) return rc;
-        bh_level_offsets_kernel<<<1, 256, 0, c->stream>>>(info, lvl_count, lvl_cur, cnt, m, 0, 0);
-        PNB_CHECK_LAUNCH(c);
+        if ((rc = count_levels(c, s, m, 0, 0))) return rc;
         if (!s->host_info) PNB_HIP(c, hipHostMalloc(reinterpret_cast<void**>(&s->host_info), sizeof(BhInfo)));
         PNB_HIP(c, hipMemcpyAsync(s->host_info, info, sizeof(BhInfo), hipMemcpyDeviceToHost, c->stream));
         PNB_HIP(c, hipStreamSynchronize(c->stream));
@@ -1830,6 +1908,7 @@ static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = fa
         s->internal = off[levels];
         s->last_lvl.assign(h.lvl_count, h.lvl_count + levels);
         uint32_t* ilist = s->ilist.as<uint32_t>();
+        const unsigned lg = std::min<unsigned>(g, 4 * std::max(c->cu_count, 1));
         bh_level_list_kernel<<<lg, 256, 0, c->stream>>>(lcp, s->ip.as<int>(), cnt, m, lvl_cur,
                                                         ilist, info);
         PNB_CHECK_LAUNCH(c);
@@ -1968,13 +2047,7 @@ static int build_tree_dd(pnb_ctx* c, const float4* afg, size_t m, bool moments, 
         bh_deep_kernel<<<g, 256, 0, c->stream>>>(sk, m, sp, si, lcp, s->key2.as<uint64_t>(), info);
         PNB_CHECK_LAUNCH(c);
         uint32_t* cnt = s->cnt.as<uint32_t>();
-        const unsigned lg = std::min<unsigned>(g, 4 * std::max(c->cu_count, 1));
-        bh_count_kernel<<<lg, 256, 0, c->stream>>>(lcp, m, cnt, s->ip.as<int>(), info, lvl_count);
-        PNB_CHECK_LAUNCH(c);
-        if ((rc = scan_u32(c, cnt, cnt, m, true))) return rc;
-        bh_level_offsets_kernel<<<1, 256, 0, c->stream>>>(info, lvl_count, lvl_cur, cnt, m,
-                                                          uint32_t(s->dd_cap), s->dd_levels);
-        PNB_CHECK_LAUNCH(c);
+        if ((rc = count_levels(c, s, m, uint32_t(s->dd_cap), s->dd_levels))) return rc;
         NodeRec* rec = s->rec.as<NodeRec>();
         uint32_t* skipv = s->skipv.as<uint32_t>();
         NodeMoments* mom = moments ? s->mom.as<NodeMoments>() : nullptr;
@@ -1987,6 +2060,7 @@ static int build_tree_dd(pnb_ctx* c, const float4* afg, size_t m, bool moments, 
                                                  s->width.as<float>(), mom, quad, skipv);
         PNB_CHECK_LAUNCH(c);
         uint32_t* ilist = s->ilist.as<uint32_t>();
+        const unsigned lg = std::min<unsigned>(g, 4 * std::max(c->cu_count, 1));
         bh_level_list_kernel<<<lg, 256, 0, c->stream>>>(lcp, s->ip.as<int>(), cnt, m, lvl_cur,
                                                         ilist, info);
         PNB_CHECK_LAUNCH(c);

@@ -251,7 +251,7 @@ __global__ void rs_bits_init_kernel(unsigned long long* or_and) {
 // vector-scalar compare with no memory access. A workgroup counts against at most RANK_SPAN keys (a
 // quarter of that from 1,025 to 8,192 keys, where there are few workgroups and each is bound by its
 // wavefronts' issue rate: 4,096 keys 17 -> 6 us): inputs above it split the count over blockIdx.y
-// and add the parts with atomics before a scatter launch.
+// into parts, whose ranks a scatter launch adds.
 constexpr uint32_t SMALL_SORT = 16384;
 constexpr uint32_t RANK_SPAN = 1024;
 
@@ -301,7 +301,7 @@ __global__ __launch_bounds__(256) void rank_count_kernel(const uint64_t* __restr
     const uint32_t c = ((cc[0] + cc[1]) + (cc[2] + cc[3])) + ((cc[4] + cc[5]) + (cc[6] + cc[7]));
     if (i >= n) return;
     if (gridDim.y > 1) {
-        atomicAdd(&rank[i], c);
+        rank[size_t(blockIdx.y) * n + i] = c;
         return;
     }
     keys_out[c] = keys[i];
@@ -309,14 +309,10 @@ __global__ __launch_bounds__(256) void rank_count_kernel(const uint64_t* __restr
     if (dst) dst[c] = src[vals[i]];
 }
 
-__global__ __launch_bounds__(256) void rank_zero_kernel(uint32_t* __restrict__ rank, uint32_t n) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) rank[i] = 0u;
-}
-
 __global__ __launch_bounds__(256) void rank_scatter_kernel(const uint64_t* __restrict__ keys,
                                                            const uint32_t* __restrict__ vals,
                                                            uint32_t n,
+                                                           uint32_t parts,
                                                            const uint32_t* __restrict__ rank,
                                                            uint64_t* __restrict__ keys_out,
                                                            uint32_t* __restrict__ vals_out,
@@ -324,9 +320,12 @@ __global__ __launch_bounds__(256) void rank_scatter_kernel(const uint64_t* __res
                                                            float4* __restrict__ dst) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    keys_out[rank[i]] = keys[i];
-    vals_out[rank[i]] = vals[i];
-    if (dst) dst[rank[i]] = src[vals[i]];
+    uint32_t c = 0;
+#pragma unroll 4
+    for (uint32_t k = 0; k < parts; ++k) c += rank[size_t(k) * n + i];
+    keys_out[c] = keys[i];
+    vals_out[c] = vals[i];
+    if (dst) dst[c] = src[vals[i]];
 }
 
 __global__ __launch_bounds__(256) void rs_gather_kernel(const float4* __restrict__ src, size_t n,
@@ -362,16 +361,15 @@ int radix_sort_pairs(pnb_ctx* c, uint64_t* keys, uint32_t* vals, uint64_t* keys_
         const uint32_t g = div_up(nn, 256u), parts = div_up(nn, span);
         uint32_t* rank = nullptr;
         if (parts > 1) {
-            PNB_HIP(c, hist_buf.ensure(size_t(nn) * sizeof(uint32_t)));
+            PNB_HIP(c, hist_buf.ensure(size_t(parts) * nn * sizeof(uint32_t)));
             rank = hist_buf.as<uint32_t>();
-            rank_zero_kernel<<<g, 256, 0, c->stream>>>(rank, nn);
-            PNB_CHECK_LAUNCH(c);
         }
         rank_count_kernel<<<dim3(g, parts), 256, 0, c->stream>>>(keys, vals, nn, span, mask, rank,
                                                                 keys_alt, vals_alt, src, dst);
         PNB_CHECK_LAUNCH(c);
         if (parts > 1) {
-            rank_scatter_kernel<<<g, 256, 0, c->stream>>>(keys, vals, nn, rank, keys_alt, vals_alt, src, dst);
+            rank_scatter_kernel<<<g, 256, 0, c->stream>>>(keys, vals, nn, parts, rank, keys_alt,
+                                                             vals_alt, src, dst);
             PNB_CHECK_LAUNCH(c);
         }
         *keys_out = keys_alt;
