@@ -42,9 +42,10 @@ struct pnb_ctx {
     int cu_count = 0;
 
     // scratch for host-pointer entry points and the massive/massless split
-    pnb::DevBuf h_affected, h_affecting, h_out, split_tmp, split_flags, bf_partial;
+    pnb::DevBuf h_affected, h_affecting, h_out, split_tmp, split_counts, bf_partial;
     pnb::DevBuf scan_tmp;
     void *pin_in = nullptr, *pin_out = nullptr;  // pinned: stage_in's two slots, stage_out's one
+    uint32_t* pin_count = nullptr;               // pinned: split_affecting's count
     pnb::DevBuf pairs_part;  // pair brute force: one partial per body and super-tile
     // device address of the allocation-free entry point's static scratch on this device
     float4* noalloc_scratch = nullptr;
