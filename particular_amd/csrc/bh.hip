@@ -160,7 +160,7 @@ struct BhState {
     DevBuf c_starts, c_pts, c_bh, c_bf, c_list, c_count, c_target, c_wgt, c_rows, c_rwave,
         c_cfeats, c_cgeom, c_cmask, c_lanes;
     DevBuf feat_out;  // pnb_bh_node_features
-    BhInfo* host_info = nullptr;  // pinned: the ordinary build's read-back
+    BhInfo* host_info = nullptr;  // pinned: what the ordinary build's host side reads (level_offsets)
     float last_theta = 0.f;
     unsigned long long last_steps = 0, last_accepted = 0;
 };
@@ -580,12 +580,13 @@ __global__ __launch_bounds__(256) void bh_count_kernel(const int* __restrict__ l
 
 // The per-level counts (n_l of thread l) and the node count into info, and the list cursors set to
 // the counts' exclusive scan; called by the first 256 threads of a workgroup and, for the barrier,
-// by all others. cap > 0 (a capturable build): a tree that needs more nodes or levels than an
+// by all others. host (an ordinary build): pinned memory that gets what the host reads of info, after
+// the stream's synchronisation. cap > 0 (a capturable build): a tree that needs more nodes or levels than an
 // earlier ordinary build sized flags the build; every later kernel of it then returns at once and
 // the walk writes NaN.
 __device__ __forceinline__ void level_offsets(BhInfo* __restrict__ info, uint32_t n_l, uint32_t total,
                                               int max_level, uint32_t* __restrict__ lvl_cur, uint32_t cap,
-                                              int levels) {
+                                              int levels, BhInfo* __restrict__ host) {
     static_assert(LVL_SLOTS <= 256, "one thread per level");
     __shared__ uint32_t wsum[4];
     const int l = threadIdx.x, lane = l & 63, w = l >> 6;
@@ -603,8 +604,14 @@ __device__ __forceinline__ void level_offsets(BhInfo* __restrict__ info, uint32_
     info->lvl_count[l] = n_l;
     info->lvl_off[l] = off;
     lvl_cur[l * LVL_STRIDE] = off;
+    if (host) host->lvl_count[l] = n_l;
     if (l == 0) {
         info->total = total;
+        if (host) {
+            host->total = total;
+            host->max_level = max_level;
+            host->flags = __atomic_load_n(&info->flags, __ATOMIC_RELAXED);
+        }
         if (cap && (total > cap || max_level > levels)) atomicOr(&info->flags, FLAG_CAPACITY);
     }
 }
@@ -613,9 +620,10 @@ __global__ __launch_bounds__(256) void bh_level_offsets_kernel(BhInfo* __restric
                                                                const uint32_t* __restrict__ lvl_count,
                                                                uint32_t* __restrict__ lvl_cur,
                                                                const uint32_t* __restrict__ S,
-                                                               size_t m, uint32_t cap, int levels) {
+                                                               size_t m, uint32_t cap, int levels,
+                                                               BhInfo* __restrict__ host) {
     level_offsets(info, threadIdx.x < LVL_SLOTS ? lvl_count[threadIdx.x * LVL_STRIDE] : 0u, S[m],
-                  info->max_level, lvl_cur, cap, levels);
+                  info->max_level, lvl_cur, cap, levels, host);
 }
 
 // The counts, their scan and the level offsets for small sets in one workgroup, in place of three
@@ -629,7 +637,8 @@ __global__ __launch_bounds__(1024) void bh_small_count_kernel(const int* __restr
                                                               int* __restrict__ ip,
                                                               BhInfo* __restrict__ info,
                                                               uint32_t* __restrict__ lvl_cur,
-                                                              uint32_t cap, int levels) {
+                                                              uint32_t cap, int levels,
+                                                              BhInfo* __restrict__ host) {
     __shared__ uint32_t hist[256], wsum[2][16];
     __shared__ int wdeep[16];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -664,18 +673,18 @@ __global__ __launch_bounds__(1024) void bh_small_count_kernel(const int* __restr
         if (deepest > MAX_LEVEL) atomicOr(&info->flags, FLAG_DEPTH);
     }
     level_offsets(info, threadIdx.x < LVL_SLOTS ? hist[threadIdx.x] : 0u, carry, deepest, lvl_cur, cap,
-                  levels);
+                  levels, host);
 }
 
 // Counts, scan (S = cnt) and offsets. Info's max_level starts at -1 and the level counters at 0.
-static int count_levels(pnb_ctx* c, BhState* s, size_t m, uint32_t cap, int levels) {
+static int count_levels(pnb_ctx* c, BhState* s, size_t m, uint32_t cap, int levels, BhInfo* host) {
     BhInfo* info = s->info.as<BhInfo>();
     uint32_t* lvl_count = s->lvl.as<uint32_t>();
     uint32_t* lvl_cur = lvl_count + LVL_SLOTS * LVL_STRIDE;
     uint32_t* cnt = s->cnt.as<uint32_t>();
     if (m <= COUNT_SMALL) {
         bh_small_count_kernel<<<1, 1024, 0, c->stream>>>(s->lcp.as<int>(), uint32_t(m), cnt, s->ip.as<int>(),
-                                                         info, lvl_cur, cap, levels);
+                                                         info, lvl_cur, cap, levels, host);
         PNB_CHECK_LAUNCH(c);
         return PNB_OK;
     }
@@ -683,7 +692,8 @@ static int count_levels(pnb_ctx* c, BhState* s, size_t m, uint32_t cap, int leve
     bh_count_kernel<<<lg, 256, 0, c->stream>>>(s->lcp.as<int>(), m, cnt, s->ip.as<int>(), info, lvl_count);
     PNB_CHECK_LAUNCH(c);
     if (int rc = scan_u32(c, cnt, cnt, m, true)) return rc;
-    bh_level_offsets_kernel<<<1, 256, 0, c->stream>>>(info, lvl_count, lvl_cur, cnt, m, cap, levels);
+    bh_level_offsets_kernel<<<1, 256, 0, c->stream>>>(info, lvl_count, lvl_cur, cnt, m, cap, levels,
+                                                      host);
     PNB_CHECK_LAUNCH(c);
     return PNB_OK;
 }
@@ -1860,9 +1870,8 @@ static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = fa
                                                  s->key2.as<uint64_t>(), info);
         PNB_CHECK_LAUNCH(c);
         uint32_t* cnt = s->cnt.as<uint32_t>();
-        if ((rc = count_levels(c, s, m, 0, 0))) return rc;
         if (!s->host_info) PNB_HIP(c, hipHostMalloc(reinterpret_cast<void**>(&s->host_info), sizeof(BhInfo)));
-        PNB_HIP(c, hipMemcpyAsync(s->host_info, info, sizeof(BhInfo), hipMemcpyDeviceToHost, c->stream));
+        if ((rc = count_levels(c, s, m, 0, 0, s->host_info))) return rc;
         PNB_HIP(c, hipStreamSynchronize(c->stream));
         const BhInfo& h = *s->host_info;
         const uint32_t total = h.total;
@@ -2047,7 +2056,7 @@ static int build_tree_dd(pnb_ctx* c, const float4* afg, size_t m, bool moments, 
         bh_deep_kernel<<<g, 256, 0, c->stream>>>(sk, m, sp, si, lcp, s->key2.as<uint64_t>(), info);
         PNB_CHECK_LAUNCH(c);
         uint32_t* cnt = s->cnt.as<uint32_t>();
-        if ((rc = count_levels(c, s, m, uint32_t(s->dd_cap), s->dd_levels))) return rc;
+        if ((rc = count_levels(c, s, m, uint32_t(s->dd_cap), s->dd_levels, nullptr))) return rc;
         NodeRec* rec = s->rec.as<NodeRec>();
         uint32_t* skipv = s->skipv.as<uint32_t>();
         NodeMoments* mom = moments ? s->mom.as<NodeMoments>() : nullptr;

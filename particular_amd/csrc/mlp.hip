@@ -22,6 +22,7 @@
 #include "mlp_common.hpp"
 
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 namespace pnb {
@@ -530,12 +531,14 @@ __global__ __launch_bounds__(64 * MLP_BWD_WAVES) void mlp_bwd_kernel(
 // grads[k] = sum over the partials in a fixed order: 8 groups of 32 threads per workgroup, group
 // g summing its contiguous eighth of the partials for 32 parameters, then the eight group sums
 // added in group order.
-// One more workgroup sums the wavefronts' loss shares.
+// One more workgroup sums the wavefronts' loss shares. host: pinned memory for a copy of the gradients
+// and the loss behind them.
 constexpr int MLP_RED_PARAMS = 32;
 __global__ __launch_bounds__(256) void mlp_reduce_kernel(const float* __restrict__ partial,
                                                          int parts, float* __restrict__ grads,
                                                          const float* __restrict__ loss_part,
-                                                         size_t waves, float* __restrict__ loss) {
+                                                         size_t waves, float* __restrict__ loss,
+                                                         float* __restrict__ host) {
     __shared__ float acc[8][MLP_RED_PARAMS];
     const int g = threadIdx.x / MLP_RED_PARAMS, t = threadIdx.x % MLP_RED_PARAMS;
     if (blockIdx.x == gridDim.x - 1) {
@@ -549,6 +552,7 @@ __global__ __launch_bounds__(256) void mlp_reduce_kernel(const float* __restrict
             __syncthreads();
         }
         if (threadIdx.x == 0) *loss = red[0];
+        if (threadIdx.x == 0 && host) host[MLP_NPARAM] = red[0];
         return;
     }
     const int k = blockIdx.x * MLP_RED_PARAMS + t;
@@ -564,6 +568,7 @@ __global__ __launch_bounds__(256) void mlp_reduce_kernel(const float* __restrict
 #pragma unroll
         for (int q = 1; q < 8; ++q) total += acc[q][t];
         grads[k] = total;
+        if (host) host[k] = total;
     }
 }
 
@@ -681,7 +686,7 @@ int mlp_append(pnb_ctx* c, const float* feats, const float4* geom, const unsigne
     return PNB_OK;
 }
 
-static int step_grads(pnb_ctx* c, float* loss_dev) {
+static int step_grads(pnb_ctx* c, float* loss_dev, float* host = nullptr) {
     MlpState* s = c->mlp;
     if (s->waves == 0) return fail(c, PNB_E_STATE, "the training set is empty");
     PNB_HIP(c, s->y.ensure(std::max<size_t>(1, s->rows) * MLP_YS * 4));
@@ -753,7 +758,7 @@ static int step_grads(pnb_ctx* c, float* loss_dev) {
         PNB_CHECK_LAUNCH(c);
         mlp_reduce_kernel<<<div_up(MLP_NPARAM, MLP_RED_PARAMS) + 1, 256, 0, c->stream>>>(
             s->partial.as<float>(), blocks, s->grads.as<float>(), s->loss_part.as<float>(), s->waves,
-            loss_dev);
+            loss_dev, host);
         PNB_CHECK_LAUNCH(c);
         return PNB_OK;
     });
@@ -914,10 +919,14 @@ int pnb_mlp_grad(pnb_ctx* c, float* loss, float* grads, size_t n) {
     if (int rc = activate(c)) return rc;
     MlpState* s = c->mlp;
     PNB_HIP(c, s->loss_hist.ensure(16));
-    if (int rc = step_grads(c, s->loss_hist.as<float>())) return rc;
-    if (loss) PNB_HIP(c, hipMemcpyAsync(loss, s->loss_hist.ptr, 4, hipMemcpyDeviceToHost, c->stream));
-    if (grads) PNB_HIP(c, hipMemcpyAsync(grads, s->grads.ptr, n * 4, hipMemcpyDeviceToHost, c->stream));
+    static_assert((MLP_NPARAM + 1) * sizeof(float) <= HOST_STAGE, "fits the staging memory");
+    void* pin;
+    if (int rc = stage_out(c, c->h_out, (MLP_NPARAM + 1) * sizeof(float), &pin)) return rc;
+    float* host = static_cast<float*>(pin);
+    if (int rc = step_grads(c, s->loss_hist.as<float>(), host)) return rc;
     PNB_HIP(c, hipStreamSynchronize(c->stream));
+    if (loss) *loss = host[MLP_NPARAM];
+    if (grads) std::memcpy(grads, host, n * sizeof(float));
     return PNB_OK;
 }
 
