@@ -438,11 +438,7 @@ int pnb_batch_read(pnb_ctx* c, double* pos3, double* vel3, float* acc4) {
     double* st = s->stage.as<double>();
     bt_unpack_kernel<<<div_up(n, 256), 256, 0, c->stream>>>(s->x.as<double4>(), s->v.as<double4>(), n, st);
     PNB_CHECK_LAUNCH(c);
-    if (pos3) PNB_HIP(c, hipMemcpyAsync(pos3, st, 3 * n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    if (vel3) PNB_HIP(c, hipMemcpyAsync(vel3, st + 3 * n, 3 * n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    if (acc4) PNB_HIP(c, hipMemcpyAsync(acc4, s->acc.ptr, n * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
-    PNB_HIP(c, hipStreamSynchronize(c->stream));
-    return PNB_OK;
+    return stage_fetch(c, {{pos3, st, 24 * n}, {vel3, st + 3 * n, 24 * n}, {acc4, s->acc.ptr, 16 * n}});
 }
 
 int pnb_batch_info(pnb_ctx* c, size_t* particles, size_t* items,

@@ -2522,13 +2522,6 @@ static int accel_dev(pnb_ctx* c, const float4* affected, size_t n, const float4*
     return walk(c, s->apts.as<float4>(), si, n, theta, softening, out, nullptr, quad, rel, dd, list);
 }
 
-static int copy_h2d(pnb_ctx* c, DevBuf& b, const float* src, size_t count) {
-    PNB_HIP(c, b.ensure(std::max<size_t>(count, 1) * sizeof(float4)));
-    if (count)
-        PNB_HIP(c, hipMemcpyAsync(b.ptr, src, count * sizeof(float4), hipMemcpyHostToDevice, c->stream));
-    return PNB_OK;
-}
-
 // ---- training data for the learned correction -------------------------------------------------
 
 __global__ void mlp_gather_waves_kernel(const float4* __restrict__ sp, const uint32_t* __restrict__ starts,
@@ -2698,17 +2691,15 @@ int pnb_bh_accel_f32(pnb_ctx* c, const float* affected, size_t n, const float* a
     if (!c->bh) c->bh = new BhState();
     BhState* s = c->bh;
     const bool same = affected == affecting && n == m;
-    if (int rc = copy_h2d(c, s->h_afg, affecting, m)) return rc;
+    if (int rc = stage_in(c, s->h_afg, affecting, m * sizeof(float4))) return rc;
     if (!same)
-        if (int rc = copy_h2d(c, s->h_aff, affected, n)) return rc;
+        if (int rc = stage_in(c, s->h_aff, affected, n * sizeof(float4), 1)) return rc;
     PNB_HIP(c, s->h_out.ensure(n * sizeof(float4)));
     const float* daff = same ? s->h_afg.as<float>() : s->h_aff.as<float>();
     if (int rc = pnb_bh_accel_f32_dev(c, daff, n, s->h_afg.as<float>(), m, theta, softening,
                                       checked, flags, s->h_out.as<float>()))
         return rc;
-    PNB_HIP(c, hipMemcpyAsync(out, s->h_out.ptr, n * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
-    PNB_HIP(c, hipStreamSynchronize(c->stream));
-    return PNB_OK;
+    return stage_fetch(c, {{out, s->h_out.ptr, n * sizeof(float4)}});
 }
 
 int pnb_reordered_bh_accel_f32_dev(pnb_ctx* c, const float* particles, size_t n, float theta,
@@ -2744,14 +2735,12 @@ int pnb_reordered_bh_accel_f32(pnb_ctx* c, const float* particles, size_t n, flo
     if (int rc = activate(c)) return rc;
     if (!c->bh) c->bh = new BhState();
     BhState* s = c->bh;
-    if (int rc = copy_h2d(c, s->h_aff, particles, n)) return rc;
+    if (int rc = stage_in(c, s->h_aff, particles, n * sizeof(float4))) return rc;
     PNB_HIP(c, s->h_out.ensure(n * sizeof(float4)));
     if (int rc = pnb_reordered_bh_accel_f32_dev(c, s->h_aff.as<float>(), n, theta, softening,
                                                 checked, flags, s->h_out.as<float>()))
         return rc;
-    PNB_HIP(c, hipMemcpyAsync(out, s->h_out.ptr, n * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
-    PNB_HIP(c, hipStreamSynchronize(c->stream));
-    return PNB_OK;
+    return stage_fetch(c, {{out, s->h_out.ptr, n * sizeof(float4)}});
 }
 
 int pnb_bh_set_relative(pnb_ctx* c, float alpha, float estimate_theta, int per_particle,

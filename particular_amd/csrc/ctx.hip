@@ -60,8 +60,9 @@ int prof_resolve(pnb_ctx* c) {
     return PNB_OK;
 }
 
-__global__ __launch_bounds__(256) void stage_kernel(const uint4* __restrict__ src, size_t n,
-                                                    uint4* __restrict__ dst) {
+template <class T>
+__global__ __launch_bounds__(256) void stage_kernel(const T* __restrict__ src, size_t n,
+                                                    T* __restrict__ dst) {
     const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < n) dst[i] = src[i];
 }
@@ -94,11 +95,37 @@ int stage_out(pnb_ctx* c, DevBuf& dev, size_t bytes, void** where) {
 }
 
 int stage_done(pnb_ctx* c, void* out, const void* where, size_t bytes) {
-    const bool pinned = where == c->pin_out;
-    if (!pinned && bytes)
-        PNB_HIP(c, hipMemcpyAsync(out, where, bytes, hipMemcpyDeviceToHost, c->stream));
+    if (where != c->pin_out) return stage_fetch(c, {{out, where, bytes}});
     PNB_HIP(c, hipStreamSynchronize(c->stream));
-    if (pinned) std::memcpy(out, where, bytes);
+    std::memcpy(out, where, bytes);
+    return PNB_OK;
+}
+
+int stage_fetch(pnb_ctx* c, std::initializer_list<Fetch> parts) {
+    size_t total = 0;
+    for (const Fetch& f : parts) total += f.dst ? f.bytes : 0;
+    const bool pinned = total > 0 && total <= HOST_STAGE;
+    if (pinned && !c->pin_out) PNB_HIP(c, hipHostMalloc(&c->pin_out, HOST_STAGE));
+    char* pin = static_cast<char*>(c->pin_out);
+    for (const Fetch& f : parts) {
+        if (!f.dst || f.bytes == 0) continue;
+        if (!pinned) {
+            PNB_HIP(c, hipMemcpyAsync(f.dst, f.src, f.bytes, hipMemcpyDeviceToHost, c->stream));
+            continue;
+        }
+        stage_kernel<<<div_up(f.bytes / 8, 256), 256, 0, c->stream>>>(
+            static_cast<const uint2*>(f.src), f.bytes / 8, reinterpret_cast<uint2*>(pin));
+        PNB_CHECK_LAUNCH(c);
+        pin += f.bytes;
+    }
+    PNB_HIP(c, hipStreamSynchronize(c->stream));
+    if (!pinned) return PNB_OK;
+    pin = static_cast<char*>(c->pin_out);
+    for (const Fetch& f : parts) {
+        if (!f.dst) continue;
+        std::memcpy(f.dst, pin, f.bytes);
+        pin += f.bytes;
+    }
     return PNB_OK;
 }
 

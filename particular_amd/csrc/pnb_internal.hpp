@@ -5,6 +5,7 @@
 
 #include <cstdarg>
 #include <cstddef>
+#include <initializer_list>
 #include <cstdint>
 #include <cstdio>
 #include <string>
@@ -97,6 +98,14 @@ constexpr size_t HOST_STAGE = size_t(1) << 20;
 int stage_in(pnb_ctx* c, DevBuf& dst, const void* src, size_t bytes, int slot = 0);
 int stage_out(pnb_ctx* c, DevBuf& dev, size_t bytes, void** where);
 int stage_done(pnb_ctx* c, void* out, const void* where, size_t bytes);
+// Device results (multiples of 8 bytes) to host arrays (null ones are left out), up to HOST_STAGE bytes together by a kernel
+// into the pinned memory, and waits for them.
+struct Fetch {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+int stage_fetch(pnb_ctx* c, std::initializer_list<Fetch> parts);
 
 // Brute force on device pointers, asynchronous on c->stream.
 int bf_launch(pnb_ctx* c, const float4* affected, size_t n, const float4* affecting, size_t m,

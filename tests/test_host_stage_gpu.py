@@ -56,3 +56,39 @@ def test_pairs_host_sums_are_the_device_sums(res, n):
     alg = pa.BruteForcePairs(res, pa.AccelerationSoftened.checked(1e-2))
     np.testing.assert_array_equal(alg.compute(a),
                                   alg.compute(torch.from_numpy(a).cuda()).cpu().numpy()[:, :3])
+
+
+@pytest.mark.parametrize("n", [1, 3, 16383, 16384, 16385])
+def test_step_states_read_back(res, n):
+    """The leapfrog state read whole and array by array, around 1 MiB of results (16,384 bodies)."""
+    p = bodies(n, 6, np.float64)
+    mu = np.zeros(n, np.float32)
+    mu[:5] = 1.0
+    pos, vel = np.ascontiguousarray(p[:, :3]), np.ascontiguousarray(p[:, 1:])
+    lib = _lib.lib()
+    res.check(lib.pnb_leapfrog_init(res.handle, pos.ctypes.data, vel.ctypes.data, mu.ctypes.data, n, 1e-2, 1))
+    x, v, a = np.empty((n, 3)), np.empty((n, 3)), np.empty((n, 4), np.float32)
+    res.check(lib.pnb_leapfrog_read(res.handle, x.ctypes.data, v.ctypes.data, a.ctypes.data))
+    np.testing.assert_array_equal(x, pos)
+    np.testing.assert_array_equal(v, vel)
+    f32 = np.concatenate([pos.astype(np.float32), mu[:, None]], 1)
+    np.testing.assert_array_equal(
+        a[:, :3], pa.BruteForce(res, pa.AccelerationSoftened.checked(1e-2)).compute(pa.Reordered.new(f32)))
+    for k, whole in enumerate((x, v, a)):
+        part = np.empty_like(whole)
+        args = [None, None, None]
+        args[k] = part.ctypes.data
+        res.check(lib.pnb_leapfrog_read(res.handle, *args))
+        np.testing.assert_array_equal(part, whole)
+
+
+@pytest.mark.parametrize("n,m", [(5, 3), (4097, 4097), (65537, 1000), (1000, 65537)])
+def test_barnes_hut_host_sums_are_the_device_sums(res, n, m):
+    import torch
+
+    a = bodies(n, 7, np.float32)
+    b = a if n == m else bodies(m, 8, np.float32)
+    alg = pa.BarnesHut(res, 0.6, pa.AccelerationSoftened.checked(1e-2))
+    da = torch.from_numpy(a).cuda()
+    dev = alg.compute(pa.Between(da, da if n == m else torch.from_numpy(b).cuda()))
+    np.testing.assert_array_equal(alg.compute(pa.Between(a, b)), dev.cpu().numpy()[:, :3])
