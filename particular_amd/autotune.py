@@ -3,7 +3,8 @@
 For every size bucket it times each candidate shape with the library's own event profiling (device
 time of the force kernel, median of a few launches) and keeps the fastest:
   * brute force: (variant, affected per lane, affecting splits) per affected-count bucket, at a
-    fixed affecting count;
+    fixed affecting count; the first buckets where no shape beats the library's own choice (which
+    has a kernel for small sums that no shape names) get no entry;
   * batched ensemble: affected per lane per system-size bucket, on uniform ensembles.
 The table is written as JSON and applied with :func:`apply`. Run on the target GPU:
 ``python -m particular_amd.autotune --out particular_amd/tuning/mi355x.json``.
@@ -59,11 +60,12 @@ def tune_bf(res, reps=3):
     allp = torch.from_numpy(src.particles.copy()).cuda()
     for n in BF_BUCKETS:
         best = None
+        own = _time_bf(res, allp.data_ptr(), n, massive.data_ptr(), BF_M, reps)
         for variant in (0, 1):
             for per_lane in (1, 2, 4, 8):
                 blocks = -(-n // (256 * per_lane))
                 for j_split in (1, 2, 4, 8, 16, 32, 64):
-                    if j_split > 1 and blocks * j_split > 64 * cus:
+                    if j_split > 1 and blocks * j_split > 256 * cus:
                         continue
                     if BF_M // j_split < 1024:
                         continue
@@ -72,7 +74,11 @@ def tune_bf(res, reps=3):
                     if best is None or t < best[0]:
                         best = (t, variant, per_lane, j_split)
         res.clear_bf_tuning()
+        own = min(own, _time_bf(res, allp.data_ptr(), n, massive.data_ptr(), BF_M, reps))
         t, variant, per_lane, j_split = best
+        if not table and t > 0.97 * own:
+            _log(f"bf n={n}: the default, {own:.3f} ms (best shape {t:.3f})")
+            continue
         rate = n * BF_M / (t * 1e-3) / 1e9
         _log(f"bf n={n}: variant={variant} per_lane={per_lane} j_split={j_split} "
              f"{t:.3f} ms ({rate:.0f} G interactions/s)")
