@@ -40,6 +40,42 @@ __device__ __forceinline__ void bf_body(const float4 q, const float (&xi)[R], co
     }
 }
 
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+// T affecting bodies at a wave-uniform address, four per scalar load, the next four requested before
+// the present four are summed: one by one, each body is five scalar instructions, a load and a wait.
+// For sums of few wavefronts (4,096 x 60,000 91 -> 82 us, 4,096 x 4,096 10.8 -> 10.1); where a SIMD
+// holds eight the waits cost nothing and this form is slower (1,048,576 x 65,536 18.7 -> 19.0 ms
+// on one card), as it is for the ensemble's items (64 systems, ten steps 0.93 -> 1.05 ms).
+template <int T, int R, bool MASK, bool SELF, bool SEQ>
+__device__ __forceinline__ void bf_tile(const float4* __restrict__ q, const float (&xi)[R],
+                                        const float (&yi)[R], const float (&zi)[R], float eps2,
+                                        float (&px)[R], float (&py)[R], float (&pz)[R],
+                                        uint32_t j0 = 0, uint32_t self = 0) {
+    const f32x16_t* g = reinterpret_cast<const f32x16_t*>(q);
+    f32x16_t a = g[0];
+    const auto four = [&](const f32x16_t& v, uint32_t j) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            bf_body<R, MASK, SELF, SEQ>(make_float4(v[4 * u], v[4 * u + 1], v[4 * u + 2], v[4 * u + 3]), xi,
+                                        yi, zi, eps2, px, py, pz, j + u, self);
+    };
+    // (the empty asm statements wait for a group where it is first needed, before the next is asked for)
+#pragma unroll 1
+    for (int j = 0; j < T; j += 8) {
+        asm volatile("" ::"s"(a));
+        __builtin_amdgcn_sched_barrier(0);
+        const f32x16_t b = g[j / 4 + 1];
+        __builtin_amdgcn_sched_barrier(0);
+        four(a, j0 + j);
+        asm volatile("" ::"s"(b));
+        __builtin_amdgcn_sched_barrier(0);
+        a = g[j + 8 < T ? j / 4 + 2 : 0];
+        __builtin_amdgcn_sched_barrier(0);
+        four(b, j0 + j + 4);
+    }
+}
+
 __device__ __forceinline__ void kahan_add(float& sum, float& comp, float v) {
     const float y = v - comp;
     const float t = sum + y;
@@ -69,7 +105,7 @@ struct CoopLds {
 // so a tile of affected bodies walked by one wavefront takes m x R x 13 x 4.8 cycles (1.7 ms for
 // 16,384 affecting bodies and R = 4); J wavefronts divide that by J without another pass over
 // memory.
-template <int R, bool MASK, bool SELF, int T, int W, bool SEQ = true>
+template <int R, bool MASK, bool SELF, int T, int W, bool SEQ = true, bool GROUPS = false>
 __device__ __forceinline__ void coop_sum(CoopLds<R, W>& lds, const float4* __restrict__ afg,
                                          uint32_t jb, uint32_t je, int J, int wave, bool live,
                                          float eps2, uint32_t self, const float (&xi)[R],
@@ -93,7 +129,9 @@ __device__ __forceinline__ void coop_sum(CoopLds<R, W>& lds, const float4* __res
         if (live && j0 < je) {
             const float4* q = afg + j0;
             const uint32_t cnt = min(uint32_t(T), je - j0);
-            if (cnt == uint32_t(T)) {
+            if (GROUPS && cnt == uint32_t(T)) {
+                bf_tile<T, R, MASK, SELF, SEQ>(q, xi, yi, zi, eps2, px, py, pz, j0, self);
+            } else if (cnt == uint32_t(T)) {
 #pragma unroll 8
                 for (int j = 0; j < T; ++j)
                     bf_body<R, MASK, SELF, SEQ>(q[j], xi, yi, zi, eps2, px, py, pz, j0 + j, self);
