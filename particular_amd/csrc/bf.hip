@@ -182,44 +182,49 @@ struct BfShape {
     int variant, per_lane, j_split;
 };
 
-// What the cooperative kernel takes: sums small enough that wavefronts walking the affecting
-// bodies alone are bound by their own issue rate (a 1,024-body range takes one 34 us), and sums
-// with few bodies on one side, which leave the others too few ranges or tiles. Measured, the best
-// split of the plain kernel / cooperative, softened: 1,000 x 1,000 34 / 8 us; 4,096 x 4,096 36 / 11;
-// 1,000 x 65,536 91 / 28; 4,096 x 65,536 102 / 96; 8,192 x 8,192 28 / 27 (6.7e7 pairs); 12,000 x
-// 16,384 67 / 92; 32,768 x 4,096 45 / 42; 300,000 x 5,000 385 / 430; 65,536 x 1,000 78 / 21;
-// 1,000,000 x 1,000 291 / 273; 256 x 100 6.0 / 8.8, 256 x 128 6.9 / 7.6, 256 x 200 9.8 / 8.7 (two
-// tiles: little to share).
+// What the cooperative kernel takes: sums too small for one wavefront per affected tile and range to
+// fill the chip evenly. Measured, plain kernel with its best split / cooperative (us, softened): 1,000
+// x 1,000 62 / 8; 4,096 x 4,096 36 / 10; 10,000 x 8,000 45 / 30; 20,000 x 20,000 142 / 122; 30,000 x
+// 65,536 628 / 568; 45,000 x 130,000 1,695 / 1,659, without softening 1,861 / 1,862; 65,536 x 16,384
+// 321 / 308; 90,000 x 30,000 781 / 775, 864 / 868; 130,000 x 4,000 163 / 160; 130,000 x 30,000 1,098 /
+// 1,116; 400,000 x 500 75 / 67, x 2,047 305 / 247 (the plain kernel does not split below 2,048). With
+// few affecting bodies there is little to share: 256 x 100 6.0 / 8.8, 256 x 128 6.9 / 7.6, 256 x 200
+// 9.8 / 8.7; 65,536 x 200 10.0 / 9.7, 90,000 x 200 11 / 13.
 static bool coop_pays(size_t n, size_t m) {
-    if (m <= 128 || (m <= 256 && n > 32768)) return false;
-    const double pairs = double(n) * double(m);
-    return pairs <= (m < 2048 ? 1e9 : n <= 4096 ? 3e8 : m <= 4096 ? 1.5e8 : 7e7);
+    if (m <= 256) return m > 128 && n <= 65536;
+    if (m < 2048) return true;
+    return n <= 50000 || (n <= 100000 && m <= 16384) || (n <= 150000 && m <= 4096);
 }
 
 static BfShape default_shape(pnb_ctx* c, size_t n, size_t m) {
     const size_t cus = c->cu_count > 0 ? size_t(c->cu_count) : 256;
     int s = 1;
     if (coop_pays(n, m)) {
-        // workgroups of 16 wavefronts over the affecting range until every CU has one, keeping a
-        // tile of 64 bodies for each wavefront
+        // Workgroups of 16 wavefronts over ranges of the affecting bodies: two per CU while a range
+        // keeps 500 of them, which is half a tile for each wavefront, and up to 16 per CU, so that
+        // no CU has twice another's work, while it keeps 700. 9,000 x 9,000 in 1 / 2 / 4 / 8 / 16
+        // ranges 50 / 54 / 40 / 32 / 32 us; 6,000 x 6,000 33 / 22 / 21 / 16 / 20; 1,000 x 8,000 41 /
+        // 25 / 16 / 10 / 8; 20,000 x 20,000 186 / 145 / 126 / 122 / 124.
         const size_t blocks = div_up(n, 64);
-        while (s < 64 && blocks * s * 2 <= cus && m / (size_t(s) * 2) >= size_t(COOP_WAVES) * 64) s <<= 1;
+        while (m >= 2048 && s < 64) {
+            const size_t wgs = blocks * s * 2, per = m / (size_t(s) * 2);
+            if (!((wgs <= 2 * cus && per >= 500) || (wgs <= 16 * cus && per >= 700))) break;
+            s <<= 1;
+        }
         return {BF_COOP, 1, s};
     }
     // Otherwise one body per lane and one wavefront per affected tile and range, the affecting
-    // bodies from scalar loads (from LDS below 32,768 affected bodies, where few wavefronts hide
-    // their latency, 12,000 x 16,384 67 / 70 us, and for at most a tile, 65,536 x 64 4 / 9 us), the
-    // affecting range from 2,048 bodies on split into up to 64 workgroups per CU of at least one
-    // tile each, up to 256 per CU while ranges stay at 1,024 bodies (small workgroups balance the
-    // load across CUs and XCDs; what is left below 2,048 has enough of them unsplit). 1,048,576 x 65,536 16.1 ms, with four
-    // bodies per lane 17.1; 65,536 x 16,384 286 us, 333.
+    // bodies from scalar loads (from LDS for at most a tile, 65,536 x 64 4 / 9 us), the affecting
+    // range from 2,048 bodies on split into up to 64 workgroups per CU of at least one tile each, up
+    // to 256 per CU while ranges stay at 1,024 bodies (small workgroups balance the load across CUs
+    // and XCDs). 1,048,576 x 65,536 16.1 ms, with four bodies per lane 17.1.
     const size_t blocks = div_up(n, size_t(BF_BLOCK));
     while (m >= 2048 && s < 64 && blocks * s * 2 <= 256 * cus) {
         const size_t per = m / (size_t(s) * 2);
         if (per < (blocks * s * 2 <= 64 * cus ? size_t(BF_TILE) : size_t(1024))) break;
         s <<= 1;
     }
-    return {n < 32768 || m <= 256 ? 0 : 1, 1, s};
+    return {m <= 256 ? 0 : 1, 1, s};
 }
 
 static BfShape choose_shape(pnb_ctx* c, size_t n, size_t m) {

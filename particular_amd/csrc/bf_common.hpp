@@ -47,18 +47,17 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 // For sums of few wavefronts (4,096 x 60,000 91 -> 82 us, 4,096 x 4,096 10.8 -> 10.1); where a SIMD
 // holds eight the waits cost nothing and this form is slower (1,048,576 x 65,536 18.7 -> 19.0 ms
 // on one card), as it is for the ensemble's items (64 systems, ten steps 0.93 -> 1.05 ms).
-template <int T, int R, bool MASK, bool SELF, bool SEQ>
+template <int T, int R, bool MASK, bool SEQ>
 __device__ __forceinline__ void bf_tile(const float4* __restrict__ q, const float (&xi)[R],
                                         const float (&yi)[R], const float (&zi)[R], float eps2,
-                                        float (&px)[R], float (&py)[R], float (&pz)[R],
-                                        uint32_t j0 = 0, uint32_t self = 0) {
+                                        float (&px)[R], float (&py)[R], float (&pz)[R]) {
     const f32x16_t* g = reinterpret_cast<const f32x16_t*>(q);
     f32x16_t a = g[0];
-    const auto four = [&](const f32x16_t& v, uint32_t j) {
+    const auto four = [&](const f32x16_t& v) {
 #pragma unroll
         for (int u = 0; u < 4; ++u)
-            bf_body<R, MASK, SELF, SEQ>(make_float4(v[4 * u], v[4 * u + 1], v[4 * u + 2], v[4 * u + 3]), xi,
-                                        yi, zi, eps2, px, py, pz, j + u, self);
+            bf_body<R, MASK, false, SEQ>(make_float4(v[4 * u], v[4 * u + 1], v[4 * u + 2], v[4 * u + 3]),
+                                         xi, yi, zi, eps2, px, py, pz);
     };
     // (the empty asm statements wait for a group where it is first needed, before the next is asked for)
 #pragma unroll 1
@@ -67,12 +66,39 @@ __device__ __forceinline__ void bf_tile(const float4* __restrict__ q, const floa
         __builtin_amdgcn_sched_barrier(0);
         const f32x16_t b = g[j / 4 + 1];
         __builtin_amdgcn_sched_barrier(0);
-        four(a, j0 + j);
+        four(a);
         asm volatile("" ::"s"(b));
         __builtin_amdgcn_sched_barrier(0);
         a = g[j + 8 < T ? j / 4 + 2 : 0];
         __builtin_amdgcn_sched_barrier(0);
-        four(b, j0 + j + 4);
+        four(b);
+    }
+}
+
+// Any number of affecting bodies at a wave-uniform address: eight at a time, then the rest requested
+// together (one by one each waits for its load: a step of 2,000 x 250 bodies 13.4 us so, 11.6 now).
+template <int R, bool MASK, bool SELF, bool SEQ>
+__device__ __forceinline__ void bf_span(const float4* __restrict__ q, uint32_t cnt, const float (&xi)[R],
+                                        const float (&yi)[R], const float (&zi)[R], float eps2,
+                                        float (&px)[R], float (&py)[R], float (&pz)[R],
+                                        uint32_t j0 = 0, uint32_t self = 0) {
+    uint32_t j = 0;
+    for (; j + 8 <= cnt; j += 8) {
+        float4 b[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u) b[u] = q[j + u];
+        if (SEQ) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u)
+            bf_body<R, MASK, SELF, SEQ>(b[u], xi, yi, zi, eps2, px, py, pz, j0 + j + u, self);
+    }
+    if (j < cnt) {
+        float4 b[7];
+#pragma unroll
+        for (uint32_t u = 0; u < 7; ++u) b[u] = q[min(j + u, cnt - 1)];
+#pragma unroll
+        for (uint32_t u = 0; u < 7; ++u)
+            if (j + u < cnt) bf_body<R, MASK, SELF, SEQ>(b[u], xi, yi, zi, eps2, px, py, pz, j0 + j + u, self);
     }
 }
 
@@ -113,6 +139,7 @@ __device__ __forceinline__ void coop_sum(CoopLds<R, W>& lds, const float4* __res
                                          float (&ax)[R], float (&ay)[R], float (&az)[R]) {
     const int lane = threadIdx.x & 63;
     const int slot = wave & (J - 1), g0 = wave - slot, g = g0 / J;
+    const uint32_t own = SELF ? uint32_t(__builtin_amdgcn_readfirstlane(int(self))) : 0u;
     float cx[R], cy[R], cz[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) ax[r] = ay[r] = az[r] = cx[r] = cy[r] = cz[r] = 0.0f;
@@ -129,30 +156,15 @@ __device__ __forceinline__ void coop_sum(CoopLds<R, W>& lds, const float4* __res
         if (live && j0 < je) {
             const float4* q = afg + j0;
             const uint32_t cnt = min(uint32_t(T), je - j0);
-            if (GROUPS && cnt == uint32_t(T)) {
-                bf_tile<T, R, MASK, SELF, SEQ>(q, xi, yi, zi, eps2, px, py, pz, j0, self);
+            if (SELF && j0 < own + 64 * R && own < j0 + cnt) {  // only here can a pair be a body with itself
+                bf_span<R, MASK, true, SEQ>(q, cnt, xi, yi, zi, eps2, px, py, pz, j0, self);
+            } else if (GROUPS && cnt == uint32_t(T)) {
+                bf_tile<T, R, MASK, SEQ>(q, xi, yi, zi, eps2, px, py, pz);
             } else if (cnt == uint32_t(T)) {
 #pragma unroll 8
-                for (int j = 0; j < T; ++j)
-                    bf_body<R, MASK, SELF, SEQ>(q[j], xi, yi, zi, eps2, px, py, pz, j0 + j, self);
+                for (int j = 0; j < T; ++j) bf_body<R, MASK, false, SEQ>(q[j], xi, yi, zi, eps2, px, py, pz);
             } else {
-                // eight at a time, then the rest requested together (one by one each waits for
-                // its load: a step of 2,000 x 250 bodies 13.4 us so, 11.6 now)
-                uint32_t j = 0;
-                for (; j + 8 <= cnt; j += 8) {
-#pragma unroll
-                    for (uint32_t u = 0; u < 8; ++u)
-                        bf_body<R, MASK, SELF, SEQ>(q[j + u], xi, yi, zi, eps2, px, py, pz, j0 + j + u, self);
-                }
-                if (j < cnt) {
-                    float4 b[7];
-#pragma unroll
-                    for (uint32_t u = 0; u < 7; ++u) b[u] = q[min(j + u, cnt - 1)];
-#pragma unroll
-                    for (uint32_t u = 0; u < 7; ++u)
-                        if (j + u < cnt)
-                            bf_body<R, MASK, SELF, SEQ>(b[u], xi, yi, zi, eps2, px, py, pz, j0 + j + u, self);
-                }
+                bf_span<R, MASK, false, SEQ>(q, cnt, xi, yi, zi, eps2, px, py, pz);
             }
         }
         if (J == 1) {
