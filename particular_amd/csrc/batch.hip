@@ -3,11 +3,11 @@
 // Every system is its own Between(system, system) brute force (all bodies massive within a
 // system), integrated with kick-drift-kick leapfrog in FP64 like the single-system loop. The force
 // pass of a step is ONE persistent launch: a few workgroups per CU that pull work items (system,
-// tiles of 64*R affected bodies) from a queue until it is empty, the wavefronts of a workgroup
+// tiles of 64 affected bodies) from a queue until it is empty, the wavefronts of a workgroup
 // sharing an item's affecting bodies (coop_sum), which they read with wave-uniform addresses
 // (scalar loads). Items are ordered by decreasing cost (system size x bodies per lane), so large
-// systems start first and small ones fill the tail. Tuning entries that ask for more than two
-// bodies per lane take the queue by single wavefronts, which need no barriers. The per-lane
+// systems start first and small ones fill the tail. Tuning entries that ask for more than one
+// body per lane take the queue by single wavefronts, which need no barriers. The per-lane
 // arithmetic and summation order are those of the brute-force kernel either way (FP32 tiles of 256
 // bodies, Kahan across tiles). A step is enqueue-only and can be captured into a hipGraph (the queue
 // counter is cleared by a kernel, not a memset).
@@ -20,7 +20,6 @@
 namespace pnb {
 
 constexpr int BT_TILE = 256;
-constexpr int BT_R_MAX = 2;  // bodies per lane of the workgroup form
 
 struct BatchItem {
     uint32_t off;  // first particle of the system
@@ -36,7 +35,7 @@ struct BatchState {
     std::vector<int64_t> offsets;
     std::vector<std::pair<size_t, int>> tuning;  // (n_min, per_lane)
     bool items_dirty = true;
-    bool coop = false;  // items for workgroups (bt_coop_kernel), else for wavefronts
+    int waves = 0;  // wavefronts of a workgroup that shares an item (bt_coop_kernel); 0: items for wavefronts
     size_t n_items = 0;
     unsigned long long interactions = 0;
     DevBuf x, v, shadow, acc, items, queue, stage;
@@ -118,55 +117,27 @@ __global__ __launch_bounds__(256) void bt_force_kernel(const BatchItem* __restri
     }
 }
 
-// The same queue taken by workgroups: BT_WAVES wavefronts share an item, J of them its affecting
-// bodies (coop_sum; the same tiles summed in the same order, so the same bits) and, in systems with
-// fewer than BT_WAVES tiles of affecting bodies, the others neighbouring affected tiles: an item
-// covers BT_WAVES / J tiles of 64 R bodies.
-constexpr int BT_WAVES = 8;
-
+// The same queue taken by workgroups, one body per lane: W wavefronts share an item, J of them its
+// affecting bodies (coop_sum; the same tiles summed in the same order, so the same bits) and, in
+// systems with fewer than W tiles of affecting bodies, the others neighbouring affected tiles: an item
+// covers W / J tiles of 64 bodies.
+template <int W>
 static __host__ __device__ inline int bt_share(uint32_t n) {  // wavefronts per affected tile
     int j = 1;
-    while (j < BT_WAVES && uint32_t(j) * BT_TILE < n) j <<= 1;
+    while (j < W && uint32_t(j) * BT_TILE < n) j <<= 1;
     return j;
 }
 
-template <int R, bool MASK, bool SEQ>
-__device__ __forceinline__ void bt_coop_tile(CoopLds<BT_R_MAX, BT_WAVES>& lds_max,
-                                             const float4* __restrict__ sh, const BatchItem w,
-                                             int wave, float eps2, float4* __restrict__ acc) {
-    // smaller R use a prefix of the same memory
-    CoopLds<R, BT_WAVES>& lds = reinterpret_cast<CoopLds<R, BT_WAVES>&>(lds_max);
-    const uint32_t lane = threadIdx.x & 63;
-    const float4* sys = sh + w.off;
-    const int J = bt_share(w.n);
-    const uint32_t i0 = w.i0 + uint32_t(wave / J) * (64 * R);
-    float xi[R], yi[R], zi[R], ax[R], ay[R], az[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const uint32_t i = i0 + r * 64 + lane;
-        const float4 p = sys[i < w.n ? i : w.n - 1];
-        xi[r] = p.x; yi[r] = p.y; zi[r] = p.z;
-    }
-    coop_sum<R, MASK, false, BT_TILE, BT_WAVES, SEQ>(lds, sys, 0, w.n, J, wave, i0 < w.n, eps2, 0, xi, yi,
-                                                zi, ax, ay, az);
-    if (wave % J != 0) return;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const uint32_t i = i0 + r * 64 + lane;
-        if (i < w.n) acc[w.off + i] = make_float4(ax[r], ay[r], az[r], 0.f);
-    }
-}
-
-template <bool MASK, bool SEQ>
-__global__ __launch_bounds__(64 * BT_WAVES) void bt_coop_kernel(const BatchItem* __restrict__ items,
-                                                                uint32_t n_items,
-                                                                uint32_t* __restrict__ queue,
-                                                                const float4* __restrict__ sh,
-                                                                float eps2,
-                                                                float4* __restrict__ acc) {
-    __shared__ CoopLds<BT_R_MAX, BT_WAVES> lds;
+template <int W, bool MASK>
+__global__ __launch_bounds__(64 * W) void bt_coop_kernel(const BatchItem* __restrict__ items,
+                                                         uint32_t n_items,
+                                                         uint32_t* __restrict__ queue,
+                                                         const float4* __restrict__ sh, float eps2,
+                                                         float4* __restrict__ acc) {
+    __shared__ CoopLds<1, W> lds;
     __shared__ uint32_t next;
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+    asm volatile("" : "+v"(eps2));  // a scalar operand halves an instruction's rate
     while (true) {
         if (threadIdx.x == 0) next = atomicAdd(queue, 1u);
         __syncthreads();
@@ -174,10 +145,15 @@ __global__ __launch_bounds__(64 * BT_WAVES) void bt_coop_kernel(const BatchItem*
         __syncthreads();  // everyone has read it before the next round's write
         if (it >= n_items) break;
         const BatchItem w = items[it];
-        switch (w.r) {
-            case 2: bt_coop_tile<2, MASK, SEQ>(lds, sh, w, wave, eps2, acc); break;
-            default: bt_coop_tile<1, MASK, SEQ>(lds, sh, w, wave, eps2, acc); break;
-        }
+        const float4* sys = sh + w.off;
+        const int J = bt_share<W>(w.n);
+        const uint32_t i0 = w.i0 + uint32_t(wave / J) * 64, i = i0 + (threadIdx.x & 63);
+        const float4 p = sys[i < w.n ? i : w.n - 1];
+        const float xi[1] = {p.x}, yi[1] = {p.y}, zi[1] = {p.z};
+        float ax[1], ay[1], az[1];
+        coop_sum<1, MASK, false, BT_TILE, W>(lds, sys, 0, w.n, J, wave, i0 < w.n, eps2, 0, xi, yi, zi, ax,
+                                             ay, az);
+        if (wave % J == 0 && i < w.n) acc[w.off + i] = make_float4(ax[0], ay[0], az[0], 0.f);
     }
 }
 
@@ -256,28 +232,36 @@ static int tuned_per_lane(const BatchState* s, size_t n) {
 
 // Bodies per lane of a system's items. Untuned: two, one for systems with at most half a
 // workgroup's lanes.
-static uint32_t per_lane_for(const BatchState* s, size_t n) {
-    const int r = tuned_per_lane(s, n);
-    return uint32_t(r ? r : n >= 256 ? 2 : 1);
-}
-
 static int build_items(pnb_ctx* c, BatchState* s) {
     std::vector<BatchItem> items;
     s->interactions = 0;
-    // Workgroups share the items unless a tuning entry asks for more bodies per lane than they
-    // hold. Force pass, wavefronts with 4 per lane / workgroups with 2: one system of 16,384 bodies
-    // 3.10 / 0.37 ms; sizes log-uniform in 64 .. 16,384: 128 systems 3.60 / 1.09, 1,024 8.25 /
-    // 7.00, 2,048 13.9 / 13.4; 512 of 64 .. 65,536 45.4 / 41.5; 2,000 of 64 .. 500 187 / 90 us.
-    s->coop = true;
-    for (size_t k = 0; k < s->systems && s->coop; ++k)
-        s->coop = tuned_per_lane(s, size_t(s->offsets[k + 1] - s->offsets[k])) <= BT_R_MAX;
+    // Workgroups share the items unless a tuning entry asks for more bodies per lane, of eight
+    // wavefronts, or of sixteen while eight make at most two items per CU. Eight steps and the
+    // state's read, wavefronts with four bodies per lane / workgroups of 8 / of 16 (ms): one system of
+    // 16,384 bodies 23.9 / 1.44 / 0.92; four 25.6 / 2.88 / 3.41; sizes log-uniform in 64 .. 500: 16
+    // systems 1.03 / 0.25 / 0.23, 2,000 3.18 / 2.23 / 2.39; in 64 .. 16,384: 128 systems 30.6 / 8.64 /
+    // 10.9, 1,024 79.2 / 67.9 / 86.7. Two bodies per lane in workgroups of 8: 2.41, 4.24, 0.29, 2.27,
+    // 9.39, 70.5 (larger items leave a longer tail).
+    s->waves = 8;
+    for (size_t k = 0; k < s->systems && s->waves; ++k)
+        if (tuned_per_lane(s, size_t(s->offsets[k + 1] - s->offsets[k])) > 1) s->waves = 0;
+    if (s->waves) {
+        size_t count = 0;
+        for (size_t k = 0; k < s->systems; ++k) {
+            const uint32_t n = uint32_t(s->offsets[k + 1] - s->offsets[k]);
+            count += div_up(n, 64 * (8 / bt_share<8>(n)));
+        }
+        if (count <= 2 * size_t(std::max(1, c->cu_count))) s->waves = 16;
+    }
     for (size_t k = 0; k < s->systems; ++k) {
         const uint32_t off = uint32_t(s->offsets[k]);
         const uint32_t n = uint32_t(s->offsets[k + 1] - s->offsets[k]);
         if (n == 0) continue;
         s->interactions += (unsigned long long)n * n;
-        const uint32_t r = per_lane_for(s, n);
-        const uint32_t tile = 64 * r * (s->coop ? uint32_t(BT_WAVES / bt_share(n)) : 1u);
+        const uint32_t r = uint32_t(std::max(1, tuned_per_lane(s, n)));
+        const uint32_t tile = s->waves == 16  ? 64 * (16 / bt_share<16>(n))
+                              : s->waves == 8 ? 64 * (8 / bt_share<8>(n))
+                                              : 64 * r;
         for (uint32_t i0 = 0; i0 < n; i0 += tile) items.push_back({off, n, i0, r});
     }
     std::stable_sort(items.begin(), items.end(), [](const BatchItem& a, const BatchItem& b) {
@@ -297,13 +281,10 @@ static int build_items(pnb_ctx* c, BatchState* s) {
 static int force(pnb_ctx* c, BatchState* s) {
     const bool mask = s->checked && s->softening == 0.0f;
     const float eps2 = s->softening * s->softening;
-    // terms in source order once the items give every SIMD four wavefronts (bf_body); below that
-    // 16 systems of 64 .. 500 bodies take 41 us so, 32 us otherwise
-    const bool seq = s->n_items * BT_WAVES >= size_t(16) * std::max(1, c->cu_count);
-    auto k = !s->coop ? (mask ? bt_force_kernel<true> : bt_force_kernel<false>)
-             : seq    ? (mask ? bt_coop_kernel<true, true> : bt_coop_kernel<false, true>)
-                      : (mask ? bt_coop_kernel<true, false> : bt_coop_kernel<false, false>);
-    const unsigned block = s->coop ? 64 * BT_WAVES : 256;
+    auto k = s->waves == 0   ? (mask ? bt_force_kernel<true> : bt_force_kernel<false>)
+             : s->waves == 8 ? (mask ? bt_coop_kernel<8, true> : bt_coop_kernel<8, false>)
+                             : (mask ? bt_coop_kernel<16, true> : bt_coop_kernel<16, false>);
+    const unsigned block = s->waves ? 64 * s->waves : 256;
     int occ = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k, int(block), 0) != hipSuccess || occ < 1) occ = 2;
     const unsigned grid = unsigned(std::max(1, c->cu_count) * occ);

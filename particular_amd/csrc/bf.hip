@@ -123,8 +123,8 @@ __global__ __launch_bounds__(64 * COOP_WAVES) void bf_coop_kernel(const float4* 
     const float xi[1] = {p.x}, yi[1] = {p.y}, zi[1] = {p.z};
     float ax[1], ay[1], az[1];
     asm volatile("" : "+v"(eps2));  // a scalar operand halves an instruction's rate
-    coop_sum<1, MASK, SELF, T, COOP_WAVES, true, true>(lds, afg, jb, je, COOP_WAVES, wave, true, eps2, i,
-                                                       xi, yi, zi, ax, ay, az);
+    coop_sum<1, MASK, SELF, T, COOP_WAVES>(lds, afg, jb, je, COOP_WAVES, wave, true, eps2, i, xi, yi,
+                                           zi, ax, ay, az);
     if (wave == 0 && i < n)
         out[size_t(blockIdx.y) * n + i] = make_float4(ax[0], ay[0], az[0], 0.0f);
 }

@@ -46,7 +46,7 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 // the present four are summed: one by one, each body is five scalar instructions, a load and a wait.
 // For sums of few wavefronts (4,096 x 60,000 91 -> 82 us, 4,096 x 4,096 10.8 -> 10.1); where a SIMD
 // holds eight the waits cost nothing and this form is slower (1,048,576 x 65,536 18.7 -> 19.0 ms
-// on one card), as it is for the ensemble's items (64 systems, ten steps 0.93 -> 1.05 ms).
+// on one card).
 template <int T, int R, bool MASK, bool SEQ>
 __device__ __forceinline__ void bf_tile(const float4* __restrict__ q, const float (&xi)[R],
                                         const float (&yi)[R], const float (&zi)[R], float eps2,
@@ -131,7 +131,7 @@ struct CoopLds {
 // so a tile of affected bodies walked by one wavefront takes m x R x 13 x 4.8 cycles (1.7 ms for
 // 16,384 affecting bodies and R = 4); J wavefronts divide that by J without another pass over
 // memory.
-template <int R, bool MASK, bool SELF, int T, int W, bool SEQ = true, bool GROUPS = false>
+template <int R, bool MASK, bool SELF, int T, int W>
 __device__ __forceinline__ void coop_sum(CoopLds<R, W>& lds, const float4* __restrict__ afg,
                                          uint32_t jb, uint32_t je, int J, int wave, bool live,
                                          float eps2, uint32_t self, const float (&xi)[R],
@@ -157,14 +157,11 @@ __device__ __forceinline__ void coop_sum(CoopLds<R, W>& lds, const float4* __res
             const float4* q = afg + j0;
             const uint32_t cnt = min(uint32_t(T), je - j0);
             if (SELF && j0 < own + 64 * R && own < j0 + cnt) {  // only here can a pair be a body with itself
-                bf_span<R, MASK, true, SEQ>(q, cnt, xi, yi, zi, eps2, px, py, pz, j0, self);
-            } else if (GROUPS && cnt == uint32_t(T)) {
-                bf_tile<T, R, MASK, SEQ>(q, xi, yi, zi, eps2, px, py, pz);
+                bf_span<R, MASK, true, true>(q, cnt, xi, yi, zi, eps2, px, py, pz, j0, self);
             } else if (cnt == uint32_t(T)) {
-#pragma unroll 8
-                for (int j = 0; j < T; ++j) bf_body<R, MASK, false, SEQ>(q[j], xi, yi, zi, eps2, px, py, pz);
+                bf_tile<T, R, MASK, true>(q, xi, yi, zi, eps2, px, py, pz);
             } else {
-                bf_span<R, MASK, false, SEQ>(q, cnt, xi, yi, zi, eps2, px, py, pz);
+                bf_span<R, MASK, false, true>(q, cnt, xi, yi, zi, eps2, px, py, pz);
             }
         }
         if (J == 1) {
