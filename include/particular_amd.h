@@ -121,8 +121,11 @@ int pnb_reordered_bf_accel_f32_dev(pnb_ctx *ctx, const float *particles, size_t 
  * (sequential.rs:288-305, 368-385) give the same sums over the whole set (pairs of two massless
  * particles add zero). checked = 0 keeps the reference's unchecked pair form (a pair at zero
  * distance is non-finite); checked = 1 drops such pairs as pnb_bf_accel_f32 does. Sums are
- * compensated, in a fixed order. n up to 2^22; device scratch of 16 * ceil(n / 4096)^2 * 4096
- * bytes (one partial sum per body and block of 4,096 bodies: 4.3 GB at n = 2^20). */
+ * compensated, in a fixed order. n up to 2^22. Below 240,000 bodies (170,000 where pairs at zero
+ * distance have to be found: checked, no softening) each body sums all others instead, which is faster
+ * there, with the scratch of pnb_bf_accel_f32_dev; from there on device scratch of
+ * 16 * ceil(n / 4096)^2 * 4096 bytes (one partial sum per body and block of 4,096 bodies: 4.3 GB at
+ * n = 2^20). */
 int pnb_bf_pairs_accel_f32(pnb_ctx *ctx, const float *particles, size_t n, float softening,
                            int checked, float *out);
 int pnb_bf_pairs_accel_f32_dev(pnb_ctx *ctx, const float *particles, size_t n, float softening,

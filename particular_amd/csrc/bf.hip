@@ -2,8 +2,8 @@
 //
 // Replaces the reference's wgpu brute force (particular/src/gpu/bruteforce_shared.wgsl:8-31 and
 // particular/src/gpu/mod.rs:179-208) with its own design for CDNA4:
-//  * each lane owns R affected particles (register blocking): one affecting body fetched per
-//    wave feeds R independent FMA chains;
+//  * each lane owns R affected particles: one by default, its terms kept in source order (bf_body), more
+//    by a tuning entry (register blocking: one affecting body fetched per wave feeds R chains);
 //  * affecting bodies are shared by the whole workgroup, either staged tile by tile in LDS and
 //    read back as broadcasts (variant 0) or read straight from memory with wave-uniform addresses,
 //    which the compiler turns into scalar loads into SGPRs (variant 1);
@@ -11,8 +11,10 @@
 //    a_i += d * (mu * rsq(r2)^3), r2 = |d|^2 + eps^2;
 //  * sums are plain FP32 within a tile of BF_TILE affecting bodies and Kahan-compensated across
 //    tiles, so the error does not grow with the affecting count;
-//  * small affected counts split the affecting range over several workgroups (j_split) whose
-//    partial sums are reduced in a fixed order, so results do not depend on scheduling.
+//  * the affecting range is split over several workgroups (j_split) whose partial sums are reduced
+//    in a fixed order, so results do not depend on scheduling;
+//  * sums of up to some ten thousand affected bodies are taken by workgroups of sixteen wavefronts
+//    per 64 affected bodies that share the affecting ones tile by tile (bf_coop_kernel).
 // Pair semantics follow particular/src/gravity/impls/mod.rs:151-166: with `checked` a pair at
 // zero unsoftened distance contributes nothing; with softening > 0 that pair contributes
 // d * finite = 0 anyway, so only checked && softening == 0 needs the explicit mask.

@@ -31,7 +31,8 @@
 // Traversal: one wavefront walks the pre-order node array with one shared cursor. A lane that
 // opens node k lets the wave step to k+1; a lane that accepts or skips k waits until the cursor
 // reaches skip[k]. Each lane therefore applies exactly the reference's decisions; node records
-// are wave-uniform, so they arrive through scalar loads.
+// are wave-uniform, so they arrive through scalar loads. Small and middle sets, whose wavefronts are too
+// few to hide a load per step, walk in batches of 64 nodes instead (bh_list.hpp), to the same bits.
 // Optional relative criterion (PNB_BH_RELATIVE, no reference counterpart): a node also opens when
 // its first neglected term exceeds alpha times the particle's estimated acceleration; an
 // estimate pass over one centroid per wavefront gives that acceleration, walk records carrying

@@ -8,6 +8,8 @@
 // at zero distance gives a non-finite result); `checked` masks such pairs as the one-sided brute
 // force does (particular/src/gravity/impls/mod.rs:160-161), unchecked keeps the reference's form.
 //
+// Smaller sets are summed one-sidedly (bf_self_launch; PR_MIN_N has both sides' times).
+//
 // Design for CDNA4 (one pair term feeds two accelerations, so a pair costs about 17 VALU against
 // 2 x 13 for the one-sided kernel):
 //  * tiles of T = 64 R bodies; one wavefront holds an i-tile in registers (R bodies per lane,
@@ -216,7 +218,7 @@ constexpr size_t PR_MAX_N = size_t(1) << 22;
 // workgroup per two super-tiles of 4,096 bodies (36 workgroups at 30,000 bodies, two resident per
 // CU), each a serial pass of 8 x 512 j bodies (2.4 ms alone, 3.7 ms with two on a CU).
 // Measured, pair kernel against one-sided, softened: 4,096 bodies 1,402 / 16 us; 30,011: 2,390 /
-// 288; 131,072: 5,980 / 4,362; 196,608: 9.83 / 9.64 ms; 262,144: 16.6 / 17.0. With the
+// 269; 131,072: 5,980 / 4,362; 196,608: 9.83 / 9.64 ms; 262,144: 16.6 / 17.0. With the
 // zero-distance mask: 131,072 6.5 / 4.9 ms; 196,608 10.5 / 10.8.
 constexpr size_t PR_MIN_N = 240000, PR_MIN_N_MASKED = 170000;
 

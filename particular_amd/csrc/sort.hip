@@ -6,7 +6,8 @@
 // the AND of eight ballot masks; the rank is the popcount of that set below the lane). A tile of
 // 2048 keys (the fastest of 1024, 2048 and 4096 at 4M keys) is split into four contiguous wave
 // segments processed in order, so the ranking is stable. Digits on which all keys agree are
-// skipped (found from one OR/AND reduction).
+// skipped (found from one OR/AND reduction). Up to MID_SORT pairs a digit is one launch
+// (ms_pass_kernel), up to SMALL_SORT pairs keys are ranked by counting (rank_count_kernel).
 #include "pnb_internal.hpp"
 
 namespace pnb {
