@@ -1527,7 +1527,7 @@ __device__ __forceinline__ float half_hi(uint32_t v) {
 // (5 bits) of a small internal node; lanes that open it add its bodies (`bodies`, the affecting
 // particles in tree order) directly and skip its subtree.
 // est_out (estimate pass): writes alpha |a| per particle, in walk order, instead of out.
-// wave_order (REL, optional): the launch's k-th wavefront (k < ceil(n / 64)) walks the particles
+// wave_order (optional, 64 lanes): the launch's k-th wavefront (k < ceil(n / 64)) walks the particles
 // of wavefront wave_order[k], so that the heaviest wavefronts start first.
 // lanes: only the first `lanes` lanes of each wavefront walk (64 except in the estimate pass).
 // packed (not with REL): the wavefront's particles are consecutive, `lanes` of them from
@@ -1575,7 +1575,7 @@ __global__ __launch_bounds__(256) void bh_walk_kernel(const NodeRec* __restrict_
         }
         total = info->total;
     }
-    if (REL && wave_order) {
+    if (wave_order) {
         const uint32_t k = i >> 6;  // this wavefront's place in the launch
         if (k < ((n + 63) >> 6)) i = (wave_order[k] << 6) | (i & 63);
     }
@@ -2209,6 +2209,43 @@ __global__ void bh_est_gather_kernel(const float* __restrict__ spread, uint32_t 
     if (w < waves) est[w] = spread[(w / EST_GROUP) * 64 + w % EST_GROUP];
 }
 
+// log2 of the diagonal of each wavefront's box of particles (in walk order).
+__global__ __launch_bounds__(256) void bh_wave_size_kernel(const float4* __restrict__ pts, uint32_t n,
+                                                           float* __restrict__ size) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    const float4 p = pts[min(i, n - 1)];
+    float mn[3] = {p.x, p.y, p.z}, mx[3] = {p.x, p.y, p.z};
+    for (int off = 32; off > 0; off >>= 1)
+        for (int a = 0; a < 3; ++a) {
+            mn[a] = fminf(mn[a], __shfl_xor(mn[a], off, 64));
+            mx[a] = fmaxf(mx[a], __shfl_xor(mx[a], off, 64));
+        }
+    const float dx = mx[0] - mn[0], dy = mx[1] - mn[1], dz = mx[2] - mn[2];
+    if ((threadIdx.x & 63) == 0 && i < n)
+        size[i >> 6] = 0.5f * log2f(fmaxf(dx * dx + dy * dy + dz * dz, 1e-37f));
+}
+
+// Sort keys that put the wavefronts with the most steps first, as far as their boxes tell: steps grow
+// where particles are dense (small boxes along the tree order, averaged over 33 wavefronts) and with a
+// box that is large for its surroundings (particles of several branches). Rank correlation with the
+// counted steps 0.85 on Plummer spheres at theta 0.45 and 0.5. A band is a factor of four in the measure,
+// some 15 % in steps: the stable sort keeps the tree order, and with it the caches' share, inside a
+// band (1,048,576 bodies, two thirds massive, theta 0.7: 2,050 us unordered, 2,060 so, 2,125 with bands
+// of 2 %).
+__global__ __launch_bounds__(256) void bh_wave_cost_kernel(const float* __restrict__ size, uint32_t waves,
+                                                           uint64_t* __restrict__ keys,
+                                                           uint32_t* __restrict__ vals) {
+    const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
+    if (w >= waves) return;
+    float sum = 0.f;
+#pragma unroll
+    for (int d = -16; d <= 16; ++d) sum += size[min(uint32_t(max(int(w) + d, 0)), waves - 1)];
+    const float f = fmaf(3.f / 33.f, sum, -size[w]);
+    keys[w] = uint64_t((fminf(fmaxf(f, -250.f), 250.f) + 256.f) * 0.5f);  // below 2^8
+    vals[w] = w;
+}
+constexpr int WAVE_COST_BITS = 8;
+
 template <int MODE, bool REL>
 static void launch_walk(bool wide, unsigned grid, hipStream_t st, const NodeRec* nr, uint32_t total,
                         const float4* pts, const uint32_t* perm, uint32_t n, float theta2,
@@ -2396,16 +2433,45 @@ static int walk(pnb_ctx* c, const float4* pts, const uint32_t* perm, size_t n, f
         } else {
             const uint32_t lanes = walk_lanes(c, n);
             const unsigned pgrid = unsigned(div_up(div_up(n, size_t(lanes)) * 64, size_t(256)));
+            // Heaviest wavefronts first where the launch's tail counts: with 14 to 64 wavefronts per
+            // CU, corrected 10 to 128 (fewer run all at once, more absorb the tail). A pass at theta
+            // 0.5 in tree order / so (us): plain 262,144 bodies 1,510 / 1,413, 524,288 2,200 / 2,115,
+            // 1,048,576 3,850 / 3,755, 2,000,000 6,874 / 6,872; corrected 165,000 2,240 / 2,083, 262,144
+            // 2,765 / 2,445, 1,048,576 7,415 / 7,010, 2,000,000 12,800 / 12,470. Plain walks of wider
+            // angles are too short for it (a uniform cube of 500,000 at theta 0.8 934 / 951). The order
+            // changes no result: every wavefront's sums are its own.
+            const uint32_t* order = nullptr;
+            const size_t cus = size_t(std::max(c->cu_count, 1));
+            if (!dd && lanes == 64 && total > 0 && (quad || theta <= 0.7f) &&
+                waves >= (quad ? 10 : 14) * cus && waves <= (quad ? 127 : 64) * cus) {
+                PNB_HIP(c, s->wkey.ensure(waves * 8));
+                PNB_HIP(c, s->wkey_alt.ensure(waves * 8));
+                PNB_HIP(c, s->wval.ensure(waves * 4));
+                PNB_HIP(c, s->wval_alt.ensure(waves * 4));
+                PNB_HIP(c, s->est.ensure(waves * sizeof(float)));
+                bh_wave_size_kernel<<<div_up(n, 256), 256, 0, c->stream>>>(pts, uint32_t(n), s->est.as<float>());
+                PNB_CHECK_LAUNCH(c);
+                bh_wave_cost_kernel<<<div_up(waves, 256), 256, 0, c->stream>>>(
+                    s->est.as<float>(), uint32_t(waves), s->wkey.as<uint64_t>(), s->wval.as<uint32_t>());
+                PNB_CHECK_LAUNCH(c);
+                uint64_t* sk;
+                uint32_t* sv;
+                if (int rc = radix_sort_pairs(c, s->wkey.as<uint64_t>(), s->wval.as<uint32_t>(),
+                                              s->wkey_alt.as<uint64_t>(), s->wval_alt.as<uint32_t>(),
+                                              waves, WAVE_COST_BITS, s->hist, s->bits, &sk, &sv))
+                    return rc;
+                order = sv;
+            }
             if (quad)
                 launch_walk<WALK_QUAD, false>(wide, pgrid, c->stream, nr, total, pts, perm,
                                               uint32_t(n), theta2, eps2, out, info, WalkRows{},
-                                              s->qh.as<QuadH>(), nullptr, 0, nullptr, 0.f, nullptr,
+                                              s->qh.as<QuadH>(), nullptr, 0, nullptr, 0.f, order,
                                               nullptr, lanes, dd ? 1 : 0, 1,
                                               s->oh.as<OctH>(), mlp_octupole(c) ? 1 : 0);
             else
                 launch_walk<WALK_PLAIN, false>(wide, pgrid, c->stream, nr, total, pts, perm,
                                                uint32_t(n), theta2, eps2, out, info, WalkRows{},
-                                               nullptr, nullptr, 0, nullptr, 0.f, nullptr, nullptr,
+                                               nullptr, nullptr, 0, nullptr, 0.f, order, nullptr,
                                                lanes, dd ? 1 : 0, 1);
         }
         PNB_CHECK_LAUNCH(c);

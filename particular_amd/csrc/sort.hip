@@ -340,7 +340,8 @@ __global__ __launch_bounds__(256) void rs_gather_kernel(const float4* __restrict
 // either the input pair or the alternate pair. Only bits [0, key_bits) are considered, and above
 // SMALL_SORT pairs only bits from low_bit on (a caller that wants neighbours together, not an order).
 // dst (optional): dst[i] = src[i-th value], written by the sort's last launch below MID_SORT pairs. Up to
-// SMALL_SORT pairs (keys of at most 63 bits) are ranked by counting, into the alternate pair;
+// SMALL_SORT pairs (keys of at most 63 bits, and more than one digit above 2,048 pairs) are ranked by
+// counting, into the alternate pair;
 // either way equal keys keep their input order.
 // Digits no two keys differ in are skipped after one read-back to the host, unless all_digits.
 int radix_sort_pairs(pnb_ctx* c, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
@@ -356,7 +357,7 @@ int radix_sort_pairs(pnb_ctx* c, uint64_t* keys, uint32_t* vals, uint64_t* keys_
         return PNB_OK;
     };
     if (n <= 1) return gather(vals);
-    if (n <= SMALL_SORT && key_bits <= 63) {
+    if (n <= SMALL_SORT && key_bits <= 63 && !(key_bits <= 8 && n > 2048)) {
         const uint64_t mask = key_bits >= 64 ? ~0ull : ((1ull << key_bits) - 1);
         const uint32_t nn = uint32_t(n), span = n > RANK_SPAN && n <= 8192 ? RANK_SPAN / 4 : RANK_SPAN;
         const uint32_t g = div_up(nn, 256u), parts = div_up(nn, span);
