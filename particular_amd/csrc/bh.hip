@@ -2438,8 +2438,10 @@ static int walk(pnb_ctx* c, const float4* pts, const uint32_t* perm, size_t n, f
             // 0.5 in tree order / so (us): plain 262,144 bodies 1,510 / 1,413, 524,288 2,200 / 2,115,
             // 1,048,576 3,850 / 3,755, 2,000,000 6,874 / 6,872; corrected 165,000 2,240 / 2,083, 262,144
             // 2,765 / 2,445, 1,048,576 7,415 / 7,010, 2,000,000 12,800 / 12,470. Plain walks of wider
-            // angles are too short for it (a uniform cube of 500,000 at theta 0.8 934 / 951). The order
-            // changes no result: every wavefront's sums are its own.
+            // angles are too short for it (a uniform cube of 500,000 at theta 0.8 934 / 951). Those are
+            // Plummer spheres; where wavefronts differ little the ordering costs more than the tail
+            // (262,144 bodies, uniform cube 1,054 / 1,071, disc 837 / 849; at 500,000 1,472 / 1,442 and
+            // 1,215 / 1,182). The order changes no result: every wavefront's sums are its own.
             const uint32_t* order = nullptr;
             const size_t cus = size_t(std::max(c->cu_count, 1));
             if (!dd && lanes == 64 && total > 0 && (quad || theta <= 0.7f) &&
