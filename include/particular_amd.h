@@ -123,9 +123,9 @@ int pnb_reordered_bf_accel_f32_dev(pnb_ctx *ctx, const float *particles, size_t 
  * distance is non-finite); checked = 1 drops such pairs as pnb_bf_accel_f32 does. Sums are
  * compensated, in a fixed order. n up to 2^22. Below 240,000 bodies (170,000 where pairs at zero
  * distance have to be found: checked, no softening) each body sums all others instead, which is faster
- * there, with the scratch of pnb_bf_accel_f32_dev; from there on device scratch of
- * 16 * ceil(n / 4096)^2 * 4096 bytes (one partial sum per body and block of 4,096 bodies: 4.3 GB at
- * n = 2^20). */
+ * there, with up to 64 partial sums of 16 bytes per body as device scratch; from there on the scratch is
+ * 16 * ceil(n / 4096)^2 * 4096 bytes, at least 246 MB (one partial sum per body and block of 4,096
+ * bodies: 4.3 GB at n = 2^20). */
 int pnb_bf_pairs_accel_f32(pnb_ctx *ctx, const float *particles, size_t n, float softening,
                            int checked, float *out);
 int pnb_bf_pairs_accel_f32_dev(pnb_ctx *ctx, const float *particles, size_t n, float softening,

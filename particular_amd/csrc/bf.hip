@@ -259,12 +259,12 @@ static BfPlan plan_for(const BfShape& sh, size_t m) {
 
 static BfPlan plan(pnb_ctx* c, size_t n, size_t m) { return plan_for(choose_shape(c, n, m), m); }
 
-// Allocates what bf_launch(n, m) will need, so that a later launch inside a graph capture
-// allocates nothing.
-int bf_prepare(pnb_ctx* c, size_t n, size_t m) {
+// Allocates in `scratch` what bf_launch(n, m) will need of it, so that a later launch inside a graph
+// capture allocates nothing.
+int bf_prepare(pnb_ctx* c, size_t n, size_t m, DevBuf& scratch) {
     if (n == 0 || m == 0) return PNB_OK;
     const BfPlan p = plan(c, n, m);
-    if (p.splits > 1) PNB_HIP(c, c->bf_partial.ensure(size_t(p.splits) * n * sizeof(float4)));
+    if (p.splits > 1) PNB_HIP(c, scratch.ensure(size_t(p.splits) * n * sizeof(float4)));
     return PNB_OK;
 }
 
@@ -323,20 +323,22 @@ static int bf_launch_with(pnb_ctx* c, const BfPlan& p, const float4* affected, s
 }
 
 // The sum over all other bodies of one set, for sizes where the pair kernel cannot fill the chip
-// (pairs.hip): a body's term with itself is left out by index, whatever the softening.
+// (pairs.hip): a body's term with itself is left out by index, whatever the softening. The split's
+// partial sums are kept in the pair kernel's scratch, so that a pair sum frees no memory that an
+// f32 brute force captured in a graph goes on using (DevBuf::ensure frees what it outgrows).
 int bf_self_launch(pnb_ctx* c, const float4* p, size_t n, float softening, int checked, float4* out) {
     const BfPlan pl = plan_for(default_shape(c, n, n), n);
     if (pl.splits > 1) {
         const size_t need = size_t(pl.splits) * n * sizeof(float4);
-        if (c->capturing && c->bf_partial.cap < need)
+        if (c->capturing && c->pairs_part.cap < need)
             return fail(c, PNB_E_STATE, "brute-force scratch not prepared before graph capture");
-        PNB_HIP(c, c->bf_partial.ensure(need));
+        PNB_HIP(c, c->pairs_part.ensure(need));
     }
-    return bf_launch_with(c, pl, p, n, p, n, softening, checked, out, c->bf_partial.as<float4>(), true);
+    return bf_launch_with(c, pl, p, n, p, n, softening, checked, out, c->pairs_part.as<float4>(), true);
 }
 
 int bf_launch(pnb_ctx* c, const float4* affected, size_t n, const float4* affecting, size_t m,
-              float softening, int checked, float4* out) {
+              float softening, int checked, float4* out, DevBuf* scratch) {
     if (n == 0) return PNB_OK;
     if (n > 0x7fffffffu || m > 0x7fffffffu)
         return fail(c, PNB_E_ARG, "brute force supports at most 2^31-1 particles per side");
@@ -346,14 +348,14 @@ int bf_launch(pnb_ctx* c, const float4* affected, size_t n, const float4* affect
         return PNB_OK;
     }
     const BfPlan p = plan(c, n, m);
+    DevBuf& part = scratch ? *scratch : c->bf_partial;
     if (p.splits > 1) {
         const size_t need = size_t(p.splits) * n * sizeof(float4);
-        if (c->capturing && c->bf_partial.cap < need)
+        if (c->capturing && part.cap < need)
             return fail(c, PNB_E_STATE, "brute-force scratch not prepared before graph capture");
-        PNB_HIP(c, c->bf_partial.ensure(need));
+        PNB_HIP(c, part.ensure(need));
     }
-    return bf_launch_with(c, p, affected, n, affecting, m, softening, checked, out,
-                          c->bf_partial.as<float4>());
+    return bf_launch_with(c, p, affected, n, affecting, m, softening, checked, out, part.as<float4>());
 }
 
 // ---- FP64 direct sum: one workgroup per affected particle, fixed-order tree reduction --------
@@ -629,14 +631,15 @@ int pnb_bf_accel_f64_dev(pnb_ctx* c, const double* affected, size_t n, const dou
     splits = std::max<size_t>(1, div_up(m, chunk));
     double4* o = reinterpret_cast<double4*>(out);
     double4* dst = o;
-    // inside a caller's capture nothing can be allocated: one range when the scratch is too small
-    if (splits > 1 && c->bf_partial.cap < splits * n * sizeof(double4) && stream_capturing(c)) {
+    // Inside a caller's capture one range and no scratch: nothing can be allocated there, and a later
+    // call that needs more would free the memory that the graph goes on using.
+    if (splits > 1 && stream_capturing(c)) {
         splits = 1;
         chunk = uint32_t(m);
     }
     if (splits > 1) {
-        PNB_HIP(c, c->bf_partial.ensure(splits * n * sizeof(double4)));
-        dst = c->bf_partial.as<double4>();
+        PNB_HIP(c, c->bf64_partial.ensure(splits * n * sizeof(double4)));
+        dst = c->bf64_partial.as<double4>();
     }
     // The self term and coincident pairs add d * s = 0 with s finite when the softening is not
     // tiny (mu < 1e263 here), so only a vanishing softening needs the mask.

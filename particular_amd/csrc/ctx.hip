@@ -420,7 +420,7 @@ void pnb_destroy(pnb_ctx* c) {
     for (void* p : {c->pin_in, c->pin_out, static_cast<void*>(c->pin_count)})
         if (p) (void)hipHostFree(p);
     for (pnb::DevBuf* b : {&c->h_affected, &c->h_affecting, &c->h_out, &c->split_tmp,
-                           &c->split_counts, &c->bf_partial, &c->scan_tmp, &c->pairs_part, &c->d2_raw_a,
+                           &c->split_counts, &c->bf_partial, &c->bf64_partial, &c->scan_tmp, &c->pairs_part, &c->d2_raw_a,
                            &c->d2_raw_b, &c->d2_a, &c->d2_b, &c->d2_out4, &c->d2_out2})
         b->release();
     for (int k = 0; k < pnb_ctx::EV_POOL; ++k) {

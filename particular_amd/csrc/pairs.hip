@@ -236,7 +236,9 @@ int pairs_launch(pnb_ctx* c, const float4* p, size_t n, float softening, int che
     if (n < (mask ? PR_MIN_N_MASKED : PR_MIN_N)) return bf_self_launch(c, p, n, softening, checked, out);
     const uint32_t ns = uint32_t(div_up(n, PR_S));
     const uint32_t n_pad = ns * uint32_t(PR_S);
-    const size_t need = size_t(ns) * n_pad * sizeof(float4);
+    // at least what any one-sided sum needs (64 ranges), so that a call on a set of any size leaves room
+    // for the smaller ones, also inside a graph capture, where nothing can be allocated
+    const size_t need = std::max(size_t(ns) * n_pad, 64 * PR_MIN_N) * sizeof(float4);
     if (c->capturing && c->pairs_part.cap < need)
         return fail(c, PNB_E_STATE, "pair scratch not prepared before graph capture");
     PNB_HIP(c, c->pairs_part.ensure(need));

@@ -43,11 +43,15 @@ struct pnb_ctx {
     int cu_count = 0;
 
     // scratch for host-pointer entry points and the massive/massless split
-    pnb::DevBuf h_affected, h_affecting, h_out, split_tmp, split_counts, bf_partial;
+    pnb::DevBuf h_affected, h_affecting, h_out, split_tmp, split_counts;
+    // partial sums of a split affecting range: f32 brute force, FP64 brute force. One buffer each: a
+    // graph that a caller captured over a call holds its buffer's address, and a buffer that grows
+    // moves, so no call may grow another entry point's.
+    pnb::DevBuf bf_partial, bf64_partial;
     pnb::DevBuf scan_tmp;
     void *pin_in = nullptr, *pin_out = nullptr;  // pinned: stage_in's two slots, stage_out's one
     uint32_t* pin_count = nullptr;               // pinned: split_affecting's count
-    pnb::DevBuf pairs_part;  // pair brute force: one partial per body and super-tile
+    pnb::DevBuf pairs_part;  // pair brute force: one partial per body and super-tile or range
     // device address of the allocation-free entry point's static scratch on this device
     float4* noalloc_scratch = nullptr;
     // two-dimensional entry points: {x, y, mu} records staged, widened to float4, results narrowed
@@ -107,9 +111,11 @@ struct Fetch {
 };
 int stage_fetch(pnb_ctx* c, std::initializer_list<Fetch> parts);
 
-// Brute force on device pointers, asynchronous on c->stream.
+// Brute force on device pointers, asynchronous on c->stream. scratch: holds the partial sums of a split
+// affecting range (the context's own by default); bf_prepare sizes it.
 int bf_launch(pnb_ctx* c, const float4* affected, size_t n, const float4* affecting, size_t m,
-              float softening, int checked, float4* out);
+              float softening, int checked, float4* out, DevBuf* scratch = nullptr);
+int bf_prepare(pnb_ctx* c, size_t n, size_t m, DevBuf& scratch);
 // Brute force of one set on itself, each body's own term left out by index.
 int bf_self_launch(pnb_ctx* c, const float4* p, size_t n, float softening, int checked, float4* out);
 

@@ -16,13 +16,12 @@
 
 namespace pnb {
 
-int bf_prepare(pnb_ctx* c, size_t n, size_t m);
-
 struct StepState {
     size_t n = 0, m = 0;
     float softening = 0.0f;
     int checked = 1;
     DevBuf x, v, acc, shadow, afg, rank, stage;
+    DevBuf partial;  // the force's partial sums: no other call may move what a kept graph writes to
     hipGraphExec_t exec = nullptr;
     hipGraph_t graph = nullptr;
     size_t graph_steps = 0;
@@ -40,7 +39,8 @@ struct StepState {
 void step_free(StepState* s) {
     if (!s) return;
     s->drop_graph();
-    for (DevBuf* b : {&s->x, &s->v, &s->acc, &s->shadow, &s->afg, &s->rank, &s->stage}) b->release();
+    for (DevBuf* b : {&s->x, &s->v, &s->acc, &s->shadow, &s->afg, &s->rank, &s->stage, &s->partial})
+        b->release();
     delete s;
 }
 
@@ -128,7 +128,7 @@ static int enqueue_steps(pnb_ctx* c, StepState* s, size_t steps, double dt) {
         });
         if (rc) return rc;
         rc = bf_launch(c, s->shadow.as<float4>(), s->n, s->afg.as<float4>(), s->m, s->softening,
-                       s->checked, s->acc.as<float4>());
+                       s->checked, s->acc.as<float4>(), &s->partial);
         if (rc) return rc;
     }
     if (steps) {
@@ -182,9 +182,9 @@ int pnb_leapfrog_init(pnb_ctx* c, const double* pos3, const double* vel3, const 
     s->m = m;
     lf_compact_kernel<<<g, 256, 0, c->stream>>>(s->shadow.as<float4>(), rank, n, s->afg.as<float4>());
     PNB_CHECK_LAUNCH(c);
-    if (int rc = bf_prepare(c, n, m)) return rc;
+    if (int rc = bf_prepare(c, n, m, s->partial)) return rc;
     if (int rc = bf_launch(c, s->shadow.as<float4>(), n, s->afg.as<float4>(), m, softening, checked,
-                           s->acc.as<float4>()))
+                           s->acc.as<float4>(), &s->partial))
         return rc;
     PNB_HIP(c, hipStreamSynchronize(c->stream));
     return PNB_OK;
@@ -196,6 +196,12 @@ int pnb_leapfrog_run(pnb_ctx* c, size_t steps, double dt, int use_graph) {
     if (!s || s->n == 0) return fail(c, PNB_E_STATE, "pnb_leapfrog_init has not been called");
     if (steps == 0) return PNB_OK;
     if (int rc = activate(c)) return rc;
+    // a tuning entry set since the last run may ask for more ranges: the graph that holds the outgrown
+    // scratch goes with it
+    const void* had = s->partial.ptr;
+    const int prepared = bf_prepare(c, s->n, s->m, s->partial);
+    if (s->partial.ptr != had) s->drop_graph();
+    if (prepared) return prepared;
     if (!use_graph) return enqueue_steps(c, s, steps, dt);
     if (!c->stream) return fail(c, PNB_E_STATE, "graph capture needs a non-null stream");
     if (!s->exec || s->graph_steps != steps || s->graph_dt != dt || s->graph_stream != c->stream) {
