@@ -19,6 +19,7 @@
 // zero unsoftened distance contributes nothing; with softening > 0 that pair contributes
 // d * finite = 0 anyway, so only checked && softening == 0 needs the explicit mask.
 #include "bf_common.hpp"
+#include "bf_shape.hpp"
 #include "pnb_internal.hpp"
 
 #include <algorithm>
@@ -26,9 +27,6 @@
 #include <vector>
 
 namespace pnb {
-
-constexpr int BF_BLOCK = 256;
-constexpr int BF_TILE = 256;
 
 struct BfTuneEntry {
     size_t n_min;
@@ -108,8 +106,6 @@ __global__ __launch_bounds__(BF_BLOCK) void bf_kernel(const float4* __restrict__
 // (and per affecting range, grid.y), the wavefronts sharing the affecting bodies tile by tile
 // (coop_sum). Up to 512 affected tiles there are too few wavefronts for one of them per tile to
 // fill the chip, and each is bound by its own issue rate.
-constexpr int COOP_WAVES = 16;
-
 template <bool MASK, bool SELF, int T>
 __global__ __launch_bounds__(64 * COOP_WAVES) void bf_coop_kernel(const float4* __restrict__ aff,
                                                                   uint32_t n,
@@ -178,56 +174,7 @@ static BfKernel pick_coop(bool mask, int tile) {
     }
 }
 
-constexpr int BF_COOP = 2;  // variant of the workgroup-cooperative kernel (not for tuning entries)
-
-struct BfShape {
-    int variant, per_lane, j_split;
-};
-
-// What the cooperative kernel takes: sums too small for one wavefront per affected tile and range to
-// fill the chip evenly. Measured, plain kernel with its best split / cooperative (us, softened): 1,000
-// x 1,000 62 / 8; 4,096 x 4,096 36 / 10; 10,000 x 8,000 45 / 30; 20,000 x 20,000 142 / 122; 30,000 x
-// 65,536 628 / 568; 45,000 x 130,000 1,695 / 1,659, without softening 1,861 / 1,862; 65,536 x 16,384
-// 321 / 308; 90,000 x 30,000 781 / 775, 864 / 868; 130,000 x 4,000 163 / 160; 130,000 x 30,000 1,098 /
-// 1,116; 400,000 x 500 75 / 67, x 2,047 305 / 247 (the plain kernel does not split below 2,048). With
-// few affecting bodies there is little to share: 256 x 100 6.0 / 8.8, 256 x 128 6.9 / 7.6, 256 x 200
-// 9.8 / 8.7; 65,536 x 200 10.0 / 9.7, 90,000 x 200 11 / 13.
-static bool coop_pays(size_t n, size_t m) {
-    if (m <= 256) return m > 128 && n <= 65536;
-    if (m < 2048) return true;
-    return n <= 50000 || (n <= 100000 && m <= 16384) || (n <= 150000 && m <= 4096);
-}
-
-static BfShape default_shape(pnb_ctx* c, size_t n, size_t m) {
-    const size_t cus = c->cu_count > 0 ? size_t(c->cu_count) : 256;
-    int s = 1;
-    if (coop_pays(n, m)) {
-        // Workgroups of 16 wavefronts over ranges of the affecting bodies: two per CU while a range
-        // keeps 500 of them, which is half a tile for each wavefront, and up to 16 per CU, so that
-        // no CU has twice another's work, while it keeps 700. 9,000 x 9,000 in 1 / 2 / 4 / 8 / 16
-        // ranges 50 / 54 / 40 / 32 / 32 us; 6,000 x 6,000 33 / 22 / 21 / 16 / 20; 1,000 x 8,000 41 /
-        // 25 / 16 / 10 / 8; 20,000 x 20,000 186 / 145 / 126 / 122 / 124.
-        const size_t blocks = div_up(n, 64);
-        while (m >= 2048 && s < 64) {
-            const size_t wgs = blocks * s * 2, per = m / (size_t(s) * 2);
-            if (!((wgs <= 2 * cus && per >= 500) || (wgs <= 16 * cus && per >= 700))) break;
-            s <<= 1;
-        }
-        return {BF_COOP, 1, s};
-    }
-    // Otherwise one body per lane and one wavefront per affected tile and range, the affecting
-    // bodies from scalar loads (from LDS for at most a tile, 65,536 x 64 4 / 9 us), the affecting
-    // range from 2,048 bodies on split into up to 64 workgroups per CU of at least one tile each, up
-    // to 256 per CU while ranges stay at 1,024 bodies (small workgroups balance the load across CUs
-    // and XCDs). 1,048,576 x 65,536 16.1 ms, with four bodies per lane 17.1.
-    const size_t blocks = div_up(n, size_t(BF_BLOCK));
-    while (m >= 2048 && s < 64 && blocks * s * 2 <= 256 * cus) {
-        const size_t per = m / (size_t(s) * 2);
-        if (per < (blocks * s * 2 <= 64 * cus ? size_t(BF_TILE) : size_t(1024))) break;
-        s <<= 1;
-    }
-    return {m <= 256 ? 0 : 1, 1, s};
-}
+static size_t cu_count(const pnb_ctx* c) { return c->cu_count > 0 ? size_t(c->cu_count) : 256; }
 
 static BfShape choose_shape(pnb_ctx* c, size_t n, size_t m) {
     if (c->bf_tune) {
@@ -236,25 +183,7 @@ static BfShape choose_shape(pnb_ctx* c, size_t n, size_t m) {
             if (e.n_min <= n && (!best || e.n_min > best->n_min)) best = &e;
         if (best) return {best->variant, best->per_lane, best->j_split};
     }
-    return default_shape(c, n, m);
-}
-
-struct BfPlan {
-    BfShape shape;
-    uint32_t splits, chunk;
-    int tile;
-};
-
-// Splits of the affecting range in whole tiles. The cooperative kernel takes smaller tiles for
-// small ranges, so that all its wavefronts get one.
-static BfPlan plan_for(const BfShape& sh, size_t m) {
-    uint32_t splits = uint32_t(sh.j_split);
-    const size_t per = m / splits / COOP_WAVES;
-    const int tile = sh.variant != BF_COOP || per >= 256 ? BF_TILE : per >= 128 ? 128 : 64;
-    uint32_t chunk = uint32_t(div_up(m, splits));
-    chunk = (chunk + tile - 1) / tile * tile;
-    splits = uint32_t(div_up(m, chunk));
-    return {sh, splits, chunk, tile};
+    return default_shape(cu_count(c), n, m);
 }
 
 static BfPlan plan(pnb_ctx* c, size_t n, size_t m) { return plan_for(choose_shape(c, n, m), m); }
@@ -307,8 +236,8 @@ static int bf_launch_with(pnb_ctx* c, const BfPlan& p, const float4* affected, s
     else k = sh.variant == 0 ? pick_mask<0>(sh.per_lane, mask) : pick_mask<1>(sh.per_lane, mask);
     const float eps2 = softening * softening;
     const uint32_t splits = p.splits, chunk = p.chunk;
-    const unsigned block = coop ? 64 * COOP_WAVES : BF_BLOCK;
-    dim3 grid(div_up(n, coop ? size_t(64) : size_t(BF_BLOCK) * sh.per_lane), splits);
+    const unsigned block = bf_block(sh);
+    dim3 grid(bf_grid_x(sh, n), splits);
     float4* dst = splits > 1 ? partial : out;
     return timed(c, PNB_PROF_BF, [&]() -> int {
         k<<<grid, block, 0, c->stream>>>(affected, uint32_t(n), affecting, uint32_t(m), chunk,
@@ -327,7 +256,7 @@ static int bf_launch_with(pnb_ctx* c, const BfPlan& p, const float4* affected, s
 // partial sums are kept in the pair kernel's scratch, so that a pair sum frees no memory that an
 // f32 brute force captured in a graph goes on using (DevBuf::ensure frees what it outgrows).
 int bf_self_launch(pnb_ctx* c, const float4* p, size_t n, float softening, int checked, float4* out) {
-    const BfPlan pl = plan_for(default_shape(c, n, n), n);
+    const BfPlan pl = plan_for(default_shape(cu_count(c), n, n), n);
     if (pl.splits > 1) {
         const size_t need = size_t(pl.splits) * n * sizeof(float4);
         if (c->capturing && c->pairs_part.cap < need)
@@ -401,8 +330,6 @@ __global__ __launch_bounds__(DF_BLOCK) void direct_f64_kernel(const float4* __re
 // wavefronts holds 64 affected bodies; the affecting range is split over grid.y and, inside a
 // workgroup, over its wavefronts (scalar loads), whose sums are added in wavefront order, and the
 // grid.y partial sums in order by bf64_reduce_kernel. checked: zero distance contributes nothing.
-
-constexpr int BF64_WAVES = 8;
 
 // |r2|^-1/2 to the last bit or two: v_rsq_f64 (about 1e-8 relative) and one third-order step
 // y (1 + e/2 + 3 e^2 / 8), e = 1 - r2 y^2. An infinite r2 (y = 0) stays 0.
@@ -620,37 +547,30 @@ int pnb_bf_accel_f64_dev(pnb_ctx* c, const double* affected, size_t n, const dou
     if (n == 0) return PNB_OK;
     if (n > 0x7fffffffu || m > 0x7fffffffu) return fail(c, PNB_E_ARG, "too many particles");
     if (int rc = activate(c)) return rc;
-    // Workgroups over the affecting range until the launch holds about four rounds of wavefronts
-    // (32 per CU), with at least 32 affecting bodies for each of a workgroup's wavefronts.
-    const size_t cus = c->cu_count > 0 ? size_t(c->cu_count) : 256;
-    const size_t blocks = div_up(n, 64);
-    size_t splits = 1;
-    while (splits < 64 && blocks * splits * BF64_WAVES < 128 * cus && m / (splits * 2) >= 32 * BF64_WAVES)
-        splits <<= 1;
-    uint32_t chunk = std::max(1u, div_up(m, splits));
-    splits = std::max<size_t>(1, div_up(m, chunk));
+    Bf64Plan p = plan64(cu_count(c), n, m);
     double4* o = reinterpret_cast<double4*>(out);
     double4* dst = o;
     // Inside a caller's capture one range and no scratch: nothing can be allocated there, and a later
     // call that needs more would free the memory that the graph goes on using.
-    if (splits > 1 && stream_capturing(c)) {
-        splits = 1;
-        chunk = uint32_t(m);
-    }
-    if (splits > 1) {
-        PNB_HIP(c, c->bf64_partial.ensure(splits * n * sizeof(double4)));
+    if (p.splits > 1 && stream_capturing(c)) p = {1, uint32_t(m)};
+    if (p.splits > 1) {
+        PNB_HIP(c, c->bf64_partial.ensure(p.splits * n * sizeof(double4)));
         dst = c->bf64_partial.as<double4>();
     }
     // The self term and coincident pairs add d * s = 0 with s finite when the softening is not
     // tiny (mu < 1e263 here), so only a vanishing softening needs the mask.
     const double eps2 = softening * softening;
     auto k = checked && eps2 < 1e-30 ? bf64_kernel<true> : bf64_kernel<false>;
-    k<<<dim3(unsigned(blocks), unsigned(splits)), 64 * BF64_WAVES, 0, c->stream>>>(
-        reinterpret_cast<const double4*>(affected), uint32_t(n),
-        reinterpret_cast<const double4*>(affecting), uint32_t(m), chunk, eps2, dst);
-    PNB_CHECK_LAUNCH(c);
-    if (splits > 1) {
-        bf64_reduce_kernel<<<div_up(n, 64), 64, 0, c->stream>>>(dst, uint32_t(n), uint32_t(splits), o);
+    const double4* aff = reinterpret_cast<const double4*>(affected);
+    for (size_t i = 0; i < n; i += BF64_SLICE) {  // one launch but for more than 2^28 bodies, never split
+        const size_t cnt = std::min(n - i, BF64_SLICE);
+        k<<<dim3(div_up(cnt, 64), unsigned(p.splits)), 64 * BF64_WAVES, 0, c->stream>>>(
+            aff + i, uint32_t(cnt), reinterpret_cast<const double4*>(affecting), uint32_t(m), p.chunk, eps2,
+            dst + i);
+        PNB_CHECK_LAUNCH(c);
+    }
+    if (p.splits > 1) {
+        bf64_reduce_kernel<<<div_up(n, 64), 64, 0, c->stream>>>(dst, uint32_t(n), uint32_t(p.splits), o);
         PNB_CHECK_LAUNCH(c);
     }
     return PNB_OK;
