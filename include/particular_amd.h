@@ -264,7 +264,9 @@ int pnb_bh_accel_f32_2d_dev(pnb_ctx *ctx, const float *affected, size_t n, const
 
 /* FP64 brute force for glam::DVec3 / f64 particles (CPU-only in the reference:
  * particular/src/gravity/impls/glam.rs:234): records are 4 doubles {x, y, z, mu} (32 B); the
- * reference's scalar kernel in FP64 with IEEE sqrt and division (impls/mod.rs:151-166). */
+ * reference's scalar kernel in FP64 (impls/mod.rs:151-166), the term mu r^-3 from a corrected reciprocal
+ * square root, as exact as an IEEE square root and division (three roundings). Zero, vanishing and
+ * infinite distances give what the division gives. */
 int pnb_bf_accel_f64(pnb_ctx *ctx, const double *affected, size_t n, const double *affecting,
                      size_t m, double softening, int checked, double *out);
 int pnb_bf_accel_f64_dev(pnb_ctx *ctx, const double *affected, size_t n, const double *affecting,

@@ -331,15 +331,48 @@ __global__ __launch_bounds__(DF_BLOCK) void direct_f64_kernel(const float4* __re
 // workgroup, over its wavefronts (scalar loads), whose sums are added in wavefront order, and the
 // grid.y partial sums in order by bf64_reduce_kernel. checked: zero distance contributes nothing.
 
-// |r2|^-1/2 to the last bit or two: v_rsq_f64 (about 1e-8 relative) and one third-order step
-// y (1 + e/2 + 3 e^2 / 8), e = 1 - r2 y^2. An infinite r2 (y = 0) stays 0.
-__device__ __forceinline__ double rsqrt64(double r2) {
-    const double y = __builtin_amdgcn_rsq(r2);
-    const double e = fma(-(fmin(r2, 1.7976931348623157e308) * y), y, 1.0);
-    return fma(y * e, fma(e, 0.375, 0.5), y);
+// mu r2^(-3/2). From the estimate y = v_rsq_f64(r2) (about 1e-8 relative, here cut to 26 bits, so that
+// y^2 is exact) and e = 1 - r2 y^2, r2^(-3/2) = y^3 (1 - e)^(-3/2), the binomial series to second order
+// (the third is 1e-22). The cube is corrected, not the root, whose error cubing would triple: three
+// roundings, as an IEEE root, product and division have. y^2 takes the correction: it stays finite where
+// the result overflows, which has to give infinity.
+// An infinite r2 (y = 0) gives 0; with ZERO, a vanishing r2 infinity, as a division by it does.
+template <bool ZERO>
+__device__ __forceinline__ double cubed64(double mu, double r2) {
+    const double y = __longlong_as_double(__double_as_longlong(__builtin_amdgcn_rsq(r2)) & ~0x7ffffffll);
+    const double y2 = y * y;
+    double r = fmin(r2, 1.7976931348623157e308);
+    if (ZERO) r = fmax(r, 4.9406564584124654e-324);
+    const double e = fma(-r, y2, 1.0);
+    return (mu * y) * fma(y2 * e, fma(e, 1.875, 1.5), y2);
 }
 
-template <bool MASK>
+// One lane's share, bodies jb .. je of afg. CHECK tests the unsoftened distance; ZERO as above.
+template <bool CHECK, bool ZERO>
+__device__ __forceinline__ double3 sum64(const double4 p, const double4* __restrict__ afg, uint32_t jb,
+                                         uint32_t je, double eps2) {
+    double ax = 0.0, ay = 0.0, az = 0.0;
+#pragma unroll 4
+    for (uint32_t j = jb; j < je; ++j) {
+        const double4 q = afg[j];  // wave-uniform: a scalar load
+        const double dx = q.x - p.x, dy = q.y - p.y, dz = q.z - p.z;
+        const double d2 = fma(dx, dx, fma(dy, dy, CHECK ? dz * dz : fma(dz, dz, eps2)));
+        double s = cubed64<ZERO>(q.w, CHECK ? d2 + eps2 : d2);
+        if (CHECK) s = d2 == 0.0 ? 0.0 : s;
+        ax = fma(dx, s, ax);
+        ay = fma(dy, s, ay);
+        az = fma(dz, s, az);
+    }
+    return make_double3(ax, ay, az);
+}
+
+// Unchecked sums, and checked ones with a softening whose square is normal (there a pair at zero distance
+// adds d s = 0 by itself unless s overflows, and an infinite mu must not reach its own body), are taken
+// without test or clamp, and again with them where they come out NaN: 40,000 x 40,000 bodies 963 us,
+// with the test in every term 1,095, with the clamp 1,005.
+constexpr int BF64_UNCHECKED = 0, BF64_CHECKED = 1, BF64_SOFTENED = 2;
+
+template <int MODE>
 __global__ __launch_bounds__(64 * BF64_WAVES) void bf64_kernel(const double4* __restrict__ aff,
                                                                uint32_t n,
                                                                const double4* __restrict__ afg,
@@ -354,31 +387,25 @@ __global__ __launch_bounds__(64 * BF64_WAVES) void bf64_kernel(const double4* __
     const uint32_t b0 = blockIdx.y * j_chunk, b1 = min(m, b0 + j_chunk);
     const uint32_t per = (b1 - b0 + BF64_WAVES - 1) / BF64_WAVES;
     const uint32_t jb = min(b1, b0 + wave * per), je = min(b1, jb + per);
-    double ax = 0.0, ay = 0.0, az = 0.0;
-#pragma unroll 4
-    for (uint32_t j = jb; j < je; ++j) {
-        const double4 q = afg[j];  // wave-uniform: a scalar load
-        const double dx = q.x - p.x, dy = q.y - p.y, dz = q.z - p.z;
-        // MASK tests the unsoftened distance
-        const double d2 = fma(dx, dx, fma(dy, dy, MASK ? dz * dz : fma(dz, dz, eps2)));
-        double inv = rsqrt64(MASK ? d2 + eps2 : d2);
-        if (MASK) inv = d2 == 0.0 ? 0.0 : inv;
-        const double s = (q.w * inv) * (inv * inv);
-        ax = fma(dx, s, ax);
-        ay = fma(dy, s, ay);
-        az = fma(dz, s, az);
+    double3 a = sum64<MODE == BF64_CHECKED, false>(p, afg, jb, je, eps2);
+    if (MODE != BF64_CHECKED) {
+        const bool again = isnan(a.x) || isnan(a.y) || isnan(a.z);
+        if (__ballot(again)) {
+            const double3 b = sum64<MODE == BF64_SOFTENED, MODE == BF64_UNCHECKED>(p, afg, jb, je, eps2);
+            if (again) a = b;
+        }
     }
-    part[wave][0][lane] = ax;
-    part[wave][1][lane] = ay;
-    part[wave][2][lane] = az;
+    part[wave][0][lane] = a.x;
+    part[wave][1][lane] = a.y;
+    part[wave][2][lane] = a.z;
     __syncthreads();
     if (wave != 0) return;
     for (int w = 1; w < BF64_WAVES; ++w) {
-        ax += part[w][0][lane];
-        ay += part[w][1][lane];
-        az += part[w][2][lane];
+        a.x += part[w][0][lane];
+        a.y += part[w][1][lane];
+        a.z += part[w][2][lane];
     }
-    if (i < n) out[size_t(blockIdx.y) * n + i] = make_double4(ax, ay, az, 0.0);
+    if (i < n) out[size_t(blockIdx.y) * n + i] = make_double4(a.x, a.y, a.z, 0.0);
 }
 
 __global__ __launch_bounds__(64) void bf64_reduce_kernel(const double4* __restrict__ partial,
@@ -557,10 +584,8 @@ int pnb_bf_accel_f64_dev(pnb_ctx* c, const double* affected, size_t n, const dou
         PNB_HIP(c, c->bf64_partial.ensure(p.splits * n * sizeof(double4)));
         dst = c->bf64_partial.as<double4>();
     }
-    // The self term and coincident pairs add d * s = 0 with s finite when the softening is not
-    // tiny (mu < 1e263 here), so only a vanishing softening needs the mask.
     const double eps2 = softening * softening;
-    auto k = checked && eps2 < 1e-30 ? bf64_kernel<true> : bf64_kernel<false>;
+    auto k = !checked ? bf64_kernel<BF64_UNCHECKED> : eps2 < 1e-300 ? bf64_kernel<BF64_CHECKED> : bf64_kernel<BF64_SOFTENED>;
     const double4* aff = reinterpret_cast<const double4*>(affected);
     for (size_t i = 0; i < n; i += BF64_SLICE) {  // one launch but for more than 2^28 bodies, never split
         const size_t cnt = std::min(n - i, BF64_SLICE);
