@@ -2508,6 +2508,23 @@ static int node_network(pnb_ctx* c) {
     });
 }
 
+// Lowest key bit by which affected particles are sorted for a tree with lvl[l] internal nodes at level l,
+// in whole digits from the top: 40 bits (13 levels), or as many as leave at most 32 internal nodes
+// below the sorted levels. Particles of one sorted cell are then in input order, which can add no more
+// than those nodes and their children to a wavefront's steps; nodes above are no smaller than the cell.
+// The digits that count where the box is far wider than the dense part: a pass at theta 0.7, a third of the
+// bodies massless, by 40 bits / so (us and million steps): 100,003 bodies with one at a distance of 10^4
+// 1,179 and 9.4 / 778 and 4.4; an uncut Plummer sphere of 1,000,000 2,350 and 37.0 / 2,253 and 32.7. A
+// digit takes 11 us of the first, 30 of the second; 100,003 bodies of two cut spheres need 40 bits, 647 us.
+static int affected_low_bit(const std::vector<uint32_t>& lvl) {
+    for (int low = 63 - 40; low > 0; low -= 8) {
+        size_t below = 0;
+        for (size_t l = size_t(63 - low) / 3 + 1; l < lvl.size(); ++l) below += lvl[l];
+        if (below <= 32) return low;
+    }
+    return 0;
+}
+
 // Orders the affected particles along the tree's key order so that each wavefront holds
 // neighbours, walks, and scatters results back to the caller's order.
 static int accel_dev(pnb_ctx* c, const float4* affected, size_t n, const float4* afg, size_t m,
@@ -2579,13 +2596,14 @@ static int accel_dev(pnb_ctx* c, const float4* affected, size_t n, const float4*
     PNB_CHECK_LAUNCH(c);
     uint64_t* sk;
     uint32_t* si;
-    // Only neighbours together: thirteen levels of the key (39 bits, five digits instead of eight)
-    // put 64 particles into cells 2^-13 of the box apart; below that any order serves, and none
-    // changes a result.
-    constexpr int AFFECTED_LOW_BIT = 23;
+    // A wavefront's steps are the nodes that any of its particles opens, so it pays to put neighbours
+    // together, as far down as the tree goes. By the whole key for the relative criterion, whose estimates
+    // are taken per wavefront and decide its results, and for a capturable build, whose later trees are
+    // not known here.
+    const int low_bit = rel || dd ? 0 : affected_low_bit(s->last_lvl);
     if (int rc = radix_sort_pairs(c, s->akeys.as<uint64_t>(), s->aidx.as<uint32_t>(),
                                   s->akeys_alt.as<uint64_t>(), s->aidx_alt.as<uint32_t>(), n, 63,
-                                  s->hist, s->bits, &sk, &si, dd, AFFECTED_LOW_BIT, affected,
+                                  s->hist, s->bits, &sk, &si, dd, low_bit, affected,
                                   s->apts.as<float4>()))
         return rc;
     return walk(c, s->apts.as<float4>(), si, n, theta, softening, out, nullptr, quad, rel, dd, list);
