@@ -13,7 +13,7 @@
 //    tiles, so the error does not grow with the affecting count;
 //  * the affecting range is split over several workgroups (j_split) whose partial sums are reduced
 //    in a fixed order, so results do not depend on scheduling;
-//  * sums of up to some ten thousand affected bodies are taken by workgroups of sixteen wavefronts
+//  * sums too small to fill the chip so (coop_pays) are taken by workgroups of sixteen wavefronts
 //    per 64 affected bodies that share the affecting ones tile by tile (bf_coop_kernel).
 // Pair semantics follow particular/src/gravity/impls/mod.rs:151-166: with `checked` a pair at
 // zero unsoftened distance contributes nothing; with softening > 0 that pair contributes
@@ -82,9 +82,10 @@ __global__ __launch_bounds__(BF_BLOCK) void bf_kernel(const float4* __restrict__
 #pragma unroll 8
             for (int j = 0; j < BF_TILE; ++j)
                 bf_body<R, MASK, false, R == 1>(LDS ? tile[j] : afg[j0 + j], xi, yi, zi, eps2, px, py, pz);
+        } else if (LDS) {
+            for (uint32_t j = 0; j < cnt; ++j) bf_body<R, MASK>(tile[j], xi, yi, zi, eps2, px, py, pz);
         } else {
-            for (uint32_t j = 0; j < cnt; ++j)
-                bf_body<R, MASK>(LDS ? tile[j] : afg[j0 + j], xi, yi, zi, eps2, px, py, pz);
+            bf_span<R, MASK, false, R == 1>(afg + j0, cnt, xi, yi, zi, eps2, px, py, pz);
         }
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -104,8 +105,8 @@ __global__ __launch_bounds__(BF_BLOCK) void bf_kernel(const float4* __restrict__
 
 // Small and middle affected counts: one workgroup of COOP_WAVES wavefronts per 64 affected bodies
 // (and per affecting range, grid.y), the wavefronts sharing the affecting bodies tile by tile
-// (coop_sum). Up to 512 affected tiles there are too few wavefronts for one of them per tile to
-// fill the chip, and each is bound by its own issue rate.
+// (coop_sum). One wavefront per affected tile would leave SIMDs idle there, and each wavefront is bound
+// by its own issue rate; coop_pays holds the sizes.
 template <bool MASK, bool SELF, int T>
 __global__ __launch_bounds__(64 * COOP_WAVES) void bf_coop_kernel(const float4* __restrict__ aff,
                                                                   uint32_t n,

@@ -15,9 +15,9 @@ inline size_t ceil_div(size_t a, size_t b) { return (a + b - 1) / b; }
 
 constexpr int BF_COOP = 2;  // variant of the workgroup-cooperative kernel (not for tuning entries)
 
-// A dispatch holds fewer than 2^32 work-items along x. The cooperative kernel takes 16 per affected
-// body (2^31 for this many), the FP64 kernel 8; the plain kernel at most one.
-constexpr size_t BF_COOP_MAX_N = size_t(1) << 27, BF64_SLICE = size_t(1) << 28;
+// A dispatch holds fewer than 2^32 work-items along x. The FP64 kernel takes 8 per affected body (2^31 for
+// this many), the cooperative kernel 16, but of fewer bodies (coop_pays); the plain kernel at most one.
+constexpr size_t BF64_SLICE = size_t(1) << 28;
 
 struct BfShape {
     int variant, per_lane, j_split;
@@ -28,13 +28,21 @@ struct BfShape {
 // x 1,000 62 / 8; 4,096 x 4,096 36 / 10; 10,000 x 8,000 45 / 30; 20,000 x 20,000 142 / 122; 30,000 x
 // 65,536 628 / 568; 45,000 x 130,000 1,695 / 1,659, without softening 1,861 / 1,862; 65,536 x 16,384
 // 321 / 308; 90,000 x 30,000 781 / 775, 864 / 868; 130,000 x 4,000 163 / 160; 130,000 x 30,000 1,098 /
-// 1,116; 400,000 x 500 75 / 67, x 2,047 305 / 247 (the plain kernel does not split below 2,048). With
-// few affecting bodies there is little to share: 256 x 100 6.0 / 8.8, 256 x 128 6.9 / 7.6, 256 x 200
-// 9.8 / 8.7; 65,536 x 200 10.0 / 9.7, 90,000 x 200 11 / 13.
+// 1,116. Below 2,048 affecting bodies the plain kernel does not split, and leaves SIMDs idle up to some
+// 800,000 affected ones; the cooperative one has at most 16 tiles of 64 to share, and fewer than eight
+// leave half of its wavefronts without one:
+//   affected   x 257        300        400        450        512        700        1,000      2,047
+//   200,000    24.6 / 24.0  27.7/26.1  34.7/31.1  38.4/31.5  46.6/32.6  59.9/43.3  85.4/58.5  175 / 115
+//   262,144    25.4 / 29.4  28.5/31.8  35.5/37.9  39.0/38.2  48.2/39.8  61.1/52.8  87.4/71.3  179 / 142
+//   400,000    37.4 / 43.8  42.2/48.0  54.3/57.3  61.1/58.2  70.4/60.7  93.9/80.5  133 / 109  276 / 218
+//   600,000    49.4 / 63.8  56.1/69.7  72.8/83.5  81.8/84.8  93.7/88.6  125 / 118  180 / 161  369 / 322
+//   1,048,576  73.9 / 109   84.3/119   110 / 142  126 / 145  142 / 151  191 / 202  273 / 275  560 / 554
+//   4,194,304  269 / 424    313 / 465  413 / 558  468 / 571  521 / 596  722 / 791  1,024/1,092 2,082/2,196
+// (without softening the same to 5 %). With few affecting bodies there is little to share: 256 x 100
+// 6.0 / 8.8, 256 x 128 6.9 / 7.6, 256 x 200 9.8 / 8.7; 65,536 x 200 8.9 / 8.7, 90,000 x 200 11 / 13.
 inline bool coop_pays(size_t n, size_t m) {
-    if (n > BF_COOP_MAX_N) return false;
     if (m <= 256) return m > 128 && n <= 65536;
-    if (m < 2048) return true;
+    if (m < 2048) return n <= 200000 || (n < 800000 && m > 448);
     return n <= 50000 || (n <= 100000 && m <= 16384) || (n <= 150000 && m <= 4096);
 }
 
@@ -54,9 +62,11 @@ inline BfShape default_shape(size_t cus, size_t n, size_t m) {
         }
         return {BF_COOP, 1, s};
     }
-    // Otherwise one body per lane and one wavefront per affected tile and range, the affecting
-    // bodies from scalar loads (from LDS for at most a tile, 65,536 x 64 4 / 9 us), the affecting
-    // range from 2,048 bodies on split into up to 64 workgroups per CU of at least one tile each, up
+    // Otherwise one body per lane and one wavefront per affected tile and range, the affecting bodies
+    // from scalar loads, or from LDS for a few of them and wavefronts too few to hide the loads (us,
+    // LDS / scalar: 100,000 x 200 10.6 / 10.8, 262,144 x 256 25.2 / 27.1, 400,000 x 256 36.9 / 37.0,
+    // 600,000 x 256 49.4 / 48.6, 4,194,304 x 64 79.5 / 76.2). The affecting
+    // range is split from 2,048 bodies on into up to 64 workgroups per CU of at least one tile each, up
     // to 256 per CU while ranges stay at 1,024 bodies (small workgroups balance the load across CUs
     // and XCDs). 1,048,576 x 65,536 16.1 ms, with four bodies per lane 17.1.
     const size_t blocks = ceil_div(n, size_t(BF_BLOCK));
@@ -65,7 +75,7 @@ inline BfShape default_shape(size_t cus, size_t n, size_t m) {
         if (per < (blocks * s * 2 <= 64 * cus ? size_t(BF_TILE) : size_t(1024))) break;
         s <<= 1;
     }
-    return {m <= 256 ? 0 : 1, 1, s};
+    return {m <= 448 && n < 400000 ? 0 : 1, 1, s};
 }
 
 struct BfPlan {

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import particular_amd as pa
-from particular_amd import _lib
+from particular_amd import _lib, metrics
 
 CSRC = os.path.join(os.path.dirname(pa.__file__), "csrc")
 
@@ -33,6 +33,9 @@ int main() {
                 const size_t covered = x * (p.shape.variant == BF_COOP ? 64 : block * p.shape.per_lane);
                 const bool all = covered >= n && size_t(p.splits) * p.chunk >= m &&
                                  size_t(p.splits - 1) * p.chunk < m;
+                // few affecting bodies leave wavefronts of the cooperative kernel without a tile: only
+                // where the affected ones cannot fill the chip by themselves
+                if (cus == 256 && m <= 448 && n >= 262144 && p.shape.variant == BF_COOP) return 2;
                 const Bf64Plan q = plan64(cus, n, m);
                 const size_t x64 = ceil_div(std::min(n, BF64_SLICE), 64);
                 const bool all64 = q.splits * q.chunk >= m && (q.splits == 1 || n <= BF64_SLICE);
@@ -54,6 +57,25 @@ def test_launches_fit_a_dispatch(tmp_path):
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", f"-I{CSRC}", str(src), "-o", str(exe)], check=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("eps", [0.0, 1e-2])
+@pytest.mark.parametrize("n,m", [(200_000, 257), (200_001, 257), (262_144, 448), (262_145, 449), (399_999, 200),
+                                 (400_000, 200), (400_001, 263), (799_999, 449), (800_000, 449),
+                                 (1_000_003, 511), (1_000_003, 513), (1_000_003, 2047), (300_001, 4103)])
+def test_few_affecting(res, orc, n, m, eps):
+    """Both sides of the borders between the kernels for few affecting bodies, and tiles that end in
+    0 to 7 of them: the bars of the other brute-force tests."""
+    rng = np.random.default_rng(m)
+    a, b = (rng.normal(size=(k, 4)).astype(np.float32) for k in (n, m))
+    b[:, 3] = rng.uniform(0.5, 1.5, m)
+    b[:7, :3] = a[:7, :3]  # pairs at zero distance add nothing
+    inter = pa.AccelerationSoftened.checked(eps) if eps else pa.Acceleration.checked()
+    got = pa.BruteForce(res, inter).compute(pa.Between(a, b))
+    idx = np.concatenate([np.arange(300), np.arange(n - 300, n)])
+    ref = orc.direct_f64(a[idx], b, softening=eps)
+    assert metrics.rms_rel(got[idx], ref) < 1e-5 and metrics.max_rel(got[idx], ref) < 1e-4
 
 
 @pytest.mark.gpu
