@@ -24,6 +24,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 namespace pnb {
@@ -327,8 +328,8 @@ __global__ __launch_bounds__(DF_BLOCK) void direct_f64_kernel(const float4* __re
 }
 
 // ---- FP64 brute force (glam::DVec3 / f64: particular/src/gravity/impls/glam.rs:234) ------------
-// The reference's scalar kernel in FP64 (impls/mod.rs:151-166). A workgroup of BF64_WAVES
-// wavefronts holds 64 affected bodies; the affecting range is split over grid.y and, inside a
+// The reference's scalar kernel in FP64 (impls/mod.rs:151-166). A workgroup of W wavefronts (plan64)
+// holds 64 affected bodies; the affecting range is split over grid.y and, inside a
 // workgroup, over its wavefronts (scalar loads), whose sums are added in wavefront order, and the
 // grid.y partial sums in order by bf64_reduce_kernel. checked: zero distance contributes nothing.
 
@@ -373,20 +374,17 @@ __device__ __forceinline__ double3 sum64(const double4 p, const double4* __restr
 // with the test in every term 1,095, with the clamp 1,005.
 constexpr int BF64_UNCHECKED = 0, BF64_CHECKED = 1, BF64_SOFTENED = 2;
 
-template <int MODE>
-__global__ __launch_bounds__(64 * BF64_WAVES) void bf64_kernel(const double4* __restrict__ aff,
-                                                               uint32_t n,
-                                                               const double4* __restrict__ afg,
-                                                               uint32_t m, uint32_t j_chunk,
-                                                               double eps2,
-                                                               double4* __restrict__ out) {
-    __shared__ double part[BF64_WAVES][3][64];
-    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+template <int MODE, int W>
+__global__ __launch_bounds__(64 * W) void bf64_kernel(
+    const double4* __restrict__ aff, uint32_t n, const double4* __restrict__ afg, uint32_t m,
+    uint32_t j_chunk, double eps2, double4* __restrict__ out) {
+    __shared__ double part[W][3][64];
+    const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)) : 0;
     const int lane = threadIdx.x & 63;
     const uint32_t i = blockIdx.x * 64 + lane;
     const double4 p = aff[i < n ? i : n - 1];
     const uint32_t b0 = blockIdx.y * j_chunk, b1 = min(m, b0 + j_chunk);
-    const uint32_t per = (b1 - b0 + BF64_WAVES - 1) / BF64_WAVES;
+    const uint32_t per = (b1 - b0 + W - 1) / W;
     const uint32_t jb = min(b1, b0 + wave * per), je = min(b1, jb + per);
     double3 a = sum64<MODE == BF64_CHECKED, false>(p, afg, jb, je, eps2);
     if (MODE != BF64_CHECKED) {
@@ -396,15 +394,17 @@ __global__ __launch_bounds__(64 * BF64_WAVES) void bf64_kernel(const double4* __
             if (again) a = b;
         }
     }
-    part[wave][0][lane] = a.x;
-    part[wave][1][lane] = a.y;
-    part[wave][2][lane] = a.z;
-    __syncthreads();
-    if (wave != 0) return;
-    for (int w = 1; w < BF64_WAVES; ++w) {
-        a.x += part[w][0][lane];
-        a.y += part[w][1][lane];
-        a.z += part[w][2][lane];
+    if (W > 1) {
+        part[wave][0][lane] = a.x;
+        part[wave][1][lane] = a.y;
+        part[wave][2][lane] = a.z;
+        __syncthreads();
+        if (wave != 0) return;
+        for (int w = 1; w < W; ++w) {
+            a.x += part[w][0][lane];
+            a.y += part[w][1][lane];
+            a.z += part[w][2][lane];
+        }
     }
     if (i < n) out[size_t(blockIdx.y) * n + i] = make_double4(a.x, a.y, a.z, 0.0);
 }
@@ -580,17 +580,24 @@ int pnb_bf_accel_f64_dev(pnb_ctx* c, const double* affected, size_t n, const dou
     double4* dst = o;
     // Inside a caller's capture one range and no scratch: nothing can be allocated there, and a later
     // call that needs more would free the memory that the graph goes on using.
-    if (p.splits > 1 && stream_capturing(c)) p = {1, uint32_t(m)};
+    if (p.splits > 1 && stream_capturing(c)) p = {BF64_WAVES, 1, uint32_t(m)};
     if (p.splits > 1) {
         PNB_HIP(c, c->bf64_partial.ensure(p.splits * n * sizeof(double4)));
         dst = c->bf64_partial.as<double4>();
     }
     const double eps2 = softening * softening;
-    auto k = !checked ? bf64_kernel<BF64_UNCHECKED> : eps2 < 1e-300 ? bf64_kernel<BF64_CHECKED> : bf64_kernel<BF64_SOFTENED>;
+    const auto pick = [&](auto w) {
+        constexpr int W = decltype(w)::value;
+        return !checked         ? bf64_kernel<BF64_UNCHECKED, W>
+               : eps2 < 1e-300 ? bf64_kernel<BF64_CHECKED, W>
+                                : bf64_kernel<BF64_SOFTENED, W>;
+    };
+    const auto k = p.waves == 1 ? pick(std::integral_constant<int, 1>{})
+                                : pick(std::integral_constant<int, BF64_WAVES>{});
     const double4* aff = reinterpret_cast<const double4*>(affected);
     for (size_t i = 0; i < n; i += BF64_SLICE) {  // one launch but for more than 2^28 bodies, never split
         const size_t cnt = std::min(n - i, BF64_SLICE);
-        k<<<dim3(div_up(cnt, 64), unsigned(p.splits)), 64 * BF64_WAVES, 0, c->stream>>>(
+        k<<<dim3(div_up(cnt, 64), unsigned(p.splits)), 64 * p.waves, 0, c->stream>>>(
             aff + i, uint32_t(cnt), reinterpret_cast<const double4*>(affecting), uint32_t(m), p.chunk, eps2,
             dst + i);
         PNB_CHECK_LAUNCH(c);

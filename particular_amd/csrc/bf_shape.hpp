@@ -102,20 +102,24 @@ inline unsigned bf_grid_x(const BfShape& sh, size_t n) {
     return unsigned(ceil_div(n, sh.variant == BF_COOP ? size_t(64) : size_t(BF_BLOCK) * sh.per_lane));
 }
 
-// The FP64 sum's affecting ranges: workgroups until the launch holds about four rounds of wavefronts
-// (32 per CU), with at least 32 affecting bodies for each of a workgroup's wavefronts.
+// The FP64 sum: wavefronts per 64 affected bodies, and affecting ranges: workgroups until the launch holds
+// about four rounds of wavefronts (32 per CU), with at least 32 affecting bodies for each of a
+// workgroup's wavefronts. Up to eight affecting bodies one wavefront takes all: split, each has one or
+// none (1,000,000 x 1 15.9 us, 10.9 so; x 8 20.4, 11.9), and adding one after the other rounds less often.
 struct Bf64Plan {
+    int waves;
     size_t splits;
     uint32_t chunk;
 };
 
 inline Bf64Plan plan64(size_t cus, size_t n, size_t m) {
+    if (m <= BF64_WAVES) return {1, 1, m > 0 ? uint32_t(m) : 1};
     const size_t blocks = ceil_div(n, 64);
     size_t splits = 1;
     while (splits < 64 && blocks * splits * BF64_WAVES < 128 * cus && m / (splits * 2) >= 32 * BF64_WAVES)
         splits <<= 1;
-    const size_t chunk = m > splits ? ceil_div(m, splits) : 1;
-    return {m > chunk ? ceil_div(m, chunk) : 1, uint32_t(chunk)};
+    const size_t chunk = ceil_div(m, splits);
+    return {BF64_WAVES, ceil_div(m, chunk), uint32_t(chunk)};
 }
 
 }  // namespace pnb

@@ -30,7 +30,7 @@ def errors(res, eps, m, reps):
 
 
 @pytest.mark.parametrize("eps", [0.0, 0.01, 0.3])
-@pytest.mark.parametrize("m,reps", [(1, 64), (100, 8)])
+@pytest.mark.parametrize("m,reps", [(1, 64), (2, 64), (8, 64), (9, 32), (100, 8)])
 def test_as_exact_as_ieee(res, eps, m, reps):
     """Root mean square error no larger than that of a square root, a product and a division per term;
     5 % for the sample (its own spread is below 1 %) and for the fused additions either side makes."""
