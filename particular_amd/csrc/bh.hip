@@ -132,6 +132,7 @@ struct BhState {
     DevBuf keys, keys_alt, idx, idx_alt, sp, lcp, cnt, ip, key2, rec, sums, level, width;
     DevBuf skipv;            // per node: the skip pointer alone (the bottom-up pass's child walk)
     DevBuf kids;             // per internal node: its children's indices (the batched walk)
+    bool has_kids = false;   // the last build wrote them
     DevBuf ilist;            // internal nodes grouped by level (bottom-up pass)
     DevBuf lvl;              // padded per-level counts and list cursors (2 x LVL_SLOTS lines)
     DevBuf mom, quad, desc;  // second moments (FP64), normalised quadrupoles, child shares
@@ -1813,11 +1814,39 @@ __global__ __launch_bounds__(256) void bh_walk_kernel(const NodeRec* __restrict_
 
 // ---- host side --------------------------------------------------------------------------------
 
+// Particles per wavefront of the batched walk (bh_list_kernel), or 0 for the stackless one.
+// It pays while the stackless walk's wavefronts are too few to hide its latency; with more, the
+// work per particle decides, and a batched wavefront has fewer particles to share its rounds.
+// Walk at theta = 0.5, stackless / 4 / 16 particles per wavefront (us): plain, 1,000 bodies 71 /
+// 47 / 73; 4,096: 182 / 106 / 159; 20,000: 379 / 246 / 282; 30,000: - / 336 / 310; 50,000: 601 / 540
+// / 477; 100,003: 750 / 1,043 / 805. Corrected (no ordered sum, so nearly as cheap as plain):
+// 1,000: 100 / 45 / 99; 4,096: 321 / 100 / 226; 20,000: 739 / 241 / 416; 100,003: 1,605 / 1,047 /
+// 1,192; 262,144: 2,357 / 2,938 / 3,183.
+// PNB_WALK_LANES and PNB_WIDE_WALK name forms of the stackless walk.
+static int list_lanes(size_t n, bool mlp) {
+    if (std::getenv("PNB_WALK_LANES") || std::getenv("PNB_WIDE_WALK")) return 0;
+    if (mlp) return n <= 160000 ? 4 : 0;
+    return n <= 20000 ? 4 : n <= 75000 ? 16 : 0;
+}
+
+// Whether the child table of a tree of `nodes` nodes (32 bytes each) is worth writing for the batched walk
+// of n particles. It costs some 18 us per million nodes and saves more the more particles walk; up to 64
+// the stackless walk has only one wavefront. A pass at theta 0.5, without the table / with it (us),
+// uniform cubes: 1,000 of 1M bodies (1.4M nodes) 896 / 925, of 16M (23M) 6,164 / 6,470, of 60M (85M) 22,370
+// / 23,790; 8,000 of 16M 6,583 / 6,499, of 60M 22,900 / 23,840; 30,000 of 60M 24,570 / 25,150; 70,000 of
+// 60M 27,680 / 25,950; 64 of 60M 43,200 / 23,800, 1 of 60M 22,200 / 23,600. Plummer spheres: 1,000 of 1M 1,250 / 1,100, of 16M
+// 6,520 / 6,600. Trees of 2^27 nodes or more are not walked so.
+static bool children_pay(size_t nodes, size_t n) {
+    return nodes + 1 < (size_t(1) << 27) && (nodes <= (n <= 64 ? 20000000 : 2500) * n || nodes <= 2000000);
+}
+
+// list_n: the particles that the batched walk would take over this tree (0: none).
 static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = false,
-                      bool moments = false, bool children = false) {
+                      bool moments = false, size_t list_n = 0) {
     if (!c->bh) c->bh = new BhState();
     BhState* s = c->bh;
     s->built = false;
+    s->has_kids = false;
     s->has_moments = false;
     s->rrec_ok = false;
     s->dd_last = false;
@@ -1900,10 +1929,10 @@ static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = fa
         NodeRec* rec = s->rec.as<NodeRec>();
         PNB_HIP(c, s->skipv.ensure(size_t(total) * sizeof(uint32_t)));
         uint32_t* skipv = s->skipv.as<uint32_t>();
-        uint32_t* kids = nullptr;
-        if (children) {
-            PNB_HIP(c, s->kids.ensure(size_t(total) * 8 * sizeof(uint32_t)));
+        uint32_t* kids = nullptr;  // without memory for them the walk is the stackless one
+        if (list_n && children_pay(total, list_n) && s->kids.ensure(size_t(total) * 32) == hipSuccess) {
             kids = s->kids.as<uint32_t>();
+            s->has_kids = true;
         }
         bh_node_kernel<<<g, 256, 0, c->stream>>>(sk, s->sp.as<float4>(), lcp, s->ip.as<int>(),
                                                  cnt, m, info, rec, s->sums.as<NodeSums>(),
@@ -1985,9 +2014,11 @@ static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = fa
 // Capacities of a capturable build from an ordinary build of the same size (its node count and
 // depth known on the host): a quarter more nodes and 8 more levels, so that later trees of
 // similar inputs fit.
-static int dd_size(pnb_ctx* c, size_t m, bool mlp, bool children) {
+static int dd_size(pnb_ctx* c, size_t m, size_t n, bool mlp) {
     BhState* s = c->bh;
     const size_t cap = s->nodes + s->nodes / 4 + 1024;
+    // these sizes serve the n particles and the tree's own bodies
+    const bool children = (list_lanes(n, mlp) && children_pay(cap, n)) || (list_lanes(m, mlp) && children_pay(cap, m));
     if (cap + 1 >= (size_t(1) << 27))
         return fail(c, PNB_E_ARG, "capturable Barnes-Hut trees are limited to 2^27 nodes");
     PNB_HIP(c, s->rec.ensure((cap + 1) * sizeof(NodeRec)));
@@ -1995,7 +2026,7 @@ static int dd_size(pnb_ctx* c, size_t m, bool mlp, bool children) {
     PNB_HIP(c, s->level.ensure(cap));
     PNB_HIP(c, s->width.ensure(cap * sizeof(float)));
     PNB_HIP(c, s->skipv.ensure(cap * sizeof(uint32_t)));
-    if (children) PNB_HIP(c, s->kids.ensure(cap * 8 * sizeof(uint32_t)));
+    s->dd_kids = children && s->kids.ensure(cap * 32) == hipSuccess;
     PNB_HIP(c, s->ilist.ensure(cap * sizeof(uint32_t)));
     if (mlp) {  // the learned correction's node data and walk entries
         PNB_HIP(c, s->mom.ensure(cap * sizeof(NodeMoments)));
@@ -2005,7 +2036,6 @@ static int dd_size(pnb_ctx* c, size_t m, bool mlp, bool children) {
         PNB_HIP(c, s->oh.ensure((cap + 1) * sizeof(OctH)));
     }
     s->dd_mlp = mlp;
-    s->dd_kids = children;
     s->dd_cap = cap;
     s->dd_levels = std::min(std::max(s->max_level, 0) + 8, MAX_LEVEL + 1);
     s->dd_plan = s->last_lvl;
@@ -2019,6 +2049,7 @@ static int dd_size(pnb_ctx* c, size_t m, bool mlp, bool children) {
 static int build_tree_dd(pnb_ctx* c, const float4* afg, size_t m, bool moments, bool children) {
     BhState* s = c->bh;
     s->built = false;
+    s->has_kids = children;
     s->has_moments = false;
     s->rrec_ok = false;
     s->m = m;
@@ -2292,21 +2323,6 @@ static uint32_t walk_lanes(const pnb_ctx* c, size_t n) {
     return lanes;
 }
 
-// Particles per wavefront of the batched walk (bh_list_kernel), or 0 for the stackless one.
-// It pays while the stackless walk's wavefronts are too few to hide its latency; with more, the
-// work per particle decides, and a batched wavefront has fewer particles to share its rounds.
-// Walk at theta = 0.5, stackless / 4 / 16 particles per wavefront (us): plain, 1,000 bodies 71 /
-// 47 / 73; 4,096: 182 / 106 / 159; 20,000: 379 / 246 / 282; 30,000: - / 336 / 310; 50,000: 601 / 540
-// / 477; 100,003: 750 / 1,043 / 805. Corrected (no ordered sum, so nearly as cheap as plain):
-// 1,000: 100 / 45 / 99; 4,096: 321 / 100 / 226; 20,000: 739 / 241 / 416; 100,003: 1,605 / 1,047 /
-// 1,192; 262,144: 2,357 / 2,938 / 3,183.
-// PNB_WALK_LANES and PNB_WIDE_WALK name forms of the stackless walk.
-static int list_lanes(size_t n, bool mlp) {
-    if (std::getenv("PNB_WALK_LANES") || std::getenv("PNB_WIDE_WALK")) return 0;
-    if (mlp) return n <= 160000 ? 4 : 0;
-    return n <= 20000 ? 4 : n <= 75000 ? 16 : 0;
-}
-
 // quad: add the learned correction (the per-node moments in s->qh). rel: the relative criterion
 // in addition to the geometric one: an estimate pass (plain walk at s->rel_theta_est) gives
 // alpha |a~| per particle or, by default, per wavefront at the centroid of its 64 particles; then
@@ -2422,7 +2438,7 @@ static int walk(pnb_ctx* c, const float4* pts, const uint32_t* perm, size_t n, f
         } else if (rows) {
             launch_walk<WALK_ROWS, false>(wide, grid, c->stream, nr, total, pts, perm, uint32_t(n),
                                           theta2, eps2, out, info, *rows, nullptr);
-        } else if (list && total > 0 && !wide) {
+        } else if (list && total > 0 && s->has_kids) {
             auto go = [&](auto k) {
                 k<<<div_up(n, size_t(list)), 64, 0, c->stream>>>(
                     nr, s->kids.as<uint4>(), total, pts, perm, uint32_t(n), theta2, eps2, out, info,
@@ -2543,7 +2559,7 @@ static int accel_dev(pnb_ctx* c, const float4* affected, size_t n, const float4*
                                       "PNB_BH_RELATIVE");
         BhState* s = c->bh;
         const bool sized = s->dd_cap > 0 && s->dd_m == m && s->dd_mlp == mlp &&
-                           (s->dd_kids || !list) && ((affected == afg && n == m) || s->dd_n == n);
+                           ((affected == afg && n == m) || s->dd_n == n);
         if (sized) {
             dd = true;
         } else if (stream_capturing(c)) {
@@ -2552,6 +2568,7 @@ static int accel_dev(pnb_ctx* c, const float4* affected, size_t n, const float4*
                                         "buffers)");
         }
     }
+    const auto dd_children = [&] { return list && c->bh->dd_kids && c->bh->kids.cap >= c->bh->dd_cap * 32; };
     // inside an outside capture: no events on the stream
     const bool was_capturing = c->capturing;
     if (dd) c->capturing = c->capturing || stream_capturing(c);
@@ -2561,17 +2578,17 @@ static int accel_dev(pnb_ctx* c, const float4* affected, size_t n, const float4*
         ~Restore() { c->capturing = v; }
     } restore{c, was_capturing};
     if (dd) {
-        if (int rc = build_tree_dd(c, afg, m, mlp, list != 0)) return rc;
+        if (int rc = build_tree_dd(c, afg, m, mlp, dd_children())) return rc;
     } else {
-        if (int rc = build_tree(c, afg, m, ref_com, mlp, list != 0)) return rc;
+        if (int rc = build_tree(c, afg, m, ref_com, mlp, list && !c->bh->dd_mode ? n : 0)) return rc;
         if (c->bh->dd_mode) {
             // The sizing call of a capturable build: capacities from this tree, then the tree
             // again in the sized buffers (growing a buffer discards its contents, so the tree
             // just built may be gone), built the capturable way.
-            if (int rc = dd_size(c, m, mlp, list != 0)) return rc;
+            if (int rc = dd_size(c, m, n, mlp)) return rc;
             c->bh->dd_n = n;
             dd = true;
-            if (int rc = build_tree_dd(c, afg, m, mlp, list != 0)) return rc;
+            if (int rc = build_tree_dd(c, afg, m, mlp, dd_children())) return rc;
         }
     }
     BhState* s = c->bh;
