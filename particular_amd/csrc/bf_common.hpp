@@ -40,7 +40,9 @@ __device__ __forceinline__ void bf_body(const float4 q, const float (&xi)[R], co
     }
 }
 
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
+// Four bodies; aligned as the arrays are (a slice of a tensor, an ensemble's system), not as its size is.
+typedef float f32x16_t __attribute__((ext_vector_type(16), aligned(16)));
+static_assert(alignof(f32x16_t) == alignof(float4), "read at any body of an array");
 
 // T affecting bodies at a wave-uniform address, four per scalar load, the next four requested before
 // the present four are summed: one by one, each body is five scalar instructions, a load and a wait.

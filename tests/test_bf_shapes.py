@@ -79,6 +79,19 @@ def test_few_affecting(res, orc, n, m, eps):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("first", [1, 2, 3, 5])
+@pytest.mark.parametrize("n,m", [(300, 1100), (5000, 4099), (300_000, 2500)])
+def test_slices(res, first, n, m):
+    """Arrays that begin at any body of a larger one: the bits of a copy."""
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(n)
+    a, b = (torch.randn((k + 8, 4), generator=g, device="cuda")[first : first + k] for k in (n, m))
+    alg = pa.BruteForce(res, pa.AccelerationSoftened.checked(1e-2))
+    assert torch.equal(alg.compute(pa.Between(a, b)), alg.compute(pa.Between(a.clone(), b.clone())))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype,n,m", [("f32", (1 << 28) + 67, 300), ("f64", (1 << 29) + 67, 3)])
 def test_most_affected(res, dtype, n, m):
     """Counts whose cooperative (f32) and single (FP64) launch would hold 2^32 work-items or more.
