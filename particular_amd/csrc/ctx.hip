@@ -75,8 +75,13 @@ int stage_in(pnb_ctx* c, DevBuf& dst, const void* src, size_t bytes, int slot) {
         return PNB_OK;
     }
     if (!c->pin_in) PNB_HIP(c, hipHostMalloc(&c->pin_in, 2 * HOST_STAGE));
+    if (c->staging & (1u << slot)) {  // left by a call that failed, perhaps on another stream
+        PNB_HIP(c, hipDeviceSynchronize());
+        c->staging = 0;
+    }
     char* pin = static_cast<char*>(c->pin_in) + slot * HOST_STAGE;
     std::memcpy(pin, src, bytes);
+    c->staging |= 1u << slot;
     stage_kernel<<<div_up(bytes / 16, 256), 256, 0, c->stream>>>(
         reinterpret_cast<const uint4*>(pin), bytes / 16, dst.as<uint4>());
     PNB_CHECK_LAUNCH(c);
@@ -97,6 +102,7 @@ int stage_out(pnb_ctx* c, DevBuf& dev, size_t bytes, void** where) {
 int stage_done(pnb_ctx* c, void* out, const void* where, size_t bytes) {
     if (where != c->pin_out) return stage_fetch(c, {{out, where, bytes}});
     PNB_HIP(c, hipStreamSynchronize(c->stream));
+    c->staging = 0;
     std::memcpy(out, where, bytes);
     return PNB_OK;
 }
@@ -119,6 +125,7 @@ int stage_fetch(pnb_ctx* c, std::initializer_list<Fetch> parts) {
         pin += f.bytes;
     }
     PNB_HIP(c, hipStreamSynchronize(c->stream));
+    c->staging = 0;
     if (!pinned) return PNB_OK;
     pin = static_cast<char*>(c->pin_out);
     for (const Fetch& f : parts) {

@@ -50,6 +50,7 @@ struct pnb_ctx {
     pnb::DevBuf bf_partial, bf64_partial;
     pnb::DevBuf scan_tmp;
     void *pin_in = nullptr, *pin_out = nullptr;  // pinned: stage_in's two slots, stage_out's one
+    unsigned staging = 0;  // pin_in's slots that a kernel may still read: set until the stream was waited for
     uint32_t* pin_count = nullptr;               // pinned: split_affecting's count
     pnb::DevBuf pairs_part;  // pair brute force: one partial per body and super-tile or range
     // device address of the allocation-free entry point's static scratch on this device
@@ -88,8 +89,8 @@ bool stream_capturing(pnb_ctx* c);
 // when out has room for n + 1 entries and with_total is set.
 int scan_u32(pnb_ctx* c, const uint32_t* in, uint32_t* out, size_t n, bool with_total);
 
-// Stable compaction of the affecting particles (mu != 0) of `particles` into `dst`; writes the
-// count to *m_dev (device) and returns it in *m_host. Ordered::new (storage.rs:85-95).
+// Stable compaction of the affecting particles (mu != 0) of `particles` into `dst`; waits for the stream
+// and returns their count in *m_host. Ordered::new (storage.rs:85-95).
 int split_affecting(pnb_ctx* c, const float4* particles, size_t n, float4* dst, uint32_t* m_host);
 
 // Host arrays of 16-byte records in and out, for the entry points that take them. Up to HOST_STAGE bytes pass through

@@ -73,3 +73,21 @@ def test_f64_graph_holds_no_scratch(res):
         assert torch.equal(out, first)
     term = torch.linalg.vector_norm(want[:, :3], dim=1)
     assert float(((first - want).abs().max(1).values / term).median()) <= 1e-12
+
+
+def test_host_staging_after_a_failed_call():
+    """Host arrays staged right after a call that failed behind its own staging, on another stream: the
+    sums of the new arrays."""
+    rng = np.random.default_rng(4)
+    p, q = (np.abs(rng.normal(size=(60_000, 4))).astype(np.float32) for _ in range(2))
+    with pa.HipResources(0) as fresh, pa.HipResources(0) as res:
+        alg, corrected = (pa.BarnesHut(res, 0.7, pa.Acceleration.checked(), mlp=m) for m in (False, True))
+        want = pa.BarnesHut(fresh, 0.7, pa.Acceleration.checked()).compute(q)
+        streams = [torch.cuda.Stream() for _ in range(2)]
+        for k in range(20):
+            res.set_stream(streams[k % 2].cuda_stream)
+            with pytest.raises(pa.PnbError):  # no network
+                corrected.compute(p)
+            res.set_stream(streams[1 - k % 2].cuda_stream)
+            np.testing.assert_array_equal(alg.compute(q), want)
+        res.reset_stream()
