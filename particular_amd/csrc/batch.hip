@@ -230,8 +230,8 @@ static int tuned_per_lane(const BatchState* s, size_t n) {
     return r;
 }
 
-// Bodies per lane of a system's items. Untuned: two, one for systems with at most half a
-// workgroup's lanes.
+// The queue's items. Untuned, and tuned to one body per lane throughout, workgroups share them, one body
+// per lane; otherwise an item is 64 bodies times its system's tuning entry (one without an entry).
 static int build_items(pnb_ctx* c, BatchState* s) {
     std::vector<BatchItem> items;
     s->interactions = 0;
