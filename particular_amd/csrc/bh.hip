@@ -1822,10 +1822,19 @@ __global__ __launch_bounds__(256) void bh_walk_kernel(const NodeRec* __restrict_
 // / 477; 100,003: 750 / 1,043 / 805. Corrected (no ordered sum, so nearly as cheap as plain):
 // 1,000: 100 / 45 / 99; 4,096: 321 / 100 / 226; 20,000: 739 / 241 / 416; 100,003: 1,605 / 1,047 /
 // 1,192; 262,144: 2,357 / 2,938 / 3,183.
+// A corrected walk of wider angles has fewer steps to wait for, and its border falls with the angle. Whole
+// passes, batched over stackless, quadrupole network, two Plummer spheres / cube / disc:
+//   theta    0.3           0.45          0.6           0.7           0.8           0.9           1.1
+//   20,000   .46/.46/.68   .58/.68/.86   .75/.90/.97   .83/1.0/1.0   .90/1.1/1.0   .97/1.1/1.1   1.0/1.1/1.1
+//   40,000   .50/.51/.73   .64/.73/.92   .80/.99/1.1   .93/1.1/1.1   .99/1.2/1.2   1.1/1.3/1.2   1.2/1.4/1.3
+//   65,000   .59/.55/.80   .66/.81/1.0   .87/1.2/1.2   .99/1.3/1.3   1.1/1.3/1.3   1.2/1.4/1.4   1.3/1.5/1.4
+//   100,000  .77/.60/.94   .82/.87/1.2   .98/1.3/1.4   1.2/1.5/1.5   1.3/1.6/1.6   1.4/1.8/1.7   1.6/1.9/1.7
+//   160,000  1.1/.75/1.1   .98/1.0/1.4   1.1/1.5/1.6   1.4/1.7/1.8   1.5/1.9/1.9   1.7/2.0/1.9   1.9/2.3/2.0
+// Plain walks are even around their borders at every angle (0.86 to 1.2).
 // PNB_WALK_LANES and PNB_WIDE_WALK name forms of the stackless walk.
-static int list_lanes(size_t n, bool mlp) {
+static int list_lanes(size_t n, bool mlp, float theta) {
     if (std::getenv("PNB_WALK_LANES") || std::getenv("PNB_WIDE_WALK")) return 0;
-    if (mlp) return n <= 160000 ? 4 : 0;
+    if (mlp) return n <= 10000 || (n <= 130000 && float(n) * theta * theta * std::sqrt(theta) <= 14000.f) ? 4 : 0;
     return n <= 20000 ? 4 : n <= 75000 ? 16 : 0;
 }
 
@@ -2014,11 +2023,12 @@ static int build_tree(pnb_ctx* c, const float4* afg, size_t m, bool ref_com = fa
 // Capacities of a capturable build from an ordinary build of the same size (its node count and
 // depth known on the host): a quarter more nodes and 8 more levels, so that later trees of
 // similar inputs fit.
-static int dd_size(pnb_ctx* c, size_t m, size_t n, bool mlp) {
+static int dd_size(pnb_ctx* c, size_t m, size_t n, bool mlp, float theta) {
     BhState* s = c->bh;
     const size_t cap = s->nodes + s->nodes / 4 + 1024;
     // these sizes serve the n particles and the tree's own bodies
-    const bool children = (list_lanes(n, mlp) && children_pay(cap, n)) || (list_lanes(m, mlp) && children_pay(cap, m));
+    const bool children = (list_lanes(n, mlp, theta) && children_pay(cap, n)) ||
+                          (list_lanes(m, mlp, theta) && children_pay(cap, m));
     if (cap + 1 >= (size_t(1) << 27))
         return fail(c, PNB_E_ARG, "capturable Barnes-Hut trees are limited to 2^27 nodes");
     PNB_HIP(c, s->rec.ensure((cap + 1) * sizeof(NodeRec)));
@@ -2552,7 +2562,7 @@ static int accel_dev(pnb_ctx* c, const float4* affected, size_t n, const float4*
         return fail(c, PNB_E_STATE, "PNB_BH_MLP needs an initialised MLP (pnb_mlp_init)");
     if (!c->bh) c->bh = new BhState();
     bool dd = false;
-    const int list = rel ? 0 : list_lanes(n, mlp);
+    const int list = rel ? 0 : list_lanes(n, mlp, theta);
     if (c->bh->dd_mode) {
         if (ref_com || rel)
             return fail(c, PNB_E_ARG, "capturable Barnes-Hut takes neither PNB_BH_REF_COM nor "
@@ -2585,7 +2595,7 @@ static int accel_dev(pnb_ctx* c, const float4* affected, size_t n, const float4*
             // The sizing call of a capturable build: capacities from this tree, then the tree
             // again in the sized buffers (growing a buffer discards its contents, so the tree
             // just built may be gone), built the capturable way.
-            if (int rc = dd_size(c, m, n, mlp)) return rc;
+            if (int rc = dd_size(c, m, n, mlp, theta)) return rc;
             c->bh->dd_n = n;
             dd = true;
             if (int rc = build_tree_dd(c, afg, m, mlp, dd_children())) return rc;

@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import particular_amd as pa
-from particular_amd import workloads
+from particular_amd import learned, metrics, workloads
 from tests.test_bh_graph_gpu import capture
 
 pytestmark = pytest.mark.gpu
@@ -65,4 +65,54 @@ def test_capture_of_the_trees_own_bodies():
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(got, own)
+        res.bh_check()
+
+
+@pytest.mark.parametrize("params", ["quadrupole_params", "octupole_params"])
+@pytest.mark.parametrize("n,theta,batched", [(10_000, 1.1, True), (10_001, 1.2, False), (50_000, 0.6, True),
+                                             (51_000, 0.6, False), (130_000, 0.3, True), (130_001, 0.3, False)])
+def test_corrected_borders(monkeypatch, params, n, theta, batched):
+    """Both sides of the border between the walks, which falls with the angle: the same accepted nodes,
+    sums to rounding (the bar the stackless walk's own widths are held to), and the walk it should be
+    (the batched one adds the same terms in other groups; the stackless one's bits repeat)."""
+    p = workloads.two_plummer_case(n, seed=n).particles
+    with pa.HipResources(0) as res:
+        learned.init(res, 0)
+        learned.set_params(res, getattr(learned, params)())
+        alg = pa.BarnesHut(res, theta, pa.Acceleration.checked(), mlp=True)
+        got, counted = alg.compute(p), pa.bh_stats(res)[1]
+        steps = pa.bh_stats(res)[0]
+        lanes = 64
+        while lanes > 1 and -(-n // lanes) < 2048:
+            lanes //= 2
+        monkeypatch.setenv("PNB_WALK_LANES", str(lanes))
+        ref = alg.compute(p)
+        assert counted == pa.bh_stats(res)[1]
+        assert (steps == pa.bh_stats(res)[0]) != batched
+    if not batched:
+        np.testing.assert_array_equal(got, ref)
+    row = np.linalg.norm(got - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert metrics.rms_rel(got, ref) < 1e-6 and row.max() < 1e-5
+
+
+def test_capture_at_another_angle():
+    """Sized at an angle without a child table, a capture at one that would want it is taken."""
+    d = torch.from_numpy(workloads.two_plummer_case(60_000, seed=2).particles).cuda()
+    with pa.HipResources(0) as res:
+        learned.init(res, 0)
+        learned.set_params(res, learned.quadrupole_params())
+        wide, narrow = (pa.BarnesHut(res, th, pa.Acceleration.checked(), mlp=True) for th in (0.9, 0.4))
+        res.set_bh_capturable(True)
+        wide.compute(pa.Between(d, d))  # sizes
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with capture(graph):
+            got = narrow.compute(pa.Between(d, d))
+        for _ in range(2):
+            eager = narrow.compute(pa.Between(d, d))
+            torch.cuda.synchronize()
+            got.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(got, eager) and bool(torch.isfinite(got).all())
         res.bh_check()
