@@ -339,27 +339,29 @@ __global__ __launch_bounds__(DF_BLOCK) void direct_f64_kernel(const float4* __re
 // roundings, as an IEEE root, product and division have. y^2 takes the correction: it stays finite where
 // the result overflows, which has to give infinity.
 // An infinite r2 (y = 0) gives 0; with ZERO, a vanishing r2 infinity, as a division by it does.
+// c1, c2: 3/2 and 15/8, held by the caller in vector registers (a literal is moved there for every term).
 template <bool ZERO>
-__device__ __forceinline__ double cubed64(double mu, double r2) {
+__device__ __forceinline__ double cubed64(double mu, double r2, double c1, double c2) {
     const double y = __longlong_as_double(__double_as_longlong(__builtin_amdgcn_rsq(r2)) & ~0x7ffffffll);
     const double y2 = y * y;
     double r = fmin(r2, 1.7976931348623157e308);
     if (ZERO) r = fmax(r, 4.9406564584124654e-324);
     const double e = fma(-r, y2, 1.0);
-    return (mu * y) * fma(y2 * e, fma(e, 1.875, 1.5), y2);
+    return (mu * y) * fma(y2 * e, fma(e, c2, c1), y2);
 }
 
 // One lane's share, bodies jb .. je of afg. CHECK tests the unsoftened distance; ZERO as above.
 template <bool CHECK, bool ZERO>
 __device__ __forceinline__ double3 sum64(const double4 p, const double4* __restrict__ afg, uint32_t jb,
                                          uint32_t je, double eps2) {
-    double ax = 0.0, ay = 0.0, az = 0.0;
+    double ax = 0.0, ay = 0.0, az = 0.0, c1 = 1.5, c2 = 1.875;
+    asm volatile("" : "+v"(c1), "+v"(c2));
 #pragma unroll 4
     for (uint32_t j = jb; j < je; ++j) {
         const double4 q = afg[j];  // wave-uniform: a scalar load
         const double dx = q.x - p.x, dy = q.y - p.y, dz = q.z - p.z;
         const double d2 = fma(dx, dx, fma(dy, dy, CHECK ? dz * dz : fma(dz, dz, eps2)));
-        double s = cubed64<ZERO>(q.w, CHECK ? d2 + eps2 : d2);
+        double s = cubed64<ZERO>(q.w, CHECK ? d2 + eps2 : d2, c1, c2);
         if (CHECK) s = d2 == 0.0 ? 0.0 : s;
         ax = fma(dx, s, ax);
         ay = fma(dy, s, ay);
