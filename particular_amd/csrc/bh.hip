@@ -1822,8 +1822,10 @@ __global__ __launch_bounds__(256) void bh_walk_kernel(const NodeRec* __restrict_
 // / 477; 100,003: 750 / 1,043 / 805. Corrected (no ordered sum, so nearly as cheap as plain):
 // 1,000: 100 / 45 / 99; 4,096: 321 / 100 / 226; 20,000: 739 / 241 / 416; 100,003: 1,605 / 1,047 /
 // 1,192; 262,144: 2,357 / 2,938 / 3,183.
-// A corrected walk of wider angles has fewer steps to wait for, and its border falls with the angle. Whole
-// passes, batched over stackless, quadrupole network, two Plummer spheres / cube / disc:
+// A corrected walk of wider angles has fewer steps to wait for, and its border falls with the angle: up to
+// n theta = 47,000 no pass over any of these sets takes longer than it did before the stackless walk was
+// last sped up (0.75 to 0.85 of that). Whole passes, batched over stackless, quadrupole network, two
+// Plummer spheres / cube / disc:
 //   theta    0.3           0.45          0.6           0.7           0.8           0.9           1.1
 //   20,000   .46/.46/.68   .58/.68/.86   .75/.90/.97   .83/1.0/1.0   .90/1.1/1.0   .97/1.1/1.1   1.0/1.1/1.1
 //   40,000   .50/.51/.73   .64/.73/.92   .80/.99/1.1   .93/1.1/1.1   .99/1.2/1.2   1.1/1.3/1.2   1.2/1.4/1.3
@@ -1834,7 +1836,7 @@ __global__ __launch_bounds__(256) void bh_walk_kernel(const NodeRec* __restrict_
 // PNB_WALK_LANES and PNB_WIDE_WALK name forms of the stackless walk.
 static int list_lanes(size_t n, bool mlp, float theta) {
     if (std::getenv("PNB_WALK_LANES") || std::getenv("PNB_WIDE_WALK")) return 0;
-    if (mlp) return n <= 10000 || (n <= 130000 && float(n) * theta * theta * std::sqrt(theta) <= 14000.f) ? 4 : 0;
+    if (mlp) return n <= 40000 || (n <= 150000 && float(n) * theta <= 47000.f) ? 4 : 0;
     return n <= 20000 ? 4 : n <= 75000 ? 16 : 0;
 }
 

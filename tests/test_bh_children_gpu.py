@@ -69,8 +69,8 @@ def test_capture_of_the_trees_own_bodies():
 
 
 @pytest.mark.parametrize("params", ["quadrupole_params", "octupole_params"])
-@pytest.mark.parametrize("n,theta,batched", [(10_000, 1.1, True), (10_001, 1.2, False), (50_000, 0.6, True),
-                                             (51_000, 0.6, False), (130_000, 0.3, True), (130_001, 0.3, False)])
+@pytest.mark.parametrize("n,theta,batched", [(40_000, 1.3, True), (40_001, 1.3, False), (78_000, 0.6, True),
+                                             (79_000, 0.6, False), (150_000, 0.3, True), (150_001, 0.3, False)])
 def test_corrected_borders(monkeypatch, params, n, theta, batched):
     """Both sides of the border between the walks, which falls with the angle: the same accepted nodes,
     sums to rounding (the bar the stackless walk's own widths are held to), and the walk it should be
@@ -97,7 +97,7 @@ def test_corrected_borders(monkeypatch, params, n, theta, batched):
 
 def test_capture_at_another_angle():
     """Sized at an angle without a child table, a capture at one that would want it is taken."""
-    d = torch.from_numpy(workloads.two_plummer_case(60_000, seed=2).particles).cuda()
+    d = torch.from_numpy(workloads.two_plummer_case(70_000, seed=2).particles).cuda()
     with pa.HipResources(0) as res:
         learned.init(res, 0)
         learned.set_params(res, learned.quadrupole_params())
