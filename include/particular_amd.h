@@ -241,7 +241,8 @@ int pnb_bh_tree_size(pnb_ctx *ctx, size_t *nodes, int *max_level);
 /* Copies the nodes (cap >= nodes) and, if `order` is not NULL, the original index of every
  * affecting particle in tree order (m >= affecting count). */
 int pnb_bh_tree_export(pnb_ctx *ctx, pnb_tree_node *nodes, size_t cap, uint32_t *order, size_t m);
-/* Counters of the walks since the last build: wavefront node steps and accepted pair terms (with
+/* Counters of the walks since the last build: wavefront node steps (for small and middle sets, which are
+ * walked in batches of nodes, the nodes each wavefront summed) and accepted pair terms (with
  * PNB_BH_RELATIVE, the estimate pass's included). */
 int pnb_bh_stats(pnb_ctx *ctx, uint64_t *wave_steps, uint64_t *accepted);
 
@@ -266,7 +267,8 @@ int pnb_bh_accel_f32_2d_dev(pnb_ctx *ctx, const float *affected, size_t n, const
  * particular/src/gravity/impls/glam.rs:234): records are 4 doubles {x, y, z, mu} (32 B); the
  * reference's scalar kernel in FP64 (impls/mod.rs:151-166), the term mu r^-3 from a corrected reciprocal
  * square root, as exact as an IEEE square root and division (three roundings). Zero, vanishing and
- * infinite distances give what the division gives. */
+ * infinite distances give what the division gives. Inside a stream capture a sum takes one affecting range
+ * and no scratch. */
 int pnb_bf_accel_f64(pnb_ctx *ctx, const double *affected, size_t n, const double *affecting,
                      size_t m, double softening, int checked, double *out);
 int pnb_bf_accel_f64_dev(pnb_ctx *ctx, const double *affected, size_t n, const double *affecting,
